@@ -231,7 +231,31 @@ __device__ __forceinline__ void vm_wait_n(int n) {
     default: RSPX_VMW(63); break;
   }
 }
-#undef RSPX_VMW
+
+// Columns n .. n + 3 of output row m (chunk s): the fp32 chunk partial, the
+// SwiGLU of the two (gate, up) column pairs, or the result in fp32 or bf16.
+__device__ __forceinline__ void store_tile(const Args& A, int s, int m, int n, f32x4 v) {
+  if (m >= A.M) return;
+  if (A.S > 1 || A.to_part) {
+    *reinterpret_cast<f32x4*>(A.part + ((size_t)s * A.M + m) * A.N + n) = v;
+  } else if (A.out_fp32) {
+    *reinterpret_cast<f32x4*>(static_cast<float*>(A.out) + (int64_t)m * A.so + n) = v;
+  } else if (A.silu) {
+    // The bf16 gate/up values rspx_linear would store, then rspx_silu_mul's
+    // arithmetic: bf16(bf16(silu(g)) * u) for columns n / 2 and n / 2 + 1.
+    const uint32_t p0 = pack_bf16x2(v[0], v[1]);
+    const uint32_t p1 = pack_bf16x2(v[2], v[3]);
+    const float a0 = round_bf16(silu_f32(bf16_lo(p0))), a1 = round_bf16(silu_f32(bf16_lo(p1)));
+    uint16_t* dst = static_cast<uint16_t*>(A.out) +
+                    (A.out_tiled ? tiled_offset(m, n / 2, A.N / 2) : (int64_t)m * A.so + n / 2);
+    *reinterpret_cast<uint32_t*>(dst) = pack_bf16x2(a0 * bf16_hi(p0), a1 * bf16_hi(p1));
+  } else {
+    u32x2 o;
+    o[0] = pack_bf16x2(v[0], v[1]);
+    o[1] = pack_bf16x2(v[2], v[3]);
+    *reinterpret_cast<u32x2*>(static_cast<uint16_t*>(A.out) + (int64_t)m * A.so + n) = o;
+  }
+}
 
 // Pipeline: W (the HBM stream) is requested 3 rounds ahead into a ring of 4
 // register buffers, X (L2-resident) 1 round ahead into 2 LDS buffers.  Round
@@ -374,31 +398,165 @@ __global__ __launch_bounds__(64 * W) void gemm_kernel(Args A) {
 
   // D[n][m]: lane (n16, g4) holds columns col + 4 g4 + e of row 16 t + n16.
 #pragma unroll
-  for (int t = 0; t < MT; ++t) {
-    const int m = row0 + 16 * t + n16;
-    if (m >= A.M) continue;
-    const int n = col + 4 * g4;
-    if (A.S > 1 || A.to_part) {
-      *reinterpret_cast<f32x4*>(A.part + ((size_t)s * A.M + m) * A.N + n) = acc[t];
-    } else if (A.out_fp32) {
-      *reinterpret_cast<f32x4*>(static_cast<float*>(A.out) + (int64_t)m * A.so + n) = acc[t];
-    } else if (A.silu) {
-      // The bf16 gate/up values rspx_linear would store, then rspx_silu_mul's
-      // arithmetic: bf16(bf16(silu(g)) * u) for columns n / 2 and n / 2 + 1.
-      const uint32_t p0 = pack_bf16x2(acc[t][0], acc[t][1]);
-      const uint32_t p1 = pack_bf16x2(acc[t][2], acc[t][3]);
-      const float a0 = round_bf16(silu_f32(bf16_lo(p0))), a1 = round_bf16(silu_f32(bf16_lo(p1)));
-      uint16_t* dst = static_cast<uint16_t*>(A.out) +
-                      (A.out_tiled ? tiled_offset(m, n / 2, A.N / 2) : (int64_t)m * A.so + n / 2);
-      *reinterpret_cast<uint32_t*>(dst) = pack_bf16x2(a0 * bf16_hi(p0), a1 * bf16_hi(p1));
+  for (int t = 0; t < MT; ++t) store_tile(A, s, row0 + 16 * t + n16, col + 4 * g4, acc[t]);
+}
+
+// More than 64 rows: workgroup = (64 CT output columns, chunk s, 16 MT rows), 4
+// waves of CT 16-column tiles, every wave over all MT row tiles.  The same MFMA
+// chain per element as gemm_kernel, in the same k order: the same bits.
+//
+// What bounds it: at one 16-column tile per wave (gemm_kernel) a k-block's X
+// fragments (1 KB of LDS reads per MFMA) take twice the time of its MFMAs, and
+// every 64 rows read W again.  A wave that owns CT column tiles reads an X
+// fragment once for CT MFMAs, and MT = 8 row tiles read a W fragment once for 8.
+// W still goes from memory straight into registers (each fragment is read by one
+// wave only), X through an LDS ring; both are requested 3 rounds of KB k-blocks
+// ahead, one barrier per round: the barrier that publishes round r's X also says
+// that every wave is done with round r - 1, whose buffer then takes round r + 3.
+//
+// Tiles of one 64 CT-column slice and chunk follow each other on one XCD
+// (workgroups are dealt round-robin over the 8 XCDs), so its L2 reads the slice of
+// W from memory once for all row tiles.
+//
+// 512 rows, q/k/v [6144, 4096], o [4096, 4096], gate/up [24576, 4096] and down
+// [4096, 12288]: 35.6 / 23.0 / 103 / 49 us (0.72 / 0.75 / 1.0 / 1.05 PFLOP/s)
+// instead of 77.7 / 44.9 / 257 / 132 us in 64-row tiles of gemm_kernel.
+constexpr int kWideRing = 4;    // rounds of X in LDS and of W in registers
+template <int CT> constexpr int wide_kb() { return CT >= 3 ? 1 : 2; }   // k-blocks of a round
+
+template <int MT, int CT, bool WT>
+__global__ __launch_bounds__(256, 2) void gemm_wide_kernel(Args A, int units, int mtiles) {
+  constexpr int KB = wide_kb<CT>();
+  constexpr int NC = KB * MT;             // 1 KB X chunks of a round
+  constexpr int XL = (NC + 3) / 4;        // chunks a wave requests per round (those past NC read nothing)
+  constexpr int WL = KB * CT;             // W loads of a wave per round
+  constexpr int WKB = WT ? 1024 : 64;     // bytes between a lane's consecutive k-blocks of W
+  static_assert(2 * (XL + WL) < 64 && kWideRing == 4 && 256 % (32 * KB * kWideRing) == 0, "vmcnt range");
+  __shared__ __attribute__((aligned(16))) char xs[(kWideRing * NC + 1) * 1024];   // the last KB takes chunks past NC
+  const int lane = __lane_id();
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int n16 = lane & 15, g4 = lane >> 4;
+  // Workgroup id -> (unit = column slice and chunk, row tile): ids equal mod 8 share an XCD.
+  const int j = blockIdx.x >> 3;
+  const int unit = (blockIdx.x & 7) + 8 * (j / mtiles), mt = j % mtiles;
+  if (unit >= units) return;
+  const int s = unit % A.S, nt = unit / A.S;
+  const int col = nt * 64 * CT + 16 * CT * w;   // this wave's first column
+  const int row0 = mt * 16 * MT;
+  const int k0 = s * A.KC;
+  const int nr = A.KC / (32 * KB);              // a multiple of kWideRing: KC % 256 == 0
+  const int ncol = min(CT, (A.N - col + 15) / 16);   // column tiles of this wave inside N (may be <= 0)
+
+  // X: lane offset of the wave's chunk jj of a round: c = w + 4 jj, k-block
+  // c / MT, row tile c % MT.
+  const int mrows = min(16 * MT, A.M - row0);
+  const int t0 = row0 / 16;                      // first 16-row tile
+  const __amdgpu_buffer_rsrc_t rx =
+      A.x_tiled ? rsrc(A.x + (int64_t)(t0 >> 2) * 64 * A.K, (int64_t)(((t0 + MT - 1) >> 2) - (t0 >> 2) + 1) * A.K * 128)
+                : rsrc(A.x + (int64_t)row0 * A.sx + k0, 2 * ((int64_t)(mrows - 1) * A.sx + (A.K - k0)));
+  const int xkb = A.x_tiled ? 4096 : 64;
+  int xo[XL];
+#pragma unroll
+  for (int jj = 0; jj < XL; ++jj) {
+    const int c = w + 4 * jj, kb = c / MT, t = c % MT;
+    int o;
+    if (A.x_tiled) {
+      const int T = t0 + t;
+      o = (((T >> 2) - (t0 >> 2)) * (A.K >> 5) + (k0 >> 5) + kb) * 4096 + (T & 3) * 1024 + 16 * lane;
     } else {
-      u32x2 o;
-      o[0] = pack_bf16x2(acc[t][0], acc[t][1]);
-      o[1] = pack_bf16x2(acc[t][2], acc[t][3]);
-      *reinterpret_cast<u32x2*>(static_cast<uint16_t*>(A.out) + (int64_t)m * A.so + n) = o;
+      o = 2 * ((16 * t + n16) * (int)A.sx + 8 * g4) + 64 * kb;
+    }
+    xo[jj] = c < NC && 16 * t < mrows ? o : kOOBRow;
+  }
+  const __amdgpu_buffer_rsrc_t rw =
+      WT ? rsrc(A.w + (int64_t)(col / 16) * ((A.K / 32) * 512 + kWSlabPad) + (k0 / 32) * 512,
+                ncol > 0 ? (int64_t)(ncol - 1) * (A.K * 32 + 2 * kWSlabPad) + A.KC * 32 : 0)
+         : rsrc(A.w + (int64_t)(ncol > 0 ? col : 0) * A.sw + k0,
+                ncol > 0 ? 2 * ((int64_t)(16 * ncol - 1) * A.sw + A.KC) : 0);
+  const int woff = WT ? 16 * lane : 2 * (n16 * (int)A.sw + 8 * g4);
+  const int wcol = WT ? A.K * 32 + 2 * kWSlabPad : 32 * (int)A.sw;   // bytes between column tiles
+
+  lds_char_t* xl = (lds_char_t*)xs;
+  f32x4 acc[MT][CT];
+#pragma unroll
+  for (int t = 0; t < MT; ++t)
+#pragma unroll
+    for (int c = 0; c < CT; ++c) acc[t][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+  u32x4 wf[kWideRing][KB][CT];
+
+  // Round rr's W into ring slot rr % 4, then its X chunks: with X issued last, a
+  // count that covers round rr's X covers its W too.
+  auto issue = [&](int rr, u32x4 (&wr)[KB][CT], int slot) {
+#pragma unroll
+    for (int c = 0; c < CT; ++c)
+#pragma unroll
+      for (int kb = 0; kb < KB; ++kb)
+        wr[kb][c] = __builtin_bit_cast(
+            u32x4, __builtin_amdgcn_raw_buffer_load_b128(rw, woff + c * wcol + WKB * (KB * rr + kb), 0, 0));
+#pragma unroll
+    for (int jj = 0; jj < XL; ++jj) {
+      const int c = w + 4 * jj;
+      x_dma16(rx, xo[jj] + xkb * KB * rr, xl + (c < NC ? slot * NC + c : kWideRing * NC) * 1024);
+    }
+    asm volatile("" ::: "memory");
+  };
+  // The X fragments of a k-block are read two row tiles ahead of their MFMAs.
+  auto compute = [&](const u32x4 (&wr)[KB][CT], int slot) {
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) {
+      u32x4 xf[MT];
+#pragma unroll
+      for (int t = 0; t < MT; ++t)
+        xf[t] = *(const __attribute__((address_space(3))) u32x4*)(xl + (slot * NC + kb * MT + t) * 1024 + 16 * lane);
+#pragma unroll
+      for (int t = 0; t < MT; ++t)
+#pragma unroll
+        for (int c = 0; c < CT; ++c)
+          acc[t][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wr[kb][c]),
+                                                              __builtin_bit_cast(bf16x8, xf[t]), acc[t][c], 0, 0, 0);
+    }
+    __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);   // LDS reads
+#pragma unroll
+    for (int t = 0; t < MT * KB; ++t) {
+      __builtin_amdgcn_sched_group_barrier(0x008, CT, 0);   // MFMAs
+      if (t + 3 < MT * KB) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+    }
+  };
+  constexpr int PER = XL + WL;   // loads a wave issues per round
+#pragma unroll
+  for (int r = 0; r < kWideRing - 1; ++r) issue(r, wf[r], r);
+  int r = 0;
+  for (; r + kWideRing < nr; r += kWideRing) {
+#pragma unroll
+    for (int u = 0; u < kWideRing; ++u) {
+      RSPX_VMW(2 * PER);   // round r + u has landed (this wave's part)
+      raw_barrier();       // every wave's part, and every wave is done with round r + u - 1
+      issue(r + u + kWideRing - 1, wf[(u + kWideRing - 1) % kWideRing], (u + kWideRing - 1) % kWideRing);
+      compute(wf[u], u);
     }
   }
+  // The last four rounds: one more to request.
+  RSPX_VMW(2 * PER);
+  raw_barrier();
+  issue(r + 3, wf[3], 3);
+  compute(wf[0], 0);
+  RSPX_VMW(2 * PER);
+  raw_barrier();
+  compute(wf[1], 1);
+  RSPX_VMW(PER);
+  raw_barrier();
+  compute(wf[2], 2);
+  RSPX_VMW(0);
+  raw_barrier();
+  compute(wf[3], 3);
+#pragma unroll
+  for (int c = 0; c < CT; ++c)
+    if (c < ncol)
+#pragma unroll
+      for (int t = 0; t < MT; ++t) store_tile(A, s, row0 + 16 * t + n16, col + 16 * c + 4 * g4, acc[t][c]);
 }
+
+#undef RSPX_VMW
 
 // out[m][n] = round(((p0 + p1) + p2) + ...), 4 columns per thread.  Grid:
 // x = 256-thread blocks along a row, y = rows from row0 (at most 65535 per
@@ -573,6 +731,66 @@ extern "C" int64_t rspx_linear_workspace_bytes(int M, int N, int K) {
 }
 
 namespace rspx {
+// The chunk sums of a split product that no consumer takes, and the launch status.
+static int reduce_launch(const gemm::Args& a, hipStream_t s) {
+  if (a.S > 1 && !a.to_part) {
+    const unsigned bx = (unsigned)((a.N / 4 + 255) / 256);
+    for (int row0 = 0; row0 < a.M; row0 += 65535) {
+      const dim3 rg(bx, (unsigned)min(a.M - row0, 65535));
+      RSPX_WITH_SPLITS(a.S, SC,
+                       hipLaunchKernelGGL((gemm::reduce_kernel<SC>), rg, dim3(256), 0, s, a.part, a.S, a.M, a.N, a.out,
+                                          a.so, a.out_fp32, row0));
+    }
+  }
+  return hipGetLastError() == hipSuccess ? RSPX_OK : RSPX_ELAUNCH;
+}
+
+// 31-bit byte offsets inside a 128-row tile of x and a wave's 64 rows of w.
+static bool wide_fits(const gemm::Args& a) {
+  return (a.x_tiled || (int64_t)128 * a.sx * 2 < (1ll << 30)) && (a.sw == kTiled || (int64_t)64 * a.sw * 2 < (1ll << 30)) &&
+         (int64_t)a.K * 384 < (1ll << 30);
+}
+
+static int wide_launch(const gemm::Args& a, hipStream_t s) {
+  // Row tiles of at most 128 rows, all of the same height.
+  const int mtiles = (a.M + 127) / 128;
+  const int mt = ((a.M + mtiles - 1) / mtiles + 15) / 16;
+  // Column tiles per wave: the least time for the busiest CU, workgroups per CU
+  // times a workgroup's time for its 16 ct columns per wave.  Narrower waves read
+  // each X fragment for fewer MFMAs, so ct = 1 .. 4 cost 14 : 24 : 31 : 40 and not
+  // 1 : 2 : 3 : 4 (512 rows, o projection [4096, 4096]: 33.1 / 27.5 / 32.6 / 23.0 us
+  // at ct = 1 .. 4 with 4 / 2 / 2 / 1 workgroups per CU; 512 rows, gate/up
+  // [24576, 4096]: 144.8 / 115.8 / 103.3 / 116.7 us with 6 / 3 / 2 / 2; 128 rows,
+  // q/k/v [6144, 4096]: 20.1 / 16.5 / 19.3 / 22.2 us with 2 / 1 / 1 / 1).
+  static const int cost[5] = {0, 14, 24, 31, 40};
+  int ct = 4;
+  int64_t best = 0;
+  for (int c = 4; c >= 1; --c) {
+    const int64_t t = ((int64_t)((a.N + 64 * c - 1) / (64 * c)) * a.S * mtiles + 255) / 256 * cost[c];
+    if (c == 4 || t < best) { ct = c; best = t; }
+  }
+  const int64_t units = (int64_t)((a.N + 64 * ct - 1) / (64 * ct)) * a.S;
+  const int64_t wgs = (units + 7) / 8 * 8 * mtiles;
+  if (wgs > 0x7fffffff) return RSPX_EUNSUPPORTED;
+  const dim3 g((unsigned)wgs), b(256);
+#define RSPX_WIDE(MTV, CTV)                                                                                        \
+  if (a.sw == kTiled)                                                                                              \
+    hipLaunchKernelGGL((gemm::gemm_wide_kernel<MTV, CTV, true>), g, b, 0, s, a, (int)units, mtiles);               \
+  else hipLaunchKernelGGL((gemm::gemm_wide_kernel<MTV, CTV, false>), g, b, 0, s, a, (int)units, mtiles);
+#define RSPX_WIDE_CT(MTV)                                \
+  if (ct == 4) { RSPX_WIDE(MTV, 4) }                     \
+  else if (ct == 3) { RSPX_WIDE(MTV, 3) }                \
+  else if (ct == 2) { RSPX_WIDE(MTV, 2) }                \
+  else { RSPX_WIDE(MTV, 1) }
+  if (mt == 8) { RSPX_WIDE_CT(8) }
+  else if (mt == 7) { RSPX_WIDE_CT(7) }
+  else if (mt == 6) { RSPX_WIDE_CT(6) }
+  else { RSPX_WIDE_CT(5) }
+#undef RSPX_WIDE_CT
+#undef RSPX_WIDE
+  return reduce_launch(a, s);
+}
+
 static int linear_launch(const void* x, int64_t sx, const void* w, int64_t sw, void* out, int64_t so, int M, int N,
                          int K, int out_fp32, float* part, int to_part, hipStream_t s, int silu = 0) {
   const int S = linear_splits(N, K);
@@ -585,6 +803,7 @@ static int linear_launch(const void* x, int64_t sx, const void* w, int64_t sw, v
   a.silu = silu;
   a.x_tiled = sx == kTiled;
   a.out_tiled = silu && so == kTiled;
+  if (M > gemm::kRows && wide_fits(a)) return wide_launch(a, s);
   const int MTILES = (M + gemm::kRows - 1) / gemm::kRows;
   // 8 waves (128 columns) share each X round between twice the columns; worth
   // it while the grid keeps >= 192 workgroups, and for the widest layers
@@ -636,16 +855,7 @@ static int linear_launch(const void* x, int64_t sx, const void* w, int64_t sw, v
 #undef RSPX_GEMM_W
 #undef RSPX_GEMM_MT
 #undef RSPX_GEMM_NR
-  if (S > 1 && !to_part) {
-    const unsigned bx = (unsigned)((N / 4 + 255) / 256);
-    for (int row0 = 0; row0 < M; row0 += 65535) {
-      const dim3 rg(bx, (unsigned)min(M - row0, 65535));
-      RSPX_WITH_SPLITS(S, SC,
-                       hipLaunchKernelGGL((gemm::reduce_kernel<SC>), rg, dim3(256), 0, s, part, S, M, N, out, so,
-                                          a.out_fp32, row0));
-    }
-  }
-  return hipGetLastError() == hipSuccess ? RSPX_OK : RSPX_ELAUNCH;
+  return reduce_launch(a, s);
 }
 
 static int linear_check(const void* x, int64_t sx, const void* w, int64_t sw, int M, int N, int K) {

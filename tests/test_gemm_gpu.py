@@ -418,3 +418,45 @@ def test_linear_silu_tiled_w(M):
         outs.append(o)
     torch.cuda.synchronize()
     assert torch.equal(outs[0], outs[1])
+
+
+@pytest.mark.parametrize("M,N,K", [(65, 16, 256), (80, 272, 512), (81, 64, 256), (96, 4112, 256), (112, 1040, 768),
+                                   (113, 4096, 1024), (127, 12304, 512), (128, 6144, 256), (129, 528, 1280),
+                                   (257, 8208, 256), (513, 4096, 512)])
+def test_linear_many_rows(M, N, K):
+    """More than 64 rows (row tiles of 80 .. 128 rows, 1 .. 4 column tiles per wave, ragged last
+    tiles): the bits of 64-row calls from row-major and tiled operands, in bf16, fp32, chunk
+    partials and the SwiGLU epilogue, and the parity bound of test_linear_parity_bf16."""
+    from _tiled import to_tiled
+    from respect_amd import _lib
+    from respect_amd.kernels.gemm import linear, tile_weight
+    print(f"[linear many rows] M={M} N={N} K={K}", flush=True)
+    x, w = _xw(M * 5 + N + K, M, N, K)
+    xd, wd = _dev(x), _dev(w)
+    wt = tile_weight(wd)
+    for dt in (torch.bfloat16, torch.float32):
+        ref = torch.cat([linear(xd[i:i + 64], wd, out_dtype=dt) for i in range(0, M, 64)])
+        assert torch.equal(linear(xd, wd, out_dtype=dt), ref)
+        assert torch.equal(linear(xd, wt, out_dtype=dt), ref)
+    ex = G.linear_exact(x, w)
+    assert np.all(np.abs(ref.cpu().numpy().astype(np.float64) - ex) <= G.linear_error_bound(x, w) + 1e-30)
+    # tiled x (the last block's rows past M hold NaN, which must not reach a result)
+    L, s, T = _lib.lib(), _lib.stream_ptr(xd.device), _lib.RSPX_TILED
+    xt = to_tiled(xd, fill=float("nan"))
+    S = L.rspx_linear_splits(N, K)
+    parts = [torch.full((S, M, N), float("nan"), device="cuda") for _ in range(3)]
+    for p, xa, sx, wa in ((parts[0], xd, K, wd), (parts[1], xt, T, wd), (parts[2], xt, T, wt)):
+        _lib.check("rspx_linear_partials", L.rspx_linear_partials(xa.data_ptr(), sx, wa.data_ptr(), wa.stride(0),
+                                                                  p.data_ptr(), M, N, K, s))
+    acc = parts[0][0]
+    for c in range(1, S):
+        acc = acc + parts[0][c]
+    assert torch.equal(acc, ref) and torch.equal(parts[0], parts[1]) and torch.equal(parts[0], parts[2])
+    if S == 1 and N % 32 == 0:
+        def silu(m0, m1):
+            o = torch.empty(m1 - m0, N // 2, device="cuda", dtype=torch.bfloat16)
+            xa = xd[m0:m1]
+            _lib.check("rspx_linear_silu", L.rspx_linear_silu(xa.data_ptr(), K, wt.data_ptr(), T, o.data_ptr(),
+                                                              N // 2, m1 - m0, N, K, s))
+            return o
+        assert torch.equal(silu(0, M), torch.cat([silu(i, min(M, i + 64)) for i in range(0, M, 64)]))
