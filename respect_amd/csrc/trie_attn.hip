@@ -270,22 +270,14 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_rsrc(const void* base, 
 
 // The transposing LDS read: within each 16-lane row, lane i receives
 // element (i % 4) of the 8 bytes addressed by lane 4 e + i / 4, for e = 0..3.
-__device__ __forceinline__ s16x4 lds_read_tr(const lds_char* p) {
+// Callers read data that is in place (its loads waited for, the barrier passed).
+// __restrict__: once inlined, the intrinsic's memory operand then carries alias
+// information; without any, the compiler puts s_waitcnt vmcnt(0) in front of it
+// -- a wait for every direct-to-LDS load in flight, the next round's K/V included,
+// in the middle of every step.
+__device__ __forceinline__ s16x4 lds_read_tr(const lds_char* __restrict__ p) {
   typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
   return __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)p);
-}
-
-// lds_read_tr pair without the compiler's fence: the intrinsic's memory
-// operand carries no alias information, so the compiler puts s_waitcnt
-// vmcnt(0) in front of it -- a wait for every vector-memory operation in
-// flight, the group partial's counter add included.  For LDS data that is
-// known to be in place (its loads waited for), read the two halves in asm and
-// wait for them (lgkmcnt) inside the asm that hands them out.
-__device__ __forceinline__ void lds_read_tr2_nofence(const lds_char* p0, const lds_char* p1, s16x4& lo, s16x4& hi) {
-  asm volatile("ds_read_b64_tr_b16 %0, %2\n\tds_read_b64_tr_b16 %1, %3\n\ts_waitcnt lgkmcnt(0)"
-               : "=&v"(lo), "=&v"(hi)
-               : "v"(p0), "v"(p1)
-               : "memory");
 }
 
 __device__ __forceinline__ void lds_barrier() {
@@ -330,6 +322,111 @@ struct PromptLds {
   static constexpr int MLBYTES = 8 * kRT * 16 * 8;
   static_assert(BYTES + MLBYTES <= 160 * 1024, "LDS budget");
 };
+
+// One step of 32 keys from first key ks, K/V in LDS at `slot`, for the wave's kRT
+// row tiles: scores, online softmax against the lazily moved reference maximum,
+// and the PV product.  kro / trv: the lane's LDS offsets of the K fragments and of
+// the V operand halves inside a slot.
+template <int D, int kRT>
+__device__ __forceinline__ void prompt_step(const TrieAttnArgs& A, const lds_char* slot, int ks,
+                                            const int (&kro)[2][StepGeom<D>::DQ], const int (&trv)[2][StepGeom<D>::DT],
+                                            const bf16x8 (&qop)[kRT][StepGeom<D>::DQ], float (&mref)[kRT],
+                                            float (&lrow)[kRT], f32x4 (&acc)[kRT][StepGeom<D>::DT]) {
+  constexpr int DQ = StepGeom<D>::DQ, DT = StepGeom<D>::DT;
+  const int g4 = __lane_id() >> 4;
+    u32x4 kf[2][DQ];
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+      for (int i = 0; i < DQ; ++i)
+        kf[kb][i] = *(const __attribute__((address_space(3))) u32x4*)(slot + kro[kb][i]);
+
+    // S^T = K Q^T for two blocks of 16 keys.
+    f32x4 sc[kRT][2];
+#pragma unroll
+    for (int t = 0; t < kRT; ++t)
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb) {
+        f32x4 sv = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < DQ; ++i)
+          sv = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, kf[kb][i]), qop[t][i], sv,
+                                                       0, 0, 0);
+        sc[t][kb] = sv;
+      }
+
+    // Lane (n16, g4) holds row n16, keys 16 kb + 4 g4 + e of the step.  Raw
+    // scores; keys past P (only in the last step) are masked to -inf.  Since
+    // scale > 0, max(s) * c is exactly the max of the scaled scores.
+    bf16x8 pop[kRT];
+    float m8[kRT];
+    float s8[kRT][8];
+    bool any_move = false;
+    const bool full = ks + kStep <= A.P;
+#pragma unroll
+    for (int t = 0; t < kRT; ++t) {
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s8[t][4 * kb + e] = sc[t][kb][e];
+      if (!full) {
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (ks + 16 * kb + 4 * g4 + e >= A.P) s8[t][4 * kb + e] = kNegInf;
+      }
+      m8[t] = s8[t][0];
+#pragma unroll
+      for (int i = 1; i < 8; ++i) m8[t] = fmaxf(m8[t], s8[t][i]);
+      any_move |= m8[t] * A.c > mref[t] + kLazyTau;
+    }
+    // Move the reference maximum of rows that outgrew it (wave-uniform branch;
+    // rows that did not move get alpha = 2^0 = 1 exactly).  A row outgrew it
+    // exactly if one of the four lanes that share it holds such a score, so the
+    // row's maximum over those lanes is taken inside the branch only.
+    if (__builtin_amdgcn_ballot_w64(any_move) != 0) {
+#pragma unroll
+      for (int t = 0; t < kRT; ++t) {
+        const float mx = rows4_max(m8[t]) * A.c;
+        const float mn = mx > mref[t] + kLazyTau ? mx : mref[t];
+        const float alpha = fexp2(mref[t] - mn);
+        lrow[t] = lrow[t] * alpha;
+        mref[t] = mn;
+#pragma unroll
+        for (int j = 0; j < DT; ++j) acc[t][j] = acc[t][j] * alpha;
+      }
+    }
+#pragma unroll
+    for (int t = 0; t < kRT; ++t) {
+      float p[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) p[i] = fexp2(__builtin_fmaf(s8[t][i], A.c, -mref[t]));
+      float rs = p[0];
+#pragma unroll
+      for (int i = 1; i < 8; ++i) rs = rs + p[i];
+      lrow[t] = lrow[t] + rows4_sum(rs);
+      u32x4 pw;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) pw[i] = pack_bf16x2(p[2 * i], p[2 * i + 1]);
+      pop[t] = __builtin_bit_cast(bf16x8, pw);
+    }
+
+    // O^T += V^T bf16(P)^T.  B operand: lane (n16, g4) holds row n16's p at
+    // k-slots 8 g4 + i <-> keys 4 g4 + i (i < 4) and 12 + 4 g4 + i.  A operand
+    // of head_dim tile j: V[key(k-slot)][16 j + n16], two transposing reads.
+    // Output lane: row n16, head_dim 16 j + 4 g4 + e -- each lane holds four
+    // consecutive head_dim columns of the row whose softmax state it keeps.
+#pragma unroll
+    for (int j = 0; j < DT; ++j) {
+      const s16x4 lo = lds_read_tr(slot + trv[0][j]);
+      const s16x4 hi = lds_read_tr(slot + trv[1][j]);
+      const bf16x8 vop = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+#pragma unroll
+      for (int t = 0; t < kRT; ++t)
+        acc[t][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vop, pop[t], acc[t][j], 0, 0, 0);
+    }
+}
 
 // The prompt work of workgroup (g, rb, q) -- kv head g, rows [32 kRT rb,
 // +32 kRT), key group q = steps [q S, q S + S) -- up to its group partial in
@@ -468,98 +565,8 @@ __device__ __forceinline__ void prompt_block(const TrieAttnArgs& A, char* lds, i
     const int sl = kQuarters * r + k;  // step of this wave within the group
     if (has_rows && sl < ns) {
 
-    const lds_char* slot = ring + (r % G::RING) * G::ROUND + k * G::SLOT;
-    const int ks = (s0 + sl) * kStep;
-    u32x4 kf[2][DQ];
-#pragma unroll
-    for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-      for (int i = 0; i < DQ; ++i)
-        kf[kb][i] = *(const __attribute__((address_space(3))) u32x4*)(slot + kro[kb][i]);
-
-    // S^T = K Q^T for two blocks of 16 keys.
-    f32x4 sc[kRT][2];
-#pragma unroll
-    for (int t = 0; t < kRT; ++t)
-#pragma unroll
-      for (int kb = 0; kb < 2; ++kb) {
-        f32x4 sv = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int i = 0; i < DQ; ++i)
-          sv = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, kf[kb][i]), qop[t][i], sv,
-                                                       0, 0, 0);
-        sc[t][kb] = sv;
-      }
-
-    // Lane (n16, g4) holds row n16, keys 16 kb + 4 g4 + e of the step.  Raw
-    // scores; keys past P (only in the last step) are masked to -inf.  Since
-    // scale > 0, max(s) * c is exactly the max of the scaled scores.
-    bf16x8 pop[kRT];
-    float mx[kRT];
-    float s8[kRT][8];
-    bool any_move = false;
-    const bool full = ks + kStep <= P;
-#pragma unroll
-    for (int t = 0; t < kRT; ++t) {
-#pragma unroll
-      for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) s8[t][4 * kb + e] = sc[t][kb][e];
-      if (!full) {
-#pragma unroll
-        for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            if (ks + 16 * kb + 4 * g4 + e >= P) s8[t][4 * kb + e] = kNegInf;
-      }
-      float m8 = s8[t][0];
-#pragma unroll
-      for (int i = 1; i < 8; ++i) m8 = fmaxf(m8, s8[t][i]);
-      mx[t] = rows4_max(m8) * A.c;
-      any_move |= mx[t] > mref[t] + kLazyTau;
-    }
-    // Move the reference maximum of rows that outgrew it (wave-uniform branch;
-    // rows that did not move get alpha = 2^0 = 1 exactly).
-    if (__builtin_amdgcn_ballot_w64(any_move) != 0) {
-#pragma unroll
-      for (int t = 0; t < kRT; ++t) {
-        const float mn = mx[t] > mref[t] + kLazyTau ? mx[t] : mref[t];
-        const float alpha = fexp2(mref[t] - mn);
-        lrow[t] = lrow[t] * alpha;
-        mref[t] = mn;
-#pragma unroll
-        for (int j = 0; j < DT; ++j) acc[t][j] = acc[t][j] * alpha;
-      }
-    }
-#pragma unroll
-    for (int t = 0; t < kRT; ++t) {
-      float p[8];
-#pragma unroll
-      for (int i = 0; i < 8; ++i) p[i] = fexp2(__builtin_fmaf(s8[t][i], A.c, -mref[t]));
-      float rs = p[0];
-#pragma unroll
-      for (int i = 1; i < 8; ++i) rs = rs + p[i];
-      lrow[t] = lrow[t] + rows4_sum(rs);
-      u32x4 pw;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) pw[i] = pack_bf16x2(p[2 * i], p[2 * i + 1]);
-      pop[t] = __builtin_bit_cast(bf16x8, pw);
-    }
-
-    // O^T += V^T bf16(P)^T.  B operand: lane (n16, g4) holds row n16's p at
-    // k-slots 8 g4 + i <-> keys 4 g4 + i (i < 4) and 12 + 4 g4 + i.  A operand
-    // of head_dim tile j: V[key(k-slot)][16 j + n16], two transposing reads.
-    // Output lane: row n16, head_dim 16 j + 4 g4 + e -- each lane holds four
-    // consecutive head_dim columns of the row whose softmax state it keeps.
-#pragma unroll
-    for (int j = 0; j < DT; ++j) {
-      const s16x4 lo = lds_read_tr(slot + trv[0][j]);
-      const s16x4 hi = lds_read_tr(slot + trv[1][j]);
-      const bf16x8 vop = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-#pragma unroll
-      for (int t = 0; t < kRT; ++t)
-        acc[t][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vop, pop[t], acc[t][j], 0, 0, 0);
-    }
+    prompt_step<D, kRT>(A, ring + (r % G::RING) * G::ROUND + k * G::SLOT, (s0 + sl) * kStep, kro, trv, qop, mref, lrow,
+                        acc);
     }
     if (r < 3) RSPX_MARK(2 + 2 * r);
     // Round r is consumed by every wave: its ring slot takes round r + RING.
@@ -1141,14 +1148,8 @@ __device__ __forceinline__ void node_task(const TrieAttnArgs& A, int g, int p0, 
 #pragma unroll
     for (int jj = 0; jj < NJ; ++jj) {
       const int b = 2 * (NJ * sl + jj) + (c4 >> 1);
-      s16x4 lo, hi;
-      if constexpr (RES) {
-        // V rows resident since before the caller's wait: no fence needed.
-        lds_read_tr2_nofence(vrow0 + 16 * (b ^ vsw0) + 8 * (c4 & 1), vrow1 + 16 * (b ^ vsw1) + 8 * (c4 & 1), lo, hi);
-      } else {
-        lo = lds_read_tr(vrow0 + 16 * (b ^ vsw0) + 8 * (c4 & 1));
-        hi = lds_read_tr(vrow1 + 16 * (b ^ vsw1) + 8 * (c4 & 1));
-      }
+      const s16x4 lo = lds_read_tr(vrow0 + 16 * (b ^ vsw0) + 8 * (c4 & 1));
+      const s16x4 hi = lds_read_tr(vrow1 + 16 * (b ^ vsw1) + 8 * (c4 & 1));
       const bf16x8 vop = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
       acc[jj] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vop, hop, acc[jj], 0, 0, 0);
       acc[jj] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vop, lop, acc[jj], 0, 0, 0);
