@@ -49,7 +49,8 @@
 // (MFMA scores and rank-tiled MFMA sums) and, once the block's groups are all
 // counted, merges its rows.  A grid up to twice what the device holds at once
 // runs as fused2_kernel (two row blocks per workgroup, one after the other);
-// a larger one as prompt_kernel then node_merge_kernel -- the same bits.
+// a larger one as prompt_kernel, then node_block_kernel (64 rows a workgroup)
+// or node_merge_kernel (8) -- the same bits.
 //   Rows are packed GQA-wise (row = query * GQA + head-in-group), so a kv
 //   head's K/V is read once from HBM for all query heads that share it.  With
 //   8 kv heads, workgroup g of kernel A lands on XCD g (round-robin dispatch),
@@ -1599,6 +1600,339 @@ __global__ __launch_bounds__(64 * kWavesA) void node_merge_kernel(TrieAttnArgs A
   merge_rounds<D, false>(A, g, p0, rend, np, w);
 }
 
+// ------------------------------------------------------------------ many rows: nodes and merge
+// The node partials and the merge of calls with many rows and a long node
+// segment (prefill chunks, wide tries): workgroup (g, rb) takes rows [64 rb, +64)
+// of kv head g, wave w the 16 rows of tile w / 2 and half w % 2 of the head_dim
+// tiles.  The arithmetic of a row is node_rows': the exact maximum over the
+// allowed slots, then the allowed slots in slot order in tiles of kNodeTile ranks.
+//
+// Where the allowed slots of a row begin with an unbroken run -- committed tokens,
+// which every row sees, or the whole of a causal row -- rank r of that run is slot
+// r for every row, so one staged K/V tile and one pair of MFMAs serve 16 rows of
+// any queries (a rank past a row's count has p = 0).  Such tiles [0, tend) are
+// taken from K/V chunks staged once per workgroup; the ranks beyond them are
+// gathered query by query, as in node_task.  p = 0 leaves a row's sums alone only
+// if V is finite, so where a shared tile reaches past some row's count the V rows
+// are checked first, and any infinity or NaN sends the block to the gathered form.
+//
+// What bounded the calls: node_merge_kernel takes 8 rows a workgroup, each
+// workgroup reading the whole segment twice and gathering every tile query by
+// query, a memory round trip per tile, on 2 of its 8 waves.
+template <int D>
+struct BlockLds {
+  static constexpr int CB = kChunk * 2 * D;     // one chunk's K (or V)
+  static constexpr int KOFF = 0;                // two chunks of K, two of V; the gathered form's V stages
+  static constexpr int VOFF = 2 * CB;
+  static constexpr int STAGE = kNodeTile * 2 * D;   // one wave's gathered V rows
+  static_assert(kWavesA * STAGE <= 4 * CB, "stages fit the chunk buffers");
+  static constexpr int MWS = (kMaxNodeSlots / kChunk + 1) * 8;   // mask words of a query, padded against bank conflicts
+  static constexpr int MWOFF = 4 * CB;
+  static constexpr int TOFF = MWOFF + 64 * MWS;           // rank -> slot tables, one per wave
+  static constexpr int MXOFF = TOFF + kWavesA * kRankTab * 2;
+  static constexpr int INFOFF = MXOFF + kWavesA * 16 * 4;    // [64 queries] n, tiles of the run, last slot + 1
+  static constexpr int FLAGOFF = INFOFF + 64 * 16;
+  static constexpr int BYTES = FLAGOFF + 16;
+  static_assert(BYTES <= 160 * 1024, "LDS budget");
+};
+
+__device__ __forceinline__ int wave_min(int v) {
+#pragma unroll
+  for (int s = 32; s >= 1; s >>= 1) v = min(v, shfl_idx_i(v, __lane_id() ^ s));
+  return __builtin_amdgcn_readfirstlane(v);
+}
+
+// Chunk c (kChunk slots) of kv head g's node K as score fragments, and with VALS
+// its V rows, into buffers b (the layouts of NodeLds); slots past NN read zeros.
+template <int D, bool VALS>
+__device__ __forceinline__ void block_issue(const TrieAttnArgs& A, int g, int c, lds_char* kv, int b, int w) {
+  using LY = BlockLds<D>;
+  constexpr int DQ = D / 32, RB = 2 * D, KX = LY::CB / 1024;
+  const int lane = __lane_id();
+  const int c0 = c * kChunk, left = A.NN - c0 - 1;
+  const __amdgpu_buffer_rsrc_t rk = buffer_rsrc(A.kn + (g * A.sknh + c0 * A.sknn), 2 * (left * A.sknn + D));
+  const __amdgpu_buffer_rsrc_t rv = buffer_rsrc(A.vn + (g * A.svnh + c0 * A.svnn), 2 * (left * A.svnn + D));
+  for (int x = w; x < KX; x += kWavesA)
+    bdma16(rk, 2 * ((16 * (x / DQ) + (lane & 15)) * A.sknn + 32 * (x % DQ) + 8 * (lane >> 4)),
+           kv + LY::KOFF + b * LY::CB + x * 1024);
+  if constexpr (VALS) {
+    for (int x = w; x < KX; x += kWavesA) {
+      const int byte = x * 1024 + 16 * lane, row = byte / RB, u = (byte % RB) / 16;
+      bdma16(rv, 2 * row * A.svnn + 16 * (u ^ vswz<D>(row)), kv + LY::VOFF + b * LY::CB + x * 1024);
+    }
+  }
+}
+
+template <int D>
+__global__ __launch_bounds__(512) void node_block_kernel(TrieAttnArgs A) {
+  using LY = BlockLds<D>;
+  constexpr int DQ = D / 32, DT = D / 16, NJ = DT / 2, RB = 2 * D;
+  __shared__ __attribute__((aligned(16))) char lds[LY::BYTES];
+  lds_char* kv = (lds_char*)lds;
+  const int lane = __lane_id();
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int rt = w >> 1, dh = w & 1;
+  const int n16 = lane & 15, g4 = lane >> 4, e4 = n16 >> 2, c4 = n16 & 3;
+  const int g = blockIdx.x, row0 = 64 * blockIdx.y;
+  const int p0 = row0 + 16 * rt;                 // this wave's rows p0 + n16
+  const int q0 = row0 >> A.GQS;                  // the block's first query
+  const int nq = min(64 >> A.GQS, A.M - q0);     // and its queries
+  const int NN = A.NN, nch = (NN + kChunk - 1) / kChunk;
+  const RowRef R = row_ref(A, g, p0 + n16, row0);
+  const int ql = R.mq - q0;
+  typedef __attribute__((address_space(3))) int lds_int;
+  typedef __attribute__((address_space(3))) uint64_t lds_u64;
+  lds_int* info = (lds_int*)(kv + LY::INFOFF);
+  lds_int* flag = (lds_int*)(kv + LY::FLAGOFF);
+
+  bf16x8 qf[DQ];
+  node_q<D>(A, g, p0 < A.R ? p0 : row0, A.R, qf);
+
+  // Mask words, and per query the allowed count n, the tiles of its run (all of
+  // them when every allowed slot is in the run) and the slot after its last.
+  for (int qi = w; qi < nq; qi += kWavesA) {
+    const uint8_t* mrow = A.msk + (int64_t)(q0 + qi) * A.smm;
+    int n = 0, z = 0, last = 0;
+    bool run = true;
+    for (int cb = 0; cb < nch; cb += 8) {
+      uint8_t b[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) b[u] = mrow[(int64_t)min(kChunk * (cb + u) + lane, NN - 1) * A.smn];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const int c = cb + u;
+        const uint64_t mm = __builtin_amdgcn_ballot_w64(kChunk * c + lane < NN && b[u] != 0);
+        if (c >= nch) break;
+        if (lane == 0) *(lds_u64*)(kv + LY::MWOFF + qi * LY::MWS + 8 * c) = mm;
+        n += __builtin_popcountll(mm);
+        if (mm) last = kChunk * c + 64 - __builtin_clzll(mm);
+        if (run) {
+          z += ~mm ? __builtin_ctzll(~mm) : 64;
+          run = ~mm == 0;
+        }
+      }
+    }
+    if (lane == 0) {
+      info[4 * qi] = n;
+      info[4 * qi + 1] = n == z ? 0x7fffffff : z / kNodeTile;
+      info[4 * qi + 2] = last;
+    }
+  }
+  if (threadIdx.x == 0) *flag = 0;
+  lds_barrier();
+  const int ii = 4 * (lane < nq ? lane : 0);
+  const int nmin = wave_min(info[ii]), nmax = -wave_min(-info[ii]);
+  const int last = -wave_min(-info[ii + 2]);
+  int tend = min(wave_min(info[ii + 1]), (nmax + kNodeTile - 1) / kNodeTile);   // shared tiles
+  const int n = info[4 * ql];                                                   // this row's allowed slots
+  const lds_char* mw = kv + LY::MWOFF + ql * LY::MWS;
+
+  // The maxima, chunk by chunk: wave half dh scores slots [32 dh, +32) of a chunk.
+  const int nc1 = (last + kChunk - 1) / kChunk;
+  if (nc1 > 0) block_issue<D, false>(A, g, 0, kv, 0, w);
+  if (nmin < kNodeTile * tend) {
+    // A shared tile past some row's count: its V rows must be finite.
+    const __amdgpu_buffer_rsrc_t rv = buffer_rsrc(A.vn + g * A.svnh, 2 * ((NN - 1) * A.svnn + D));
+    uint32_t bad = 0;
+    const int units = min(kNodeTile * tend, NN) * (D / 8);
+    for (int x0 = threadIdx.x; x0 < units; x0 += 8 * 512) {
+      u32x4 v[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const int x = x0 + 512 * j;
+        v[j] = __builtin_bit_cast(
+            u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                       rv, x < units ? 2 * (x / (D / 8)) * A.svnn + 16 * (x % (D / 8)) : 0x7ffffff0, 0, 0));
+      }
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) bad |= ((v[j][e] & 0x7f807f80u) + 0x00800080u) & 0x80008000u;   // an all-ones exponent
+    }
+    if (__builtin_amdgcn_ballot_w64(bad != 0) != 0 && lane == 0) *flag = 1;
+  }
+  float x = kNegInf;
+  for (int c = 0; c < nc1; ++c) {
+    __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0): this wave's part of chunk c
+    lds_barrier();                        // every wave's part; every wave is done with chunk c - 1
+    if (c + 1 < nc1) block_issue<D, false>(A, g, c + 1, kv, (c + 1) & 1, w);
+    const lds_char* kb = kv + LY::KOFF + (c & 1) * LY::CB;
+    const uint64_t mm = *(const lds_u64*)(mw + 8 * c);
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) {
+      const int kt = 2 * dh + kk;
+      f32x4 sv = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int i = 0; i < DQ; ++i)
+        sv = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+            *(const __attribute__((address_space(3))) bf16x8*)(kb + (kt * DQ + i) * 1024 + 16 * lane), qf[i], sv, 0, 0, 0);
+      const uint32_t bits = (uint32_t)(mm >> (16 * kt + 4 * g4));
+#pragma unroll
+      for (int j = 0; j < 4; ++j) x = fmaxf(x, (bits >> j) & 1 ? sv[j] * A.c : kNegInf);
+    }
+  }
+  x = rows4_max(x);
+  lds_float* MX = (lds_float*)(kv + LY::MXOFF);
+  if (g4 == 0) MX[16 * w + n16] = x;
+  lds_barrier();
+  const float m = fmaxf(MX[16 * (w & ~1) + n16], MX[16 * (w | 1) + n16]);
+  if (__builtin_amdgcn_readfirstlane(*flag)) tend = 0;
+
+  const uint32_t one2 = 0x3f803f80u;   // two bf16 1.0
+  const bf16x8 ones = __builtin_bit_cast(bf16x8, u32x4{one2, one2, one2, one2});
+  f32x4 acc[NJ], lacc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int j = 0; j < NJ; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // One tile: p of the lane's ranks r0 + 16 kb + 4 g4 + j from the scores sc, V rows
+  // of ranks 4 g4 + e4 and 16 + 4 g4 + e4 at vr / swizzle vs.
+  auto tile = [&](const f32x4 (&sc)[2], int r0, int cnt, bool col, const lds_char* const (&vr)[2], const int (&vs)[2],
+                  f32x4 (&ac)[NJ], f32x4& lc) {
+    float pv[8];
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const bool on = col && r0 + 16 * kb + 4 * g4 + j < cnt;
+        pv[4 * kb + j] = on ? fexp2(sc[kb][j] * A.c - m) : 0.f;
+      }
+    u32x4 hw, lw;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      hw[i] = pack_bf16x2(pv[2 * i], pv[2 * i + 1]);
+      lw[i] = pack_bf16x2(pv[2 * i] - bf16_lo(hw[i]), pv[2 * i + 1] - bf16_hi(hw[i]));
+    }
+    const bf16x8 hop = __builtin_bit_cast(bf16x8, hw), lop = __builtin_bit_cast(bf16x8, lw);
+    bf16x8 vop[NJ];   // all requested before the first is used
+#pragma unroll
+    for (int jj = 0; jj < NJ; ++jj) {
+      const int b = 2 * (NJ * dh + jj) + (c4 >> 1);
+      const s16x4 lo = lds_read_tr(vr[0] + 16 * (b ^ vs[0]) + 8 * (c4 & 1));
+      const s16x4 hi = lds_read_tr(vr[1] + 16 * (b ^ vs[1]) + 8 * (c4 & 1));
+      vop[jj] = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+    }
+    __builtin_amdgcn_sched_group_barrier(0x100, 2 * NJ, 0);   // LDS reads
+#pragma unroll
+    for (int jj = 0; jj < NJ; ++jj) ac[jj] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vop[jj], hop, ac[jj], 0, 0, 0);
+#pragma unroll
+    for (int jj = 0; jj < NJ; ++jj) ac[jj] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vop[jj], lop, ac[jj], 0, 0, 0);
+    lc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, hop, lc, 0, 0, 0);
+    lc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, lop, lc, 0, 0, 0);
+  };
+
+  // The shared tiles, two per chunk.
+  const int nc2 = (tend + 1) / 2;
+  if (nc2 > 0) block_issue<D, true>(A, g, 0, kv, 0, w);
+  for (int c = 0; c < nc2; ++c) {
+    __builtin_amdgcn_s_waitcnt(0x0F70);
+    lds_barrier();
+    if (c + 1 < nc2) block_issue<D, true>(A, g, c + 1, kv, (c + 1) & 1, w);
+    const lds_char* kb0 = kv + LY::KOFF + (c & 1) * LY::CB;
+    const lds_char* vb0 = kv + LY::VOFF + (c & 1) * LY::CB;
+#pragma unroll
+    for (int hh = 0; hh < 2; ++hh) {
+      const int t = 2 * c + hh;
+      if (t >= tend) break;
+      f32x4 sc[2];
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb) {
+        sc[kb] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < DQ; ++i)
+          sc[kb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              *(const __attribute__((address_space(3))) bf16x8*)(kb0 + ((2 * hh + kb) * DQ + i) * 1024 + 16 * lane), qf[i],
+              sc[kb], 0, 0, 0);
+      }
+      const int rr0 = 32 * hh + 4 * g4 + e4, rr1 = rr0 + 16;
+      const lds_char* const vr[2] = {vb0 + rr0 * RB, vb0 + rr1 * RB};
+      const int vs[2] = {vswz<D>(rr0), vswz<D>(rr1)};
+      tile(sc, kNodeTile * t, n, R.live, vr, vs, acc, lacc);
+    }
+  }
+  // The ranks past the shared tiles, gathered query by query.
+  lds_barrier();   // every wave is done with the chunk buffers
+  const __amdgpu_buffer_rsrc_t rk = buffer_rsrc(A.kn + g * A.sknh, 2 * ((NN - 1) * A.sknn + D));
+  const __amdgpu_buffer_rsrc_t rv = buffer_rsrc(A.vn + g * A.svnh, 2 * ((NN - 1) * A.svnn + D));
+  lds_char* st = kv + w * LY::STAGE;
+  lds_i16* tab = (lds_i16*)(kv + LY::TOFF) + w * kRankTab;
+  const int qa = (16 * rt) >> A.GQS, qb = min(((16 * rt + 15) >> A.GQS) + 1, nq);
+  for (int qi = qa; qi < qb; ++qi) {
+    const int nn = __builtin_amdgcn_readfirstlane(info[4 * qi]);
+    if (nn <= kNodeTile * tend) continue;
+    const bool col = R.live && ql == qi;
+    f32x4 ac[NJ], lc = lacc;
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) ac[j] = acc[j];
+    int rc = tend / 2, rbase = kChunk * (tend / 2);   // ranks below 32 tend are slots below 32 tend
+    for (int r0 = kNodeTile * tend; r0 < nn; r0 += kNodeTile) {
+      rank_fill(rc, rbase, r0 + kNodeTile, nch, kv + LY::MWOFF + qi * LY::MWS, tab);
+      u32x4 kf[2][DQ];
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb) {
+        const int rr = r0 + 16 * kb + n16;
+        const int s = rr < nn ? tab[rr & (kRankTab - 1)] : 0;
+#pragma unroll
+        for (int i = 0; i < DQ; ++i)
+          kf[kb][i] = __builtin_bit_cast(
+              u32x4, __builtin_amdgcn_raw_buffer_load_b128(rk, 2 * (s * A.sknn + 32 * i + 8 * g4), 0, 0));
+      }
+#pragma unroll
+      for (int y = 0; y < LY::STAGE / 1024; ++y) {
+        const int byte = y * 1024 + 16 * lane, rr = byte / RB, u = (byte % RB) / 16;
+        const int s = r0 + rr < nn ? tab[(r0 + rr) & (kRankTab - 1)] : -1;
+        bdma16(rv, s >= 0 ? 2 * s * A.svnn + 16 * (u ^ vswz<D>(rr)) : 0x7ffffff0, st + y * 1024);
+      }
+      __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0): K fragments and this wave's V rows
+      asm volatile("" ::: "memory");
+      f32x4 sc[2];
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb) {
+        sc[kb] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < DQ; ++i)
+          sc[kb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, kf[kb][i]), qf[i], sc[kb], 0, 0, 0);
+      }
+      const int rr0 = 4 * g4 + e4, rr1 = rr0 + 16;
+      const lds_char* const vr[2] = {st + rr0 * RB, st + rr1 * RB};
+      const int vs[2] = {vswz<D>(rr0), vswz<D>(rr1)};
+      tile(sc, r0, nn, col, vr, vs, ac, lc);
+      __builtin_amdgcn_s_waitcnt(0xc07f);   // lgkmcnt(0): the stage and the table are read before they are written again
+      asm volatile("" ::: "memory");
+    }
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) acc[j] = col ? ac[j] : acc[j];
+    lacc = col ? lc : lacc;
+  }
+
+  // The groups of the prompt left to right, then the nodes (lane: row p0 + n16,
+  // head_dim 16 (NJ dh + j) + 4 g4 + e).
+  float fm = kNegInf, fl = 0.f, facc[4 * NJ], v[4 * NJ];
+#pragma unroll
+  for (int i = 0; i < 4 * NJ; ++i) facc[i] = 0.f;
+  for (int q = 0; q < A.NG; ++q) {
+    const size_t o = ((size_t)g * A.R + R.rr) * A.NG + q;
+    const f32x2 ml = *reinterpret_cast<const f32x2*>(A.gp_ml + 2 * o);
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      const f32x4 y = *reinterpret_cast<const f32x4*>(A.gp_acc + o * D + 16 * (NJ * dh + j) + 4 * g4);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[4 * j + e] = y[e];
+    }
+    combine<4 * NJ>(fm, fl, facc, ml.x, ml.y, v);
+  }
+#pragma unroll
+  for (int j = 0; j < NJ; ++j)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[4 * j + e] = acc[j][e];
+  combine<4 * NJ>(fm, fl, facc, m, lacc[0], v);
+  if (!R.live) return;
+#pragma unroll
+  for (int j = 0; j < NJ; ++j) {
+    uint16_t* o = A.out + out_offset<D>(A.soh, A.som, A.HK << A.GQS, R.hd, R.mq, 16 * (NJ * dh + j) + 4 * g4);
+    *reinterpret_cast<u32x2*>(o) = u32x2{pack_bf16x2(facc[4 * j] / fl, facc[4 * j + 1] / fl),
+                                         pack_bf16x2(facc[4 * j + 2] / fl, facc[4 * j + 3] / fl)};
+  }
+}
+
 // NaN in every element of rows [p0, rend) of kv head g (row p0 + w + 8 i on
 // wave w): the output of a workgroup whose wait for the group partials gave up.
 template <int D>
@@ -2030,6 +2364,18 @@ static void launch_rt(const TrieAttnArgs& a, const Plan& pl, hipStream_t s, int 
     return;
   }
   if (pl.prompt_wgs > 0) hipLaunchKernelGGL((prompt_kernel<D, RT>), dim3(a.HK, pl.NRB, pl.NG), dim3(64 * kWavesA), 0, s, a);
+  if constexpr (D <= 128) {
+    // Nodes and merge: 64-row blocks once they give a quarter of the CUs a workgroup
+    // (8B heads, causal rows after 2560 prompt keys: 130 rows 36.8 us for the call
+    // instead of 44.4 with node_merge_kernel, 192 rows 46.9 / 56.7, 512 rows 89 / 241;
+    // 8 q / 2 kv heads of 64, 320 rows, 40 blocks: 29.4 / 27.4, so below that
+    // node_merge_kernel's 8-row workgroups stay).
+    const int nrb64 = (pl.R + 63) / 64;
+    if (a.NN > 0 && nrb64 <= 65535 && a.HK * nrb64 >= 64) {
+      hipLaunchKernelGGL((node_block_kernel<D>), dim3(a.HK, nrb64), dim3(64 * kWavesA), 0, s, a);
+      return;
+    }
+  }
   hipLaunchKernelGGL((node_merge_kernel<D>), dim3(pl.node_wgs), dim3(64 * kWavesA), 0, s, a);
 }
 

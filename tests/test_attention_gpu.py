@@ -508,3 +508,60 @@ def test_tiled_output_rejects_a_head_stride_other_than_d():
     torch.cuda.synchronize()
     assert torch.all(out == 7.0)
     assert L.rspx_trie_attn(*args, D, _lib.RSPX_TILED, *tail) == 0
+
+
+@pytest.mark.parametrize("H,HK,D,M,P,mask", [
+    (32, 8, 128, 512, 2560, "causal"),     # a late prefill chunk: 7 key groups
+    (32, 8, 128, 300, 0, "causal"),        # the first chunk: no prompt; ragged rows and slots
+    (8, 2, 64, 333, 33, "causal"),         # one group of two steps
+    (16, 2, 32, 250, 5000, "causal"),      # GQA 8, 8 groups, a last group of 5 steps
+    (4, 4, 128, 200, 1025, "causal"),      # GQA 1: 64 queries a block
+    (32, 2, 64, 257, 1000, "causal"),      # GQA 16: 4 queries a block
+    (8, 2, 128, 224, 700, "open32k"),      # a common run of 96 slots, then slots of each row's own
+    (8, 2, 64, 300, 64, "random"),         # no common run
+    (8, 8, 128, 230, 40, "holes"),         # rows without any node slot, and causal rows
+    (8, 2, 128, 320, 100, "nan"),          # NaN / inf K and V in slots that later rows alone may see
+])
+def test_many_rows(H, HK, D, M, P, mask):
+    """Calls whose grid never fits the device at once (prompt part and node part in a launch
+    each; forced for the smaller ones): every checked row bit for bit what its call alone gives,
+    over causal masks, common runs of open slots with and without own slots after them, and
+    masked slots that hold NaN or infinities; rows and slots that end inside a tile."""
+    from _tiled import from_tiled
+    from respect_amd.kernels.attention import trie_attn
+    print(f"[many rows] H={H} HK={HK} D={D} M={M} P={P} {mask}", flush=True)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(M + P + D)
+    NN = -(-M // 32) * 32
+
+    def rnd(*s):
+        return torch.randn(*s, generator=g, device="cuda").to(torch.bfloat16)
+
+    q, kp, vp, kn, vn = rnd(H, M, D), rnd(HK, P, D), rnd(HK, P, D), rnd(HK, NN, D), rnd(HK, NN, D)
+    msk = torch.ones(M, NN, dtype=torch.bool, device="cuda").tril()
+    own = torch.rand(M, NN, generator=g, device="cuda") < 0.2
+    if mask == "open32k":
+        msk = own.clone()
+        msk[:, :97] = True
+        msk[0, 99:] = False
+    elif mask == "random":
+        msk = own.clone()
+        msk[:, 0] = True
+    elif mask == "holes":
+        msk[::7] = False
+    elif mask == "nan":
+        kn[:, 290], vn[:, 290] = float("nan"), float("inf")
+        vn[:, 301] = float("nan")
+    def same(a, b):   # bit for bit; NaN equals NaN
+        return torch.equal(a.isnan(), b.isnan()) and torch.equal(a.nan_to_num(0.0), b.nan_to_num(0.0))
+
+    out = trie_attn(q, kp, vp, kn, vn, msk, launches=2)
+    assert same(trie_attn(q, kp, vp, kn, vn, msk), out)
+    assert out[:, :290].isfinite().all()
+    tiled = torch.zeros(-(-M // 64) * 64 * H * D, dtype=torch.bfloat16, device="cuda")
+    trie_attn(q, kp, vp, kn, vn, msk, out=tiled, out_tiled=True)
+    assert same(from_tiled(tiled, M, H * D).view(M, H, D), out.transpose(0, 1))
+    for m in sorted({0, 1, 15, 16, 31, 32, 63, 64, 95, 97, 128, 191, 192, M // 2, M - 32, M - 2, M - 1}):
+        n = NN if P else min(NN, -(-(m + 1) // 32) * 32)   # without a prompt: a shorter node segment, held whole
+        one = trie_attn(q[:, m:m + 1], kp, vp, kn[:, :n], vn[:, :n], msk[m:m + 1, :n], launches=1 if P else 2)
+        assert same(one[:, 0], out[:, m]), f"row {m}"
