@@ -48,9 +48,10 @@
 // counts itself, computes the node partials of its share of the block's rows
 // (MFMA scores and rank-tiled MFMA sums) and, once the block's groups are all
 // counted, merges its rows.  A grid up to twice what the device holds at once
-// runs as fused2_kernel (two row blocks per workgroup, one after the other);
-// a larger one as prompt_kernel, then node_block_kernel (64 rows a workgroup)
-// or node_merge_kernel (8) -- the same bits.
+// runs as fused_pair_kernel (128-row blocks; at D = 256 fused2_kernel, two row
+// blocks one after the other); a larger one as prompt_pair_kernel (D = 256:
+// prompt_kernel), then node_block_kernel (64 rows a workgroup) or
+// node_merge_kernel (8) -- the same bits.
 //   Rows are packed GQA-wise (row = query * GQA + head-in-group), so a kv
 //   head's K/V is read once from HBM for all query heads that share it.  With
 //   8 kv heads, workgroup g of kernel A lands on XCD g (round-robin dispatch),
@@ -324,6 +325,56 @@ struct PromptLds {
   static_assert(BYTES + MLBYTES <= 160 * 1024, "LDS budget");
 };
 
+// Wave w's chunks of a round: c = w + 8 j, step-in-round c / CH, chunk c % CH.
+// voff[t] is the lane's byte offset of chunk w + 8 t (mod CH) relative to the
+// step's first key.
+template <int D> constexpr int chunk_voffs() { return StepGeom<D>::CH >= kWavesA ? StepGeom<D>::CH / kWavesA : 1; }
+template <int D>
+__device__ __forceinline__ void chunk_offsets(const TrieAttnArgs& A, int w, int (&voff)[chunk_voffs<D>()]) {
+  using G = StepGeom<D>;
+  const int lane = __lane_id();
+#pragma unroll
+  for (int t = 0; t < chunk_voffs<D>(); ++t) {
+    const int cc = (w + kWavesA * t) % G::CH;
+    if (cc < G::KCH) {
+      const int key = G::KPV * cc + lane / G::U;
+      const int b = (lane % G::U) ^ kswz<D>(key);
+      voff[t] = 2 * key * A.skpn + 16 * b;
+    } else {
+      const int key = G::KPV * (cc - G::KCH) + lane / G::U;
+      const int b = (lane % G::U) ^ vswz<D>(key);
+      voff[t] = 2 * key * A.svpn + 16 * b;
+    }
+  }
+}
+
+// The lane's LDS offsets inside a step slot: transposing-read addresses of the V
+// operand halves (keys 4 g4 + e and 16 + 4 g4 + e) for head_dim tile j, and
+// A-fragment addresses of the K operand (lane (n16, g4) reads key 16 kb + n16,
+// head_dim [32 i + 8 g4, +8) = 16-byte unit 4 i + g4).
+template <int D>
+__device__ __forceinline__ void slot_offsets(int (&trv)[2][StepGeom<D>::DT], int (&kro)[2][StepGeom<D>::DQ]) {
+  using G = StepGeom<D>;
+  const int lane = __lane_id(), n16 = lane & 15, g4 = lane >> 4;
+  const int e = n16 >> 2, c4 = n16 & 3;
+#pragma unroll
+  for (int kh = 0; kh < 2; ++kh) {
+    const int key = 16 * kh + 4 * g4 + e;
+#pragma unroll
+    for (int j = 0; j < G::DT; ++j) {
+      const int b = 2 * j + (c4 >> 1);
+      trv[kh][j] = G::KBYTES + 16 * (key * G::U + (b ^ vswz<D>(key))) + 8 * (c4 & 1);
+    }
+  }
+#pragma unroll
+  for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+    for (int i = 0; i < G::DQ; ++i) {
+      const int key = 16 * kb + n16;
+      kro[kb][i] = 16 * (key * G::U + ((4 * i + g4) ^ kswz<D>(key)));
+    }
+}
+
 // One step of 32 keys from first key ks, K/V in LDS at `slot`, for the wave's kRT
 // row tiles: scores, online softmax against the lazily moved reference maximum,
 // and the PV product.  kro / trv: the lane's LDS offsets of the K fragments and of
@@ -476,53 +527,13 @@ __device__ __forceinline__ void prompt_block(const TrieAttnArgs& A, char* lds, i
     dma16(A.q + (((g << A.GQS) + jh) * A.sqh + mq * A.sqm + 32 * i + 8 * g4), qreg + c * 1024);
   }
 
-  // This wave's chunks of a round: c = w + 8 j, step-in-round c / CH, chunk
-  // c % CH.  voff[t] is the lane's byte offset of chunk w + 8 t (mod CH)
-  // relative to the step's first key.
-  constexpr int NV = G::CH >= kWavesA ? G::CH / kWavesA : 1;
+  constexpr int NV = chunk_voffs<D>();
   int voff[NV];
-#pragma unroll
-  for (int t = 0; t < NV; ++t) {
-    const int cc = (w + kWavesA * t) % G::CH;
-    if (cc < G::KCH) {
-      const int key = G::KPV * cc + lane / G::U;
-      const int b = (lane % G::U) ^ kswz<D>(key);
-      voff[t] = 2 * key * A.skpn + 16 * b;
-    } else {
-      const int key = G::KPV * (cc - G::KCH) + lane / G::U;
-      const int b = (lane % G::U) ^ vswz<D>(key);
-      voff[t] = 2 * key * A.svpn + 16 * b;
-    }
-  }
+  chunk_offsets<D>(A, w, voff);
   const uint16_t* kpg = A.kp + g * A.skph;
   const uint16_t* vpg = A.vp + g * A.svph;
-
-  // Transposing-read addresses of the V operand halves (keys 4 g4 + e and
-  // 16 + 4 g4 + e) for head_dim tile j, relative to a step slot.
-  int trv[2][DT];
-  {
-    const int e = n16 >> 2, c4 = n16 & 3;
-#pragma unroll
-    for (int kh = 0; kh < 2; ++kh) {
-      const int key = 16 * kh + 4 * g4 + e;
-#pragma unroll
-      for (int j = 0; j < DT; ++j) {
-        const int b = 2 * j + (c4 >> 1);
-        trv[kh][j] = G::KBYTES + 16 * (key * G::U + (b ^ vswz<D>(key))) + 8 * (c4 & 1);
-      }
-    }
-  }
-
-  // A-fragment addresses of the K operand: lane (n16, g4) reads key
-  // 16 kb + n16, head_dim [32 i + 8 g4, +8) = 16-byte unit 4 i + g4.
-  int kro[2][DQ];
-#pragma unroll
-  for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-    for (int i = 0; i < DQ; ++i) {
-      const int key = 16 * kb + n16;
-      kro[kb][i] = 16 * (key * G::U + ((4 * i + g4) ^ kswz<D>(key)));
-    }
+  int trv[2][DT], kro[2][DQ];
+  slot_offsets<D>(trv, kro);
 
   float mref[kRT], lrow[kRT];
   f32x4 acc[kRT][DT];
@@ -700,6 +711,188 @@ template <int D, int kRT>
 __global__ __launch_bounds__(512) void prompt_kernel(TrieAttnArgs A) {
   __shared__ __attribute__((aligned(16))) char lds[PromptLds<D, kRT>::BYTES];
   prompt_block<D, kRT, false, true>(A, lds, blockIdx.x, blockIdx.y, blockIdx.z, [] {}, [] {}, [] {});
+}
+
+// ------------------------------------------------------------------ 128-row blocks
+// The prompt work of a block of 128 rows, for calls with more rows than one
+// 64-row block per workgroup covers: rows [128 rb, +128) of kv head g, key group q,
+// up to the group partial in memory.  Wave w: rows 32 (w / 2) of the block (two
+// tiles) and the key quarters 2 p, 2 p + 1 (p = w % 2), each with its own
+// softmax state; the arithmetic and the order of every sum are prompt_block's.
+//
+// Why: with 64-row blocks a workgroup reads 64 KB of K/V per round of four steps
+// through L2 for 64 rows, and the 256 workgroups of a long call drew about
+// 12 TB/s from the L2s, whatever they computed (a round took 1.4 us).  A block of
+// 128 rows halves those bytes.  Two quarters per wave instead of one keep a wave at
+// 32 rows (one K or V fragment read from LDS per two MFMAs), and their sum needs no
+// exchange: only half a pair's sum crosses to the other wave.
+template <int D>
+struct PairLds {
+  using G = StepGeom<D>;
+  static constexpr int RINGBYTES = G::RING * G::ROUND;
+  static constexpr int MLBYTES = 4 * kQuarters * 2 * 16 * 8;   // [4 row groups][quarter][tile][16 rows] (m, l)
+  static constexpr int BYTES = RINGBYTES + MLBYTES;
+  static constexpr int BOX = 32 * D * 2;                       // 32 rows x D / 2 floats, one per wave
+  static_assert(kWavesA * BOX <= RINGBYTES && BYTES <= 160 * 1024, "LDS budget");
+};
+
+template <int D, bool ATOMIC, class Hook>
+__device__ __forceinline__ void pair_block(const TrieAttnArgs& A, char* lds, int g, int rb, int q,
+                                           const Hook& before_stores) {
+  using G = StepGeom<D>;
+  using L = PairLds<D>;
+  constexpr int kRT = 2, DQ = G::DQ, DT = G::DT, HT = DT / 2;
+  typedef __attribute__((address_space(3))) f32x2 lds_f32x2;
+  typedef __attribute__((address_space(3))) f32x4 lds_f32x4;
+  lds_char* ring = (lds_char*)lds;
+  lds_char* ml = ring + L::RINGBYTES;
+  const int lane = __lane_id();
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int h = w >> 1, p = w & 1;
+  const int n16 = lane & 15, g4 = lane >> 4;
+  const int P = A.P;
+  const int steps = (P + kStep - 1) / kStep;
+  const int s0 = q * A.S;
+  const int ns = min(A.S, steps - s0);
+  const int nr = (ns + kQuarters - 1) / kQuarters;
+  const int trow = 128 * rb + 32 * h;
+  const bool has_rows = trow < A.R;
+
+  int voff[chunk_voffs<D>()];
+  chunk_offsets<D>(A, w, voff);
+  const int ks0 = s0 * kStep;
+  const __amdgpu_buffer_rsrc_t rk =
+      buffer_rsrc(A.kp + (g * A.skph + ks0 * A.skpn), 2 * ((P - ks0 - 1) * A.skpn + D));
+  const __amdgpu_buffer_rsrc_t rv =
+      buffer_rsrc(A.vp + (g * A.svph + ks0 * A.svpn), 2 * ((P - ks0 - 1) * A.svpn + D));
+  const int kstep = 2 * kStep * A.skpn, vstep = 2 * kStep * A.svpn;
+  issue_round<D>(rk, rv, kstep, vstep, 0, voff, ring, w);
+
+  // Q fragments straight from memory (rows past R read row 0 and are never stored).
+  bf16x8 qop[kRT][DQ];
+#pragma unroll
+  for (int t = 0; t < kRT; ++t) {
+    const int r = trow + 16 * t + n16, rc = r < A.R ? r : 0;
+    const int mq = rc >> A.GQS, jh = rc & ((1 << A.GQS) - 1);
+    const uint16_t* qp = A.q + (((g << A.GQS) + jh) * A.sqh + mq * A.sqm + 8 * g4);
+#pragma unroll
+    for (int i = 0; i < DQ; ++i) qop[t][i] = *reinterpret_cast<const bf16x8*>(qp + 32 * i);
+  }
+  int trv[2][DT], kro[2][DQ];
+  slot_offsets<D>(trv, kro);
+  float mref[2][kRT], lrow[2][kRT];
+  f32x4 acc[2][kRT][DT];
+#pragma unroll
+  for (int u = 0; u < 2; ++u)
+#pragma unroll
+    for (int t = 0; t < kRT; ++t) {
+      mref[u][t] = kNegInf;
+      lrow[u][t] = 0.f;
+#pragma unroll
+      for (int j = 0; j < DT; ++j) acc[u][t][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+
+  for (int r = 0; r < nr; ++r) {
+    wait_rounds<G::OWN, G::RING>(r == 0 ? 0 : min(nr - 1 - r, G::RING - 1));
+    lds_barrier();   // every wave's chunks of round r are in LDS
+    if (r == 0) {
+      for (int rr = 1; rr < min(nr, G::RING); ++rr)
+        issue_round<D>(rk, rv, kstep, vstep, kQuarters * rr, voff, ring + rr * G::ROUND, w);
+    }
+    const lds_char* slot = ring + (r % G::RING) * G::ROUND;
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int sl = kQuarters * r + 2 * p + u;
+      if (has_rows && sl < ns)
+        prompt_step<D, kRT>(A, slot + (2 * p + u) * G::SLOT, (s0 + sl) * kStep, kro, trv, qop, mref[u], lrow[u], acc[u]);
+    }
+    if (r + G::RING < nr) {
+      lds_barrier();   // round r is consumed by every wave
+      issue_round<D>(rk, rv, kstep, vstep, kQuarters * (r + G::RING), voff, ring + (r % G::RING) * G::ROUND, w);
+    }
+  }
+
+  // The quarters combined as in prompt_block: scaled to the row's maximum M over
+  // them, (q0 + q1) + (q2 + q3).  A wave adds its own two, hands the half of the
+  // head_dim tiles it does not keep to the other wave of its rows, and stores
+  // tiles [HT p, +HT) of the sum.
+  if (g4 == 0) {
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int t = 0; t < kRT; ++t)
+        *(lds_f32x2*)(ml + (((kQuarters * h + 2 * p + u) * kRT + t) * 16 + n16) * 8) = f32x2{mref[u][t], lrow[u][t]};
+  }
+  lds_barrier();   // (m, l) written; every wave is past its last step
+  float Mr[kRT], Lr[kRT];
+  lds_char* box = ring + w * L::BOX + 16 * lane;
+#pragma unroll
+  for (int t = 0; t < kRT; ++t) {
+    float mk[4], lk[4], sk[4];
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk) {
+      const f32x2 v = *(const lds_f32x2*)(ml + (((kQuarters * h + kk) * kRT + t) * 16 + n16) * 8);
+      mk[kk] = v.x;
+      lk[kk] = v.y;
+    }
+    const float M = fmaxf(fmaxf(mk[0], mk[1]), fmaxf(mk[2], mk[3]));
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk) sk[kk] = mk[kk] == kNegInf ? 0.f : fexp2(mk[kk] - M);
+    Mr[t] = M;
+    Lr[t] = (lk[0] * sk[0] + lk[1] * sk[1]) + (lk[2] * sk[2] + lk[3] * sk[3]);
+    const float sa = p ? sk[2] : sk[0], sb = p ? sk[3] : sk[1];
+#pragma unroll
+    for (int j = 0; j < DT; ++j) acc[0][t][j] = acc[0][t][j] * sa + acc[1][t][j] * sb;
+  }
+  // Branches with constant indices: a run-time choice between accumulators would
+  // put them in scratch memory.
+  f32x4 sv[kRT][HT];
+#pragma unroll
+  for (int t = 0; t < kRT; ++t)
+#pragma unroll
+    for (int j = 0; j < HT; ++j) {
+      f32x4 give;
+      if (p) {
+        give = acc[0][t][j];
+        sv[t][j] = acc[0][t][HT + j];
+      } else {
+        give = acc[0][t][HT + j];
+        sv[t][j] = acc[0][t][j];
+      }
+      *(lds_f32x4*)(box + (t * HT + j) * 1024) = give;
+    }
+  lds_barrier();
+  const lds_char* other = ring + (w ^ 1) * L::BOX + 16 * lane;
+#pragma unroll
+  for (int t = 0; t < kRT; ++t)
+#pragma unroll
+    for (int j = 0; j < HT; ++j) sv[t][j] = sv[t][j] + *(const lds_f32x4*)(other + (t * HT + j) * 1024);
+  lds_barrier();   // every wave's ring reads are complete: before_stores may load into it
+  before_stores();
+  const __amdgpu_buffer_rsrc_t racc = buffer_rsrc(A.gp_acc, 0x7fffffff);
+#pragma unroll
+  for (int t = 0; t < kRT; ++t) {
+    const int r = trow + 16 * t + n16;
+    if (r >= A.R) continue;
+    const size_t mo = ((size_t)g * A.R + r) * A.NG + q;   // (m, l) pair index
+    if (p == 0 && g4 == 0) {
+      if constexpr (ATOMIC)
+        __builtin_amdgcn_raw_buffer_store_b64(f32x2{Mr[t], Lr[t]}, buffer_rsrc(A.gp_ml, 0x7fffffff), (int)(mo * 8), 0, 16);
+      else *reinterpret_cast<f32x2*>(A.gp_ml + 2 * mo) = f32x2{Mr[t], Lr[t]};
+    }
+#pragma unroll
+    for (int j = 0; j < HT; ++j) {
+      const size_t off = mo * D + 16 * (HT * p + j) + 4 * g4;
+      if constexpr (ATOMIC) __builtin_amdgcn_raw_buffer_store_b128(sv[t][j], racc, (int)(off * 4), 0, 16);
+      else *reinterpret_cast<f32x4*>(A.gp_acc + off) = sv[t][j];
+    }
+  }
+}
+
+template <int D>
+__global__ __launch_bounds__(512) void prompt_pair_kernel(TrieAttnArgs A) {
+  __shared__ __attribute__((aligned(16))) char lds[PairLds<D>::BYTES];
+  pair_block<D, false>(A, lds, blockIdx.x, blockIdx.y, blockIdx.z, [] {});
 }
 
 // ------------------------------------------------------------------ node partials and merge
@@ -2013,15 +2206,15 @@ static_assert((kCountUnit & (kCountUnit - 1)) == 0, "2^32 is a multiple of the u
 template <int kRT>
 __device__ __forceinline__ void merge_share(const TrieAttnArgs& A, int rb, int q, int& r0, int& rend) {
   const int rows_blk = 32 * kRT;
-  // ceil(rows_blk / 4 / NG) for NG = 1 .. kGroupTarget, 5 bits each: no division.
+  // ceil(rows_blk / 4 / NG) for NG = 1 .. kGroupTarget, 6 bits each: no division.
   constexpr int a = rows_blk / 4;
   constexpr uint64_t tab = [] {
     uint64_t t = 0;
-    for (int n = 1; n <= kGroupTarget; ++n) t |= (uint64_t)((a + n - 1) / n) << (5 * n);
+    for (int n = 1; n <= kGroupTarget; ++n) t |= (uint64_t)((a + n - 1) / n) << (6 * n);
     return t;
   }();
-  static_assert(a < 32, "5-bit table entries");
-  const int rpw = 4 * (int)((tab >> (5 * A.NG)) & 31);
+  static_assert(a < 64 && 6 * (kGroupTarget + 1) <= 64, "6-bit table entries");
+  const int rpw = 4 * (int)((tab >> (6 * A.NG)) & 63);
   r0 = rb * rows_blk + q * rpw;
   rend = min(rb * rows_blk + min(rows_blk, (q + 1) * rpw), A.R);
 }
@@ -2169,17 +2362,16 @@ __global__ __launch_bounds__(512) void fused_kernel(TrieAttnArgs A) {
   block_tail<D, kRT>(A, lds, g, rb, q, r0, rend, pre, pf, old);
 }
 
-// The same work as fused_kernel for grids twice as large as the device holds
-// at once (e.g. 128-node tries at 8B heads: 512 rows per kv head): workgroup
-// (g, rbw, q) runs the prompt groups of row blocks rbw and rbw + NRBW
-// (NRBW = ceil(NRB / 2)) one after the other, counting each, then the node
-// partials and merges of its merge rows (its shares of both blocks, or with
-// NG = 2, 4 or 8 twice a share of one block).  Every count precedes every
-// wait, so the waits end as in fused_kernel; the arithmetic of every row is
-// the same: the same bits.
+// The same work as fused_kernel for grids twice as large as the device holds at
+// once, at D = 256 (fused_pair_kernel's accumulators do not fit the registers
+// there): workgroup (g, rbw, q) runs the prompt groups of row blocks rbw and
+// rbw + NRBW (NRBW = ceil(NRB / 2)) one after the other, counting each, then the
+// node partials and merges of its merge rows (its shares of both blocks, or with
+// NG = 2, 4 or 8 twice a share of one block).  Every count precedes every wait, so
+// the waits end as in fused_kernel; the arithmetic of every row is the same: the
+// same bits.
 template <int D, int kRT>
 __global__ __launch_bounds__(512) void fused2_kernel(TrieAttnArgs A) {
-  using LY = NodeLds<D>;
   using PL = PromptLds<D, kRT>;
   constexpr int NB = node_area_bytes<D>() + 16;
   constexpr int LB = PL::BYTES + PL::MLBYTES > NB ? PL::BYTES + PL::MLBYTES : NB;
@@ -2197,14 +2389,7 @@ __global__ __launch_bounds__(512) void fused2_kernel(TrieAttnArgs A) {
   // With two blocks and NG = 2, 4 or 8 the merges are split by workgroup, not
   // by block: workgroup q merges 2 (32 kRT) / NG consecutive rows of one block
   // (block rbw for q < NG / 2, block rb1 above), so it has one node phase, one
-  // wait and one merge for twice the rows of a block's share.  With a resident
-  // node segment (up to D = 128) its node data is requested during the second
-  // block's prompt part: the first chunk's K/V into registers before that
-  // block's quarter combine (written into the ring after it, further chunks as
-  // direct-to-LDS loads) with the rows' mask bytes, and the score fragment from
-  // memory (rows of block rbw) or from the second block's Q fragments, kept in
-  // LDS (rows of block rb1).
-  constexpr bool kEarly = D <= 128;
+  // wait and one merge for twice the rows of a block's share.
   const int rows_blk = 32 * kRT;
   const bool pairs = nb > 1 && (A.NG == 2 || A.NG == 4 || A.NG == 8);
   const bool second = pairs && q >= (A.NG >> 1);
@@ -2215,45 +2400,19 @@ __global__ __launch_bounds__(512) void fused2_kernel(TrieAttnArgs A) {
     m0 = mrb * rows_blk + (second ? q - (A.NG >> 1) : q) * rpw2;
     mend = min(m0 + rpw2, A.R);
   }
-  const int mend0 = min(mend, m0 + kNodeRows);
-  const bool pf = kEarly && pairs && A.NN > 0 && A.NN <= LY::RES * kChunk && m0 < mend;
-  NodePre<D> pre;
-  u32x4 pc[node_pieces<D>()];
-  const lds_char* qreg = (const lds_char*)lds + PL::RINGBYTES;
+  NodePre<D> none;
   prompt_block<D, kRT, true, true>(A, lds, g, rbw, q, [] {}, [] {}, [] {});
   // With a second block the first block's count waits for nothing: it is added
   // once the second block's round 0 has landed, by when the first block's
   // stores (issued before that round's loads) are complete in every wave.
   if (nb == 1) count_partial(A, g, rbw, q);
   if (nb > 1) {
-    prompt_block<D, kRT, true, false, true>(
-        A, lds, g, rb1, q,
-        [&] {
-          if constexpr (kEarly) {
-            // Unconditional, so that no path leaves the register loads pending.
-            node_put<D>(A, g, 0, (lds_char*)lds, 0, pc, w);
-            if (!pf) return;
-            for (int b = 1; b < LY::RES && b * kChunk < A.NN; ++b) node_issue<D>(A, g, b * kChunk, (lds_char*)lds, b, w);
-          }
-        },
-        [&] {
-          if constexpr (kEarly) {
-            if (pf) {
-              node_load<D>(A, g, 0, pc, w);
-              node_prefetch_masks<D>(A, m0, mend0, w, pre);
-              if (!second) node_q<D>(A, g, m0, mend0, pre.qf);
-            }
-          }
-        },
-        [&] { count_add(A, g, rbw, q); });
+    prompt_block<D, kRT, true, true>(A, lds, g, rb1, q, [] {}, [] {}, [&] { count_add(A, g, rbw, q); });
     count_partial(A, g, rb1, q);
-    if constexpr (kEarly)
-      if (pf && second) node_q_lds<D>(qreg, rb1 * rows_blk, m0, mend0, pre.qf);
   }
   if (pairs) {
-    block_tail<D, kRT>(A, lds, g, mrb, q, m0, mend, pre, pf, second ? old[1] : old[0]);
+    block_tail<D, kRT>(A, lds, g, mrb, q, m0, mend, none, false, second ? old[1] : old[0]);
   } else {
-    NodePre<D> none;
     int r0, rend;
     merge_share<kRT>(A, rbw, q, r0, rend);
     block_tail<D, kRT>(A, lds, g, rbw, q, r0, rend, none, false, old[0]);
@@ -2262,6 +2421,34 @@ __global__ __launch_bounds__(512) void fused2_kernel(TrieAttnArgs A) {
       block_tail<D, kRT>(A, lds, g, rb1, q, r0, rend, none, false, old[1]);
     }
   }
+}
+
+// The same work as fused_kernel with 128-row blocks (pair_block), for grids up to
+// twice as large as the device holds at once in 64-row blocks (e.g. 128-node
+// tries at 8B heads: 512 rows per kv head): A.NRB counts 128-row blocks.
+template <int D>
+__global__ __launch_bounds__(512) void fused_pair_kernel(TrieAttnArgs A) {
+  using LY = NodeLds<D>;
+  using PL = PairLds<D>;
+  constexpr int NB = node_area_bytes<D>() + 16;
+  static_assert(NB <= PL::RINGBYTES, "node LDS and the wait flag inside the ring");
+  __shared__ __attribute__((aligned(16))) char lds[PL::BYTES];
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int g = blockIdx.x, rb = blockIdx.y, q = blockIdx.z;
+  // Every argument the prologue needs, requested in one batch.
+  asm volatile("" ::"s"(A.q), "s"(A.kp), "s"(A.vp), "s"(A.sync), "s"(A.sqh), "s"(A.sqm), "s"(A.skph), "s"(A.skpn),
+               "s"(A.svph), "s"(A.svpn), "s"(A.P), "s"(A.NRB), "s"(A.NG), "s"(A.S), "s"(A.R), "s"(A.GQS));
+  int r0, rend;
+  merge_share<4>(A, rb, q, r0, rend);
+  const int rend0 = min(rend, r0 + kNodeRows);               // the first batch of node rows
+  const int old = counter_before(A, g, rb);
+  const bool pf = A.NN > 0 && A.NN <= LY::RES * kChunk && r0 < rend;
+  NodePre<D> pre;
+  pair_block<D, true>(A, lds, g, rb, q, [&] {
+    if (pf) node_prefetch<D>(A, g, r0, rend0, (lds_char*)lds, w, pre);
+  });
+  count_partial(A, g, rb, q);
+  block_tail<D, 4>(A, lds, g, rb, q, r0, rend, pre, pf, old);
 }
 
 // ------------------------------------------------------------------ host side
@@ -2325,8 +2512,8 @@ static int make_plan(int H, int HK, int M, int P, int NN, int D, int rows_per_wa
   return RSPX_OK;
 }
 
-// Workgroups of fused_kernel<D, RT> (TWO: fused2_kernel<D, RT>) the device
-// holds at once (0 if unknown).
+// Workgroups of fused_kernel<D, RT> (TWO: fused_pair_kernel<D>, or at D = 256
+// fused2_kernel<D, RT>) the device holds at once (0 if unknown).
 template <int D, int RT, bool TWO>
 static int fused_capacity() {
   static int cap[64];
@@ -2336,7 +2523,8 @@ static int fused_capacity() {
   if (!done[dev]) {
     int a = 0, cus = 0;
     hipError_t e;
-    if constexpr (TWO) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&a, fused2_kernel<D, RT>, 64 * kWavesA, 0);
+    if constexpr (TWO && D <= 128) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&a, fused_pair_kernel<D>, 64 * kWavesA, 0);
+    else if constexpr (TWO) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&a, fused2_kernel<D, RT>, 64 * kWavesA, 0);
     else e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&a, fused_kernel<D, RT>, 64 * kWavesA, 0);
     if (e != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) {
       a = cus = 0;
@@ -2357,13 +2545,27 @@ static void launch_rt(const TrieAttnArgs& a, const Plan& pl, hipStream_t s, int 
     hipLaunchKernelGGL((fused_kernel<D, RT>), dim3(a.HK, pl.NRB, pl.NG), dim3(64 * kWavesA), 0, s, a);
     return;
   }
-  // Two row blocks per workgroup (fused2_kernel) when that grid fits.
-  const int wgs2 = a.HK * ((pl.NRB + 1) / 2) * pl.NG;
-  if (one && pl.NRB > 1 && wgs2 <= fused_capacity<D, RT, true>()) {
-    hipLaunchKernelGGL((fused2_kernel<D, RT>), dim3(a.HK, (pl.NRB + 1) / 2, pl.NG), dim3(64 * kWavesA), 0, s, a);
-    return;
+  // Twice the rows per workgroup when that grid fits: 128-row blocks, or (D = 256)
+  // two blocks one after the other.  A larger grid runs the prompt part and the
+  // nodes in a launch each.
+  const int nrb2 = D == 256 ? (pl.NRB + 1) / 2 : (pl.R + 127) / 128;
+  const dim3 g2(a.HK, nrb2, pl.NG), b8(64 * kWavesA);
+  const bool two = one && pl.NRB > 1 && a.HK * nrb2 * pl.NG <= fused_capacity<D, RT, true>();
+  if constexpr (D == 256) {
+    if (two) {
+      hipLaunchKernelGGL((fused2_kernel<D, RT>), g2, b8, 0, s, a);
+      return;
+    }
+    if (pl.prompt_wgs > 0) hipLaunchKernelGGL((prompt_kernel<D, RT>), dim3(a.HK, pl.NRB, pl.NG), b8, 0, s, a);
+  } else {
+    if (two) {
+      TrieAttnArgs b = a;
+      b.NRB = nrb2;
+      hipLaunchKernelGGL((fused_pair_kernel<D>), g2, b8, 0, s, b);
+      return;
+    }
+    if (pl.prompt_wgs > 0) hipLaunchKernelGGL((prompt_pair_kernel<D>), g2, b8, 0, s, a);
   }
-  if (pl.prompt_wgs > 0) hipLaunchKernelGGL((prompt_kernel<D, RT>), dim3(a.HK, pl.NRB, pl.NG), dim3(64 * kWavesA), 0, s, a);
   if constexpr (D <= 128) {
     // Nodes and merge: 64-row blocks once they give a quarter of the CUs a workgroup
     // (8B heads, causal rows after 2560 prompt keys: 130 rows 36.8 us for the call
