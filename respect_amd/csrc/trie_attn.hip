@@ -964,9 +964,31 @@ template <int D> struct VResLds {
   static __device__ __forceinline__ lds_char* vbuf(lds_char* kv, int b) { return kv + VOFF + b * CB; }
 };
 
-// Bytes of LDS the node phase may use (either layout).
+// Node LDS of a segment of at most SLOTS slots that does not stay resident
+// (node_stream): the scores, then probabilities, of the rows over every slot, three
+// chunks of V (or four gathered tiles of V rows), and the areas of NodeLds.
+template <int D> struct StreamLds {
+  static constexpr int SLOTS = D == 256 ? 0 : D == 32 ? 512 : 1024;   // what fits beside the V chunks
+  static constexpr int CB = kChunk * 2 * D;
+  static constexpr int TILE = kNodeTile * 2 * D;       // one gathered tile
+  static constexpr int BATCH = 4;                      // gathered tiles in flight
+  static constexpr int VOFF = 0;
+  static constexpr int SR = SLOTS + 4;
+  static constexpr int NBUF = 3;                       // V chunks in LDS
+  static constexpr int SOFF = NBUF * CB;
+  static constexpr int NPROW = D + 4;
+  static constexpr int NPOFF = SOFF + kNodeRows * SR * 4;
+  static constexpr int MWOFF = NPOFF + kNodeRows * NPROW * 4;
+  static constexpr int TOFF = MWOFF + kNodeRows * (SLOTS / kChunk) * 8;
+  static constexpr int INFOFF = TOFF + kWavesA * kRankTab * 2;   // [16 groups] n, shared tiles
+  static constexpr int BYTES = INFOFF + kNodeRows * 8;
+  static_assert(BATCH * TILE <= NBUF * CB, "gathered tiles fit the chunk buffers");
+};
+
+// Bytes of LDS the node phase may use (any of the layouts).
 template <int D> constexpr int node_area_bytes() {
-  return NodeLds<D>::BYTES > VResLds<D>::BYTES ? NodeLds<D>::BYTES : VResLds<D>::BYTES;
+  const int a = NodeLds<D>::BYTES, b = VResLds<D>::BYTES, c = StreamLds<D>::SLOTS > 0 ? StreamLds<D>::BYTES : 0;
+  return a > b ? (a > c ? a : c) : (b > c ? b : c);
 }
 
 // Where a row's result goes: row r of kv head g is query r / GQA of head
@@ -1433,6 +1455,253 @@ __device__ __forceinline__ void node_res_tasks(const TrieAttnArgs& A, int g, int
   }
 }
 
+// The smallest v of the wave, in every lane.
+__device__ __forceinline__ int wave_min(int v) {
+#pragma unroll
+  for (int s = 32; s >= 1; s >>= 1) v = min(v, shfl_idx_i(v, __lane_id() ^ s));
+  return __builtin_amdgcn_readfirstlane(v);
+}
+
+// node_rows for a segment too long to stay resident (at most StreamLds::SLOTS
+// slots; e.g. some hundred committed tokens), the same sums in the same order.
+// The scores of every slot stay in LDS, so K is read once, and become
+// probabilities there.  Rows see the committed tokens alike: ranks below
+// 32 tend, tend the whole tiles of the shortest unbroken run of open slots of any
+// of the rows, are the slots themselves for every row, so their V rows are staged
+// chunk by chunk and one pair of MFMAs per 16 head_dim columns serves all rows,
+// each wave taking its own columns.  The ranks past the run are gathered query by
+// query, four tiles at a time, with p read from LDS by slot.
+//
+// What bounded it: K and V were gathered by rank for every query, a memory round
+// trip per tile of 32 ranks, on as many waves as the workgroup has queries (two
+// of eight in a 64-node call).
+template <int D>
+__device__ __forceinline__ const lds_float* node_stream(const TrieAttnArgs& A, int g, int p0, int rend, lds_char* kv,
+                                                       int w, const bf16x8 (&qf)[D / 32]) {
+  using LY = StreamLds<D>;
+  constexpr int DQ = D / 32, DT = D / 16, RB = 2 * D, nw = kWavesA;
+  int lane = __lane_id();
+  asm volatile("" : "+v"(lane));   // nothing computed from it is shared with the other forms: the registers are full
+  const int n16 = lane & 15, g4 = lane >> 4, e4 = n16 >> 2, c4 = n16 & 3;
+  const int NN = A.NN, nch = (NN + kChunk - 1) / kChunk, nt = (NN + 15) / 16;
+  const int GQA = 1 << A.GQS, q0 = p0 >> A.GQS, ng = ((rend - 1) >> A.GQS) - q0 + 1;
+  const int nrd = (rend - p0 - w + nw - 1) / nw;   // rows of this wave: p0 + w + 8 i
+  lds_float* S = (lds_float*)(kv + LY::SOFF);
+  lds_float* NP = (lds_float*)(kv + LY::NPOFF);
+  typedef __attribute__((address_space(3))) int lds_int;
+  typedef __attribute__((address_space(3))) uint64_t lds_u64;
+  lds_int* info = (lds_int*)(kv + LY::INFOFF);
+  const __amdgpu_buffer_rsrc_t rk = buffer_rsrc(A.kn + g * A.sknh, 2 * ((NN - 1) * A.sknn + D));
+  const __amdgpu_buffer_rsrc_t rv = buffer_rsrc(A.vn + g * A.svnh, 2 * ((NN - 1) * A.svnn + D));
+
+  // Mask bits of the wave's rows, one per chunk, eight chunks of bytes at a time.
+  uint32_t mbits[kNodeRounds] = {};
+#pragma unroll
+  for (int cb = 0; cb < LY::SLOTS / kChunk; cb += 8) {
+    if (cb >= nch) break;
+    uint8_t b[kNodeRounds][8];
+#pragma unroll
+    for (int i = 0; i < kNodeRounds; ++i) {
+      const uint8_t* mrow = A.msk + (int64_t)((i < nrd ? p0 + w + nw * i : p0) >> A.GQS) * A.smm;
+#pragma unroll
+      for (int u = 0; u < 8; ++u) b[i][u] = mrow[(int64_t)min(kChunk * (cb + u) + lane, NN - 1) * A.smn];
+    }
+#pragma unroll
+    for (int i = 0; i < kNodeRounds; ++i)
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        mbits[i] |= (uint32_t)(i < nrd && kChunk * (cb + u) + lane < NN && b[i][u] != 0) << (cb + u);
+  }
+  // Chunk c of V into its buffer.
+  auto issue_v = [&](int c) {
+    for (int x = w; x < LY::CB / 1024; x += nw) {
+      const int byte = x * 1024 + 16 * lane, row = byte / RB, u = (byte % RB) / 16;
+      bdma16(rv, 2 * (kChunk * c + row) * A.svnn + 16 * (u ^ vswz<D>(row)),
+             kv + LY::VOFF + (c % LY::NBUF) * LY::CB + x * 1024);
+    }
+  };
+  // Scores times A.c: waves w, w + 8, ... take 16-slot tiles, four tiles' K
+  // fragments in flight (slots past NN read zeros).
+  for (int tb = w; tb < nt; tb += 4 * nw) {
+    u32x4 kf[4][DQ];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int slot = 16 * (tb + nw * u) + n16;
+#pragma unroll
+      for (int i = 0; i < DQ; ++i)
+        kf[u][i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                                  rk, slot < NN ? 2 * (slot * A.sknn + 32 * i + 8 * g4) : 0x7ffffff0, 0, 0));
+    }
+    if (tb == w) {   // behind the first K loads: they land under the scores
+      issue_v(0);
+      issue_v(1);
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      if (tb + nw * u >= nt) break;
+      f32x4 sv = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int i = 0; i < DQ; ++i)
+        sv = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, kf[u][i]), qf[i], sv, 0, 0, 0);
+      *(lds_f32x4*)(S + n16 * LY::SR + 16 * (tb + nw * u) + 4 * g4) = sv * A.c;
+    }
+  }
+  lds_barrier();   // every score is in LDS
+  // Rows: the maximum over the allowed slots, then p in place (0 where masked); a
+  // group's first row leaves its mask words, count and run.
+#pragma unroll 1
+  for (int i = 0; i < nrd; ++i) {
+    const int row = w + nw * i, r = p0 + row;
+    const bool lead = r == p0 || (r & (GQA - 1)) == 0;
+    const int gl = (r >> A.GQS) - q0;
+    const uint32_t mb = i ? mbits[1] : mbits[0];
+    lds_float* Sr = S + row * LY::SR + lane;
+    float sc[LY::SLOTS / kChunk];
+    float x = kNegInf;
+    int n = 0, z = 0;
+    bool run = true;
+#pragma unroll
+    for (int c = 0; c < LY::SLOTS / kChunk; ++c)
+      if (c < nch) sc[c] = Sr[kChunk * c];
+#pragma unroll
+    for (int c = 0; c < LY::SLOTS / kChunk; ++c) {
+      if (c >= nch) continue;
+      const bool ok = (mb >> c) & 1;
+      x = fmaxf(x, ok ? sc[c] : kNegInf);
+      const uint64_t mm = __builtin_amdgcn_ballot_w64(ok);
+      n += __builtin_popcountll(mm);
+      if (run) {
+        z += ~mm ? __builtin_ctzll(~mm) : kChunk;
+        run = ~mm == 0;
+      }
+      if (lead && lane == 0) *(lds_u64*)(kv + LY::MWOFF + (gl * (LY::SLOTS / kChunk) + c) * 8) = mm;
+    }
+    const float m = max64(x);
+#pragma unroll
+    for (int c = 0; c < LY::SLOTS / kChunk; ++c)
+      if (c < nch) Sr[kChunk * c] = (mb >> c) & 1 ? fexp2(sc[c] - m) : 0.f;
+    if (lane == 0) {
+      NP[row * LY::NPROW] = m;
+      if (lead) {
+        info[2 * gl] = n;
+        info[2 * gl + 1] = z / kNodeTile;
+      }
+    }
+  }
+  lds_barrier();
+  const int tend = wave_min(info[2 * (lane < ng ? lane : 0) + 1]);
+  const int jd = w;                 // this wave's head_dim tile
+  const bool on = jd < DT;
+  const int b16 = 2 * jd + (c4 >> 1);   // its 16-byte units of a V row
+  const uint32_t one2 = 0x3f803f80u;    // two bf16 1.0
+  const bf16x8 ones = __builtin_bit_cast(bf16x8, u32x4{one2, one2, one2, one2});
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f}, lacc = {0.f, 0.f, 0.f, 0.f};
+  // p of ranks 4 g4 + j (j < 4) and 16 + 4 g4 + j - 4 of a tile as hi and lo bf16.
+  auto split = [&](const float (&pv)[8], bf16x8& hop, bf16x8& lop) {
+    u32x4 hw, lw;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      hw[i] = pack_bf16x2(pv[2 * i], pv[2 * i + 1]);
+      lw[i] = pack_bf16x2(pv[2 * i] - bf16_lo(hw[i]), pv[2 * i + 1] - bf16_hi(hw[i]));
+    }
+    hop = __builtin_bit_cast(bf16x8, hw);
+    lop = __builtin_bit_cast(bf16x8, lw);
+  };
+  // One tile whose V rows 0 .. 31 sit at v (row swizzle by (row + sw0)).
+  auto tile = [&](const bf16x8& hop, const bf16x8& lop, const lds_char* v, int sw0, f32x4& ac, f32x4& lc) {
+    const int r0 = 4 * g4 + e4, r1 = r0 + 16;
+    const s16x4 lo = lds_read_tr(v + r0 * RB + 16 * (b16 ^ vswz<D>(sw0 + r0)) + 8 * (c4 & 1));
+    const s16x4 hi = lds_read_tr(v + r1 * RB + 16 * (b16 ^ vswz<D>(sw0 + r1)) + 8 * (c4 & 1));
+    const bf16x8 vop = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+    ac = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vop, hop, ac, 0, 0, 0);
+    ac = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vop, lop, ac, 0, 0, 0);
+    lc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, hop, lc, 0, 0, 0);
+    lc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, lop, lc, 0, 0, 0);
+  };
+  const lds_float* Sc = S + n16 * LY::SR;   // column n16's row
+  const int ncs = (tend + 1) / 2;
+  constexpr int VPW = LY::CB / 1024 / nw;   // loads of a wave per chunk (0: some waves have none)
+  for (int c = 0; c < ncs; ++c) {
+    // This wave's part of chunk c: chunk c + 1 may still be in flight.
+    if (VPW > 0 && c + 1 < ncs) RSPX_VM(VPW);
+    else RSPX_VM(0);
+    lds_barrier();   // every wave's part; every wave is done with chunk c - 1
+    if (c + 2 < ncs) issue_v(c + 2);
+    if (on) {
+#pragma unroll
+      for (int hh = 0; hh < 2; ++hh) {
+        const int t = 2 * c + hh;
+        if (t >= tend) break;
+        const f32x4 pa = *(const lds_f32x4*)(Sc + kNodeTile * t + 4 * g4);
+        const f32x4 pb = *(const lds_f32x4*)(Sc + kNodeTile * t + 16 + 4 * g4);
+        const float pv[8] = {pa[0], pa[1], pa[2], pa[3], pb[0], pb[1], pb[2], pb[3]};
+        bf16x8 hop, lop;
+        split(pv, hop, lop);
+        tile(hop, lop, kv + LY::VOFF + (c % LY::NBUF) * LY::CB + kNodeTile * hh * RB, kNodeTile * hh, acc, lacc);
+      }
+    }
+  }
+  // The ranks past the run, query by query, up to BATCH tiles (of one or more
+  // queries) in flight.
+  lds_i16* tab = (lds_i16*)(kv + LY::TOFF) + w * kRankTab;
+  int gl = -1, rt = 0, n = 0, rc = 0, rbase = 0;   // the query, its next tile's first rank, its count
+  while (true) {
+    RSPX_VM(0);      // V chunks no tile used have landed
+    lds_barrier();   // every wave is done with the buffers
+    bf16x8 hop[LY::BATCH], lop[LY::BATCH];
+    int cols = 0, cnt = 0;
+#pragma unroll
+    for (int u = 0; u < LY::BATCH; ++u) {
+      while (rt >= n && gl < ng) {
+        ++gl;
+        rt = kNodeTile * tend;
+        n = gl < ng ? __builtin_amdgcn_readfirstlane(info[2 * gl]) : 0;
+        rc = tend / 2;   // ranks below 32 tend are slots below 32 tend
+        rbase = kChunk * rc;
+      }
+      if (gl >= ng) break;
+      cnt = u + 1;
+      rank_fill(rc, rbase, rt + kNodeTile, nch, kv + LY::MWOFF + gl * (LY::SLOTS / kChunk) * 8, tab);
+      for (int x = w; x < LY::TILE / 1024; x += nw) {
+        const int byte = x * 1024 + 16 * lane, rr = byte / RB, un = (byte % RB) / 16;
+        const int s = rt + rr < n ? tab[(rt + rr) & (kRankTab - 1)] : -1;
+        bdma16(rv, s >= 0 ? 2 * s * A.svnn + 16 * (un ^ vswz<D>(rr)) : 0x7ffffff0,
+               kv + LY::VOFF + u * LY::TILE + x * 1024);
+      }
+      const bool col = p0 + n16 < rend && ((p0 + n16) >> A.GQS) - q0 == gl;
+      cols |= (int)col << u;
+      float pv[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const int rr = rt + 4 * g4 + (j < 4 ? j : 12 + j);
+        pv[j] = col && rr < n ? Sc[tab[rr & (kRankTab - 1)]] : 0.f;
+      }
+      split(pv, hop[u], lop[u]);
+      rt += kNodeTile;
+    }
+    if (cnt == 0) break;
+    RSPX_VM(0);      // this wave's pieces
+    lds_barrier();   // every wave's
+    if (on) {
+#pragma unroll
+      for (int u = 0; u < LY::BATCH; ++u) {
+        if (u >= cnt) break;
+        f32x4 ac = acc, lc = lacc;
+        tile(hop[u], lop[u], kv + LY::VOFF + u * LY::TILE, 0, ac, lc);
+        const bool col = (cols >> u) & 1;   // other queries' columns keep their sums, whatever V holds
+        acc = col ? ac : acc;
+        lacc = col ? lc : lacc;
+      }
+    }
+  }
+  if (on && p0 + n16 < rend) {
+    *(lds_f32x4*)(NP + n16 * LY::NPROW + 4 + 16 * jd + 4 * g4) = acc;
+    if (jd == 0 && g4 == 0) NP[n16 * LY::NPROW + 1] = lacc[0];
+  }
+  lds_barrier();   // every row's partial is in NP
+  return (const lds_float*)NP;
+}
+
 // Node partials of rows [p0, rend) of kv head g (at most kNodeRows) over each
 // row's allowed node slots (attention.py:52-67): m is the exact maximum score
 // over the allowed slots; the sums run over the allowed slots in slot order
@@ -1471,6 +1740,13 @@ __device__ __forceinline__ const lds_float* node_rows(const TrieAttnArgs& A, int
     for (int i = 0; i < D / 32; ++i) qf[i] = pre.qf[i];
   } else {
     node_q<D>(A, g, p0, rend, qf);
+  }
+
+  if constexpr (StreamLds<D>::SLOTS > 0) {
+    // 264 slots (200 committed): 20.9 us for the 64-node call with V resident, 22.4
+    // with node_stream; 500 slots: 44.7 gathered, 31.7 with node_stream.
+    if (__builtin_expect(!res && !vres && NN <= StreamLds<D>::SLOTS, 0))
+      return node_stream<D>(A, g, p0, rend, kv, w, qf);
   }
 
   // Maxima, mask words, allowed counts.  The first row of each group in
@@ -1828,12 +2104,6 @@ struct BlockLds {
   static constexpr int BYTES = FLAGOFF + 16;
   static_assert(BYTES <= 160 * 1024, "LDS budget");
 };
-
-__device__ __forceinline__ int wave_min(int v) {
-#pragma unroll
-  for (int s = 32; s >= 1; s >>= 1) v = min(v, shfl_idx_i(v, __lane_id() ^ s));
-  return __builtin_amdgcn_readfirstlane(v);
-}
 
 // Chunk c (kChunk slots) of kv head g's node K as score fragments, and with VALS
 // its V rows, into buffers b (the layouts of NodeLds); slots past NN read zeros.

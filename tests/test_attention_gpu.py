@@ -521,6 +521,9 @@ def test_tiled_output_rejects_a_head_stride_other_than_d():
     (8, 2, 64, 300, 64, "random"),         # no common run
     (8, 8, 128, 230, 40, "holes"),         # rows without any node slot, and causal rows
     (8, 2, 128, 320, 100, "nan"),          # NaN / inf K and V in slots that later rows alone may see
+    (8, 2, 64, 1000, 100, "random"),       # 1024 slots: the longest segment node_stream takes
+    (8, 2, 32, 500, 64, "open32k"),        # 512 slots: its longest at head_dim 32
+    (8, 2, 32, 530, 33, "causal"),         # 544 slots: gathered
 ])
 def test_many_rows(H, HK, D, M, P, mask):
     """Calls whose grid never fits the device at once (prompt part and node part in a launch
@@ -565,3 +568,6 @@ def test_many_rows(H, HK, D, M, P, mask):
         n = NN if P else min(NN, -(-(m + 1) // 32) * 32)   # without a prompt: a shorter node segment, held whole
         one = trie_attn(q[:, m:m + 1], kp, vp, kn[:, :n], vn[:, :n], msk[m:m + 1, :n], launches=1 if P else 2)
         assert same(one[:, 0], out[:, m]), f"row {m}"
+    for m in (0, M // 2, M - 9):           # eight queries, so rows of different masks share a workgroup
+        few = trie_attn(q[:, m:m + 8], kp, vp, kn, vn, msk[m:m + 8])
+        assert same(few, out[:, m:m + 8]), f"rows {m}.."
