@@ -235,6 +235,10 @@ __device__ __forceinline__ int vswz(int key) {
   else return 2 * ((key / (16 / U)) % (U / 2));
 }
 
+// Keys 16 apart have the same K swizzle.
+template <int D>
+constexpr bool kswz_period_ok() { return D / 8 >= 16 || (16 / (16 / (D / 8))) % (D / 8) == 0; }
+
 // s_waitcnt vmcnt(v) for an immediate v.
 #define RSPX_VM(v) __builtin_amdgcn_s_waitcnt(((v) & 15) | (((v) >> 4) << 14) | 0x70 | 0xF00)
 
@@ -348,40 +352,41 @@ __device__ __forceinline__ void chunk_offsets(const TrieAttnArgs& A, int w, int 
   }
 }
 
-// The lane's LDS offsets inside a step slot: transposing-read addresses of the V
-// operand halves (keys 4 g4 + e and 16 + 4 g4 + e) for head_dim tile j, and
-// A-fragment addresses of the K operand (lane (n16, g4) reads key 16 kb + n16,
-// head_dim [32 i + 8 g4, +8) = 16-byte unit 4 i + g4).
+// The lane's LDS offsets inside a step slot (a multiple of 1 KB): kbase, its K
+// A-fragment of key n16 (key 16 kb + n16, head_dim [32 i + 8 g4, +8) = 16-byte unit
+// 4 i + g4) for kb = i = 0, and vbase[kh], its transposing read of the V operand
+// half kh (keys 16 kh + 4 g4 + e) for head_dim tile 0.  The swizzles are XORs of
+// the unit index, so fragment i sits at (slot + kbase) ^ 64 i, 16 keys further on
+// 32 D bytes later, and head_dim tile j at (slot + vbase) ^ 32 j: one register and
+// an XOR each instead of a register per address.
 template <int D>
-__device__ __forceinline__ void slot_offsets(int (&trv)[2][StepGeom<D>::DT], int (&kro)[2][StepGeom<D>::DQ]) {
+__device__ __forceinline__ void slot_offsets(int& kbase, int (&vbase)[2]) {
   using G = StepGeom<D>;
   const int lane = __lane_id(), n16 = lane & 15, g4 = lane >> 4;
   const int e = n16 >> 2, c4 = n16 & 3;
+  static_assert(kswz_period_ok<D>(), "16 keys keep the K swizzle");
+  kbase = 16 * (n16 * G::U + (g4 ^ kswz<D>(n16)));
 #pragma unroll
   for (int kh = 0; kh < 2; ++kh) {
     const int key = 16 * kh + 4 * g4 + e;
-#pragma unroll
-    for (int j = 0; j < G::DT; ++j) {
-      const int b = 2 * j + (c4 >> 1);
-      trv[kh][j] = G::KBYTES + 16 * (key * G::U + (b ^ vswz<D>(key))) + 8 * (c4 & 1);
-    }
+    vbase[kh] = G::KBYTES + 16 * (key * G::U + ((c4 >> 1) ^ vswz<D>(key))) + 8 * (c4 & 1);
   }
-#pragma unroll
-  for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-    for (int i = 0; i < G::DQ; ++i) {
-      const int key = 16 * kb + n16;
-      kro[kb][i] = 16 * (key * G::U + ((4 * i + g4) ^ kswz<D>(key)));
-    }
+}
+
+// (slot + base) ^ x as an LDS address, and the 16 bytes `off` past it.
+__device__ __forceinline__ const lds_char* lds_at(const lds_char* slot, int base, int x) {
+  return (const lds_char*)(uint32_t)(((uint32_t)(uintptr_t)slot + base) ^ x);
+}
+__device__ __forceinline__ u32x4 lds_frag(const lds_char* slot, int base, int x, int off) {
+  return *(const __attribute__((address_space(3))) u32x4*)(lds_at(slot, base, x) + off);
 }
 
 // One step of 32 keys from first key ks, K/V in LDS at `slot`, for the wave's kRT
 // row tiles: scores, online softmax against the lazily moved reference maximum,
-// and the PV product.  kro / trv: the lane's LDS offsets of the K fragments and of
-// the V operand halves inside a slot.
+// and the PV product.  kbase / vbase: slot_offsets.
 template <int D, int kRT>
 __device__ __forceinline__ void prompt_step(const TrieAttnArgs& A, const lds_char* slot, int ks,
-                                            const int (&kro)[2][StepGeom<D>::DQ], const int (&trv)[2][StepGeom<D>::DT],
+                                            int kbase, const int (&vbase)[2],
                                             const bf16x8 (&qop)[kRT][StepGeom<D>::DQ], float (&mref)[kRT],
                                             float (&lrow)[kRT], f32x4 (&acc)[kRT][StepGeom<D>::DT]) {
   constexpr int DQ = StepGeom<D>::DQ, DT = StepGeom<D>::DT;
@@ -391,7 +396,7 @@ __device__ __forceinline__ void prompt_step(const TrieAttnArgs& A, const lds_cha
     for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
       for (int i = 0; i < DQ; ++i)
-        kf[kb][i] = *(const __attribute__((address_space(3))) u32x4*)(slot + kro[kb][i]);
+        kf[kb][i] = lds_frag(slot, kbase, 64 * i, 32 * D * kb);
 
     // S^T = K Q^T for two blocks of 16 keys.
     f32x4 sc[kRT][2];
@@ -406,6 +411,19 @@ __device__ __forceinline__ void prompt_step(const TrieAttnArgs& A, const lds_cha
                                                        0, 0, 0);
         sc[t][kb] = sv;
       }
+
+    // The first V operands are requested here, before the softmax, and each of the
+    // others kAhead tiles before its MFMAs: two ahead, a tile's MFMAs (32 cycles)
+    // waited for most of an LDS read's latency each time.
+    constexpr int kAhead = DT < 4 ? DT : 4;
+    s16x4 vlo[DT], vhi[DT];
+    auto vread = [&](int j) {
+      vlo[j] = lds_read_tr(lds_at(slot, vbase[0], 32 * j));
+      vhi[j] = lds_read_tr(lds_at(slot, vbase[1], 32 * j));
+    };
+#pragma unroll
+    for (int j = 0; j < kAhead; ++j) vread(j);
+    __builtin_amdgcn_sched_barrier(0);
 
     // Lane (n16, g4) holds row n16, keys 16 kb + 4 g4 + e of the step.  Raw
     // scores; keys past P (only in the last step) are masked to -inf.  Since
@@ -471,12 +489,13 @@ __device__ __forceinline__ void prompt_step(const TrieAttnArgs& A, const lds_cha
     // consecutive head_dim columns of the row whose softmax state it keeps.
 #pragma unroll
     for (int j = 0; j < DT; ++j) {
-      const s16x4 lo = lds_read_tr(slot + trv[0][j]);
-      const s16x4 hi = lds_read_tr(slot + trv[1][j]);
-      const bf16x8 vop = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+      if (j + kAhead < DT) vread(j + kAhead);
+      const bf16x8 vop = __builtin_bit_cast(bf16x8, __builtin_shufflevector(vlo[j], vhi[j], 0, 1, 2, 3, 4, 5, 6, 7));
 #pragma unroll
       for (int t = 0; t < kRT; ++t)
         acc[t][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vop, pop[t], acc[t][j], 0, 0, 0);
+      if (j + kAhead < DT) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+      __builtin_amdgcn_sched_group_barrier(0x008, kRT, 0);
     }
 }
 
@@ -532,8 +551,8 @@ __device__ __forceinline__ void prompt_block(const TrieAttnArgs& A, char* lds, i
   chunk_offsets<D>(A, w, voff);
   const uint16_t* kpg = A.kp + g * A.skph;
   const uint16_t* vpg = A.vp + g * A.svph;
-  int trv[2][DT], kro[2][DQ];
-  slot_offsets<D>(trv, kro);
+  int kbase, vbase[2];
+  slot_offsets<D>(kbase, vbase);
 
   float mref[kRT], lrow[kRT];
   f32x4 acc[kRT][DT];
@@ -577,7 +596,7 @@ __device__ __forceinline__ void prompt_block(const TrieAttnArgs& A, char* lds, i
     const int sl = kQuarters * r + k;  // step of this wave within the group
     if (has_rows && sl < ns) {
 
-    prompt_step<D, kRT>(A, ring + (r % G::RING) * G::ROUND + k * G::SLOT, (s0 + sl) * kStep, kro, trv, qop, mref, lrow,
+    prompt_step<D, kRT>(A, ring + (r % G::RING) * G::ROUND + k * G::SLOT, (s0 + sl) * kStep, kbase, vbase, qop, mref, lrow,
                         acc);
     }
     if (r < 3) RSPX_MARK(2 + 2 * r);
@@ -709,7 +728,7 @@ __device__ __forceinline__ void prompt_block(const TrieAttnArgs& A, char* lds, i
 
 template <int D, int kRT>
 __global__ __launch_bounds__(512) void prompt_kernel(TrieAttnArgs A) {
-  __shared__ __attribute__((aligned(16))) char lds[PromptLds<D, kRT>::BYTES];
+  __shared__ __attribute__((aligned(1024))) char lds[PromptLds<D, kRT>::BYTES];
   prompt_block<D, kRT, false, true>(A, lds, blockIdx.x, blockIdx.y, blockIdx.z, [] {}, [] {}, [] {});
 }
 
@@ -778,8 +797,8 @@ __device__ __forceinline__ void pair_block(const TrieAttnArgs& A, char* lds, int
 #pragma unroll
     for (int i = 0; i < DQ; ++i) qop[t][i] = *reinterpret_cast<const bf16x8*>(qp + 32 * i);
   }
-  int trv[2][DT], kro[2][DQ];
-  slot_offsets<D>(trv, kro);
+  int kbase, vbase[2];
+  slot_offsets<D>(kbase, vbase);
   float mref[2][kRT], lrow[2][kRT];
   f32x4 acc[2][kRT][DT];
 #pragma unroll
@@ -804,7 +823,7 @@ __device__ __forceinline__ void pair_block(const TrieAttnArgs& A, char* lds, int
     for (int u = 0; u < 2; ++u) {
       const int sl = kQuarters * r + 2 * p + u;
       if (has_rows && sl < ns)
-        prompt_step<D, kRT>(A, slot + (2 * p + u) * G::SLOT, (s0 + sl) * kStep, kro, trv, qop, mref[u], lrow[u], acc[u]);
+        prompt_step<D, kRT>(A, slot + (2 * p + u) * G::SLOT, (s0 + sl) * kStep, kbase, vbase, qop, mref[u], lrow[u], acc[u]);
     }
     if (r + G::RING < nr) {
       lds_barrier();   // round r is consumed by every wave
@@ -891,7 +910,7 @@ __device__ __forceinline__ void pair_block(const TrieAttnArgs& A, char* lds, int
 
 template <int D>
 __global__ __launch_bounds__(512) void prompt_pair_kernel(TrieAttnArgs A) {
-  __shared__ __attribute__((aligned(16))) char lds[PairLds<D>::BYTES];
+  __shared__ __attribute__((aligned(1024))) char lds[PairLds<D>::BYTES];
   pair_block<D, false>(A, lds, blockIdx.x, blockIdx.y, blockIdx.z, [] {});
 }
 
@@ -2130,7 +2149,7 @@ template <int D>
 __global__ __launch_bounds__(512) void node_block_kernel(TrieAttnArgs A) {
   using LY = BlockLds<D>;
   constexpr int DQ = D / 32, DT = D / 16, NJ = DT / 2, RB = 2 * D;
-  __shared__ __attribute__((aligned(16))) char lds[LY::BYTES];
+  __shared__ __attribute__((aligned(1024))) char lds[LY::BYTES];
   lds_char* kv = (lds_char*)lds;
   const int lane = __lane_id();
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -2581,7 +2600,7 @@ __global__ __launch_bounds__(512) void fused_kernel(TrieAttnArgs A) {
   constexpr int NB = node_area_bytes<D>() + 16;
   constexpr int LB = PL::BYTES + PL::MLBYTES > NB ? PL::BYTES + PL::MLBYTES : NB;
   static_assert(NB <= PL::RINGBYTES, "node LDS and the wait flag inside the ring (the Q fragments stay)");
-  __shared__ __attribute__((aligned(16))) char lds[LB];
+  __shared__ __attribute__((aligned(1024))) char lds[LB];
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int g = blockIdx.x, rb = blockIdx.y, q = blockIdx.z;
   RSPX_MARK(0);
@@ -2646,7 +2665,7 @@ __global__ __launch_bounds__(512) void fused2_kernel(TrieAttnArgs A) {
   constexpr int NB = node_area_bytes<D>() + 16;
   constexpr int LB = PL::BYTES + PL::MLBYTES > NB ? PL::BYTES + PL::MLBYTES : NB;
   static_assert(NB <= PL::RINGBYTES, "node LDS and the wait flag inside the ring (the Q fragments stay)");
-  __shared__ __attribute__((aligned(16))) char lds[LB];
+  __shared__ __attribute__((aligned(1024))) char lds[LB];
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int g = blockIdx.x, rbw = blockIdx.y, q = blockIdx.z;
   // Every argument the prologue needs, requested in one batch.
@@ -2702,7 +2721,7 @@ __global__ __launch_bounds__(512) void fused_pair_kernel(TrieAttnArgs A) {
   using PL = PairLds<D>;
   constexpr int NB = node_area_bytes<D>() + 16;
   static_assert(NB <= PL::RINGBYTES, "node LDS and the wait flag inside the ring");
-  __shared__ __attribute__((aligned(16))) char lds[PL::BYTES];
+  __shared__ __attribute__((aligned(1024))) char lds[PL::BYTES];
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int g = blockIdx.x, rb = blockIdx.y, q = blockIdx.z;
   // Every argument the prologue needs, requested in one batch.
