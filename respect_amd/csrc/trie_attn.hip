@@ -244,17 +244,18 @@ constexpr bool kswz_period_ok() { return D / 8 >= 16 || (16 / (16 / (D / 8))) % 
 
 // Waits until at most `younger` rounds of OWN loads each (younger < RING) are
 // still in flight: vmcnt(OWN younger), the count as an immediate.
-template <int OWN, int RING>
+// EXTRA: and that many operations younger than the round waited for.
+template <int OWN, int RING, int EXTRA = 0>
 __device__ __forceinline__ void wait_rounds(int younger) {
-  static_assert(OWN * (RING - 1) < 64, "vmcnt range");
+  static_assert(OWN * (RING - 1) + EXTRA < 64, "vmcnt range");
   if constexpr (RING > 1) {
     if (younger >= RING - 1) {
-      RSPX_VM(OWN * (RING - 1));
+      RSPX_VM(OWN * (RING - 1) + EXTRA);
       return;
     }
-    wait_rounds<OWN, RING - 1>(younger);
+    wait_rounds<OWN, RING - 1, EXTRA>(younger);
   } else {
-    RSPX_VM(0);
+    RSPX_VM(EXTRA);
   }
 }
 
@@ -734,8 +735,8 @@ __global__ __launch_bounds__(512) void prompt_kernel(TrieAttnArgs A) {
 
 // ------------------------------------------------------------------ 128-row blocks
 // The prompt work of a block of 128 rows, for calls with more rows than one
-// 64-row block per workgroup covers: rows [128 rb, +128) of kv head g, key group q,
-// up to the group partial in memory.  Wave w: rows 32 (w / 2) of the block (two
+// 64-row block per workgroup covers: rows [128 rb, +128) of kv head g, key groups
+// [q, qend), up to the group partials in memory.  Wave w: rows 32 (w / 2) of the block (two
 // tiles) and the key quarters 2 p, 2 p + 1 (p = w % 2), each with its own
 // softmax state; the arithmetic and the order of every sum are prompt_block's.
 //
@@ -745,6 +746,8 @@ __global__ __launch_bounds__(512) void prompt_kernel(TrieAttnArgs A) {
 // 128 rows halves those bytes.  Two quarters per wave instead of one keep a wave at
 // 32 rows (one K or V fragment read from LDS per two MFMAs), and their sum needs no
 // exchange: only half a pair's sum crosses to the other wave.
+//   The groups follow each other without a gap: the next group's first rounds load
+// while a group is combined (in the ring slot of its last round) and stored.
 template <int D>
 struct PairLds {
   using G = StepGeom<D>;
@@ -752,11 +755,11 @@ struct PairLds {
   static constexpr int MLBYTES = 4 * kQuarters * 2 * 16 * 8;   // [4 row groups][quarter][tile][16 rows] (m, l)
   static constexpr int BYTES = RINGBYTES + MLBYTES;
   static constexpr int BOX = 32 * D * 2;                       // 32 rows x D / 2 floats, one per wave
-  static_assert(kWavesA * BOX <= RINGBYTES && BYTES <= 160 * 1024, "LDS budget");
+  static_assert(kWavesA * BOX <= G::ROUND && BYTES <= 160 * 1024, "LDS budget");
 };
 
-template <int D, bool ATOMIC, class Hook>
-__device__ __forceinline__ void pair_block(const TrieAttnArgs& A, char* lds, int g, int rb, int q,
+template <int D, bool ATOMIC, bool MULTI, class Hook>
+__device__ __forceinline__ void pair_block(const TrieAttnArgs& A, char* lds, int g, int rb, int q, int qend,
                                            const Hook& before_stores) {
   using G = StepGeom<D>;
   using L = PairLds<D>;
@@ -772,7 +775,7 @@ __device__ __forceinline__ void pair_block(const TrieAttnArgs& A, char* lds, int
   const int P = A.P;
   const int steps = (P + kStep - 1) / kStep;
   const int s0 = q * A.S;
-  const int ns = min(A.S, steps - s0);
+  const int ns = min((qend - q) * A.S, steps - s0);
   const int nr = (ns + kQuarters - 1) / kQuarters;
   const int trow = 128 * rb + 32 * h;
   const bool has_rows = trow < A.R;
@@ -811,107 +814,131 @@ __device__ __forceinline__ void pair_block(const TrieAttnArgs& A, char* lds, int
       for (int j = 0; j < DT; ++j) acc[u][t][j] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
 
+  constexpr int NST = kRT * HT + 1;   // stores of a wave per group
+  auto finish = [&](lds_char* slot) {
+    // The group's end.  The quarters combined as in prompt_block: scaled to the
+    // row's maximum M over them, (q0 + q1) + (q2 + q3).  A wave adds its own two,
+    // hands the half of the head_dim tiles it does not keep to the other wave of
+    // its rows, and stores tiles [HT p, +HT) of the sum.
+    if (g4 == 0) {
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int t = 0; t < kRT; ++t)
+          *(lds_f32x2*)(ml + (((kQuarters * h + 2 * p + u) * kRT + t) * 16 + n16) * 8) = f32x2{mref[u][t], lrow[u][t]};
+    }
+    lds_barrier();   // (m, l) written; every wave is done with the slot
+    float Mr[kRT], Lr[kRT];
+    f32x4 sv[kRT][HT];
+    lds_char* box = slot + w * L::BOX + 16 * lane;
+#pragma unroll
+    for (int t = 0; t < kRT; ++t) {
+      float mk[4], lk[4], sk[4];
+#pragma unroll
+      for (int kk = 0; kk < 4; ++kk) {
+        const f32x2 v = *(const lds_f32x2*)(ml + (((kQuarters * h + kk) * kRT + t) * 16 + n16) * 8);
+        mk[kk] = v.x;
+        lk[kk] = v.y;
+      }
+      const float M = fmaxf(fmaxf(mk[0], mk[1]), fmaxf(mk[2], mk[3]));
+#pragma unroll
+      for (int kk = 0; kk < 4; ++kk) sk[kk] = mk[kk] == kNegInf ? 0.f : fexp2(mk[kk] - M);
+      Mr[t] = M;
+      Lr[t] = (lk[0] * sk[0] + lk[1] * sk[1]) + (lk[2] * sk[2] + lk[3] * sk[3]);
+      const float sa = p ? sk[2] : sk[0], sb = p ? sk[3] : sk[1];
+#pragma unroll
+      for (int j = 0; j < DT; ++j) acc[0][t][j] = acc[0][t][j] * sa + acc[1][t][j] * sb;
+      // Branches with constant indices: a run-time choice between accumulators
+      // would put them in scratch memory.
+#pragma unroll
+      for (int j = 0; j < HT; ++j) {
+        f32x4 give;
+        if (p) {
+          give = acc[0][t][j];
+          sv[t][j] = acc[0][t][HT + j];
+        } else {
+          give = acc[0][t][HT + j];
+          sv[t][j] = acc[0][t][j];
+        }
+        *(lds_f32x4*)(box + (t * HT + j) * 1024) = give;
+      }
+    }
+    lds_barrier();
+    const lds_char* other = slot + (w ^ 1) * L::BOX + 16 * lane;
+#pragma unroll
+    for (int t = 0; t < kRT; ++t)
+#pragma unroll
+      for (int j = 0; j < HT; ++j) sv[t][j] = sv[t][j] + *(const lds_f32x4*)(other + (t * HT + j) * 1024);
+    if constexpr (!MULTI) {
+      lds_barrier();   // every wave's ring reads are complete: before_stores may load into it
+      before_stores();
+    }
+    // Rows past R and the second wave's (m, l) go past the buffers' ends (an offset
+    // of almost 2^32): no branch, the same number of stores in every wave.
+    const int parts = A.HK * A.R * A.NG;
+    const __amdgpu_buffer_rsrc_t racc = buffer_rsrc(A.gp_acc, (int64_t)parts * D * 4), rml = buffer_rsrc(A.gp_ml, (int64_t)parts * 8);
+    constexpr int AUX = ATOMIC ? 16 : 0;   // sc1: the coherence of an agent-scope atomic store
+    const int mrow = p == 0 && g4 < kRT ? trow + 16 * g4 + n16 : A.R;   // lanes g4 = t store row tile t's (m, l)
+    const float ms = g4 == 0 ? Mr[0] : Mr[kRT - 1], ls = g4 == 0 ? Lr[0] : Lr[kRT - 1];
+    __builtin_amdgcn_raw_buffer_store_b64(f32x2{ms, ls}, rml,
+                                          mrow < A.R ? ((g * A.R + mrow) * A.NG + q) * 8 : -256, 0, AUX);
+#pragma unroll
+    for (int t = 0; t < kRT; ++t) {
+      const int row = trow + 16 * t + n16;
+      const int off = row < A.R ? (((g * A.R + row) * A.NG + q) * D + 16 * HT * p + 4 * g4) * 4 : -256;
+#pragma unroll
+      for (int j = 0; j < HT; ++j) __builtin_amdgcn_raw_buffer_store_b128(sv[t][j], racc, off + 64 * j, 0, AUX);
+    }
+    asm volatile("" ::: "memory");
+  };
+  int left = A.S / kQuarters;         // rounds of the group still to come
+  bool stored = false;                // the last round ended a group: its stores are younger than round r's loads
   for (int r = 0; r < nr; ++r) {
-    wait_rounds<G::OWN, G::RING>(r == 0 ? 0 : min(nr - 1 - r, G::RING - 1));
+    const int younger = r == 0 ? 0 : min(nr - 1 - r, G::RING - 1);
+    if (stored) wait_rounds<G::OWN, G::RING, NST>(younger);
+    else wait_rounds<G::OWN, G::RING>(younger);
+    stored = false;
     lds_barrier();   // every wave's chunks of round r are in LDS
     if (r == 0) {
       for (int rr = 1; rr < min(nr, G::RING); ++rr)
         issue_round<D>(rk, rv, kstep, vstep, kQuarters * rr, voff, ring + rr * G::ROUND, w);
     }
-    const lds_char* slot = ring + (r % G::RING) * G::ROUND;
+    lds_char* slot = ring + (r % G::RING) * G::ROUND;
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
       const int sl = kQuarters * r + 2 * p + u;
       if (has_rows && sl < ns)
         prompt_step<D, kRT>(A, slot + (2 * p + u) * G::SLOT, (s0 + sl) * kStep, kbase, vbase, qop, mref[u], lrow[u], acc[u]);
     }
+    if (MULTI && (--left == 0 || r + 1 == nr)) {
+      finish(slot);
+      left = A.S / kQuarters;
+      stored = true;
+      ++q;
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int t = 0; t < kRT; ++t) {
+          mref[u][t] = kNegInf;
+          lrow[u][t] = 0.f;
+#pragma unroll
+          for (int j = 0; j < DT; ++j) acc[u][t][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+        }
     if (r + G::RING < nr) {
-      lds_barrier();   // round r is consumed by every wave
-      issue_round<D>(rk, rv, kstep, vstep, kQuarters * (r + G::RING), voff, ring + (r % G::RING) * G::ROUND, w);
+      lds_barrier();   // every wave is done with the slot
+      issue_round<D>(rk, rv, kstep, vstep, kQuarters * (r + G::RING), voff, slot, w);
     }
   }
-
-  // The quarters combined as in prompt_block: scaled to the row's maximum M over
-  // them, (q0 + q1) + (q2 + q3).  A wave adds its own two, hands the half of the
-  // head_dim tiles it does not keep to the other wave of its rows, and stores
-  // tiles [HT p, +HT) of the sum.
-  if (g4 == 0) {
-#pragma unroll
-    for (int u = 0; u < 2; ++u)
-#pragma unroll
-      for (int t = 0; t < kRT; ++t)
-        *(lds_f32x2*)(ml + (((kQuarters * h + 2 * p + u) * kRT + t) * 16 + n16) * 8) = f32x2{mref[u][t], lrow[u][t]};
-  }
-  lds_barrier();   // (m, l) written; every wave is past its last step
-  float Mr[kRT], Lr[kRT];
-  lds_char* box = ring + w * L::BOX + 16 * lane;
-#pragma unroll
-  for (int t = 0; t < kRT; ++t) {
-    float mk[4], lk[4], sk[4];
-#pragma unroll
-    for (int kk = 0; kk < 4; ++kk) {
-      const f32x2 v = *(const lds_f32x2*)(ml + (((kQuarters * h + kk) * kRT + t) * 16 + n16) * 8);
-      mk[kk] = v.x;
-      lk[kk] = v.y;
-    }
-    const float M = fmaxf(fmaxf(mk[0], mk[1]), fmaxf(mk[2], mk[3]));
-#pragma unroll
-    for (int kk = 0; kk < 4; ++kk) sk[kk] = mk[kk] == kNegInf ? 0.f : fexp2(mk[kk] - M);
-    Mr[t] = M;
-    Lr[t] = (lk[0] * sk[0] + lk[1] * sk[1]) + (lk[2] * sk[2] + lk[3] * sk[3]);
-    const float sa = p ? sk[2] : sk[0], sb = p ? sk[3] : sk[1];
-#pragma unroll
-    for (int j = 0; j < DT; ++j) acc[0][t][j] = acc[0][t][j] * sa + acc[1][t][j] * sb;
-  }
-  // Branches with constant indices: a run-time choice between accumulators would
-  // put them in scratch memory.
-  f32x4 sv[kRT][HT];
-#pragma unroll
-  for (int t = 0; t < kRT; ++t)
-#pragma unroll
-    for (int j = 0; j < HT; ++j) {
-      f32x4 give;
-      if (p) {
-        give = acc[0][t][j];
-        sv[t][j] = acc[0][t][HT + j];
-      } else {
-        give = acc[0][t][HT + j];
-        sv[t][j] = acc[0][t][j];
-      }
-      *(lds_f32x4*)(box + (t * HT + j) * 1024) = give;
-    }
-  lds_barrier();
-  const lds_char* other = ring + (w ^ 1) * L::BOX + 16 * lane;
-#pragma unroll
-  for (int t = 0; t < kRT; ++t)
-#pragma unroll
-    for (int j = 0; j < HT; ++j) sv[t][j] = sv[t][j] + *(const lds_f32x4*)(other + (t * HT + j) * 1024);
-  lds_barrier();   // every wave's ring reads are complete: before_stores may load into it
-  before_stores();
-  const __amdgpu_buffer_rsrc_t racc = buffer_rsrc(A.gp_acc, 0x7fffffff);
-#pragma unroll
-  for (int t = 0; t < kRT; ++t) {
-    const int r = trow + 16 * t + n16;
-    if (r >= A.R) continue;
-    const size_t mo = ((size_t)g * A.R + r) * A.NG + q;   // (m, l) pair index
-    if (p == 0 && g4 == 0) {
-      if constexpr (ATOMIC)
-        __builtin_amdgcn_raw_buffer_store_b64(f32x2{Mr[t], Lr[t]}, buffer_rsrc(A.gp_ml, 0x7fffffff), (int)(mo * 8), 0, 16);
-      else *reinterpret_cast<f32x2*>(A.gp_ml + 2 * mo) = f32x2{Mr[t], Lr[t]};
-    }
-#pragma unroll
-    for (int j = 0; j < HT; ++j) {
-      const size_t off = mo * D + 16 * (HT * p + j) + 4 * g4;
-      if constexpr (ATOMIC) __builtin_amdgcn_raw_buffer_store_b128(sv[t][j], racc, (int)(off * 4), 0, 16);
-      else *reinterpret_cast<f32x4*>(A.gp_acc + off) = sv[t][j];
-    }
-  }
+  if constexpr (!MULTI) finish(ring);   // (every slot is free once all waves are past their last step)
 }
 
+// Grid (kv head, 128-row block, split z of Z): key groups [z NG / Z, (z + 1) NG / Z).
 template <int D>
 __global__ __launch_bounds__(512) void prompt_pair_kernel(TrieAttnArgs A) {
   __shared__ __attribute__((aligned(1024))) char lds[PairLds<D>::BYTES];
-  pair_block<D, false>(A, lds, blockIdx.x, blockIdx.y, blockIdx.z, [] {});
+  const int z = blockIdx.z, Z = gridDim.z;
+  pair_block<D, false, true>(A, lds, blockIdx.x, blockIdx.y, z * A.NG / Z, (z + 1) * A.NG / Z, [] {});
 }
 
 // ------------------------------------------------------------------ node partials and merge
@@ -2733,7 +2760,7 @@ __global__ __launch_bounds__(512) void fused_pair_kernel(TrieAttnArgs A) {
   const int old = counter_before(A, g, rb);
   const bool pf = A.NN > 0 && A.NN <= LY::RES * kChunk && r0 < rend;
   NodePre<D> pre;
-  pair_block<D, true>(A, lds, g, rb, q, [&] {
+  pair_block<D, true, false>(A, lds, g, rb, q, q + 1, [&] {
     if (pf) node_prefetch<D>(A, g, r0, rend0, (lds_char*)lds, w, pre);
   });
   count_partial(A, g, rb, q);
@@ -2825,6 +2852,20 @@ static int fused_capacity() {
 }
 
 
+// How many workgroups share the NG key groups of a 128-row block (S steps each),
+// blocks = kv heads x row blocks: the least time for the busiest CU, from what a
+// workgroup spends (8B heads, in 0.1 us): 45 before its first round, 28 a round of
+// four steps, 15 a group's end.
+static int pair_splits(int blocks, int NG, int S) {
+  int best = 1;
+  int64_t t_best = 0;
+  for (int z = 1; z <= NG; ++z) {
+    const int64_t t = ((int64_t)blocks * z + 255) / 256 * (45 + (int64_t)((NG + z - 1) / z) * (28 * (S / kQuarters) + 15));
+    if (z == 1 || t < t_best) { best = z; t_best = t; }
+  }
+  return best;
+}
+
 template <int D, int RT>
 static void launch_rt(const TrieAttnArgs& a, const Plan& pl, hipStream_t s, int mode) {
   const bool one = pl.NG > 0 && mode != 2 && 1 + 2 * pl.NRB * a.HK <= kSyncWords &&
@@ -2853,7 +2894,8 @@ static void launch_rt(const TrieAttnArgs& a, const Plan& pl, hipStream_t s, int 
       hipLaunchKernelGGL((fused_pair_kernel<D>), g2, b8, 0, s, b);
       return;
     }
-    if (pl.prompt_wgs > 0) hipLaunchKernelGGL((prompt_pair_kernel<D>), g2, b8, 0, s, a);
+    if (pl.prompt_wgs > 0)
+      hipLaunchKernelGGL((prompt_pair_kernel<D>), dim3(a.HK, nrb2, pair_splits(a.HK * nrb2, pl.NG, pl.S)), b8, 0, s, a);
   }
   if constexpr (D <= 128) {
     // Nodes and merge: 64-row blocks once they give a quarter of the CUs a workgroup
