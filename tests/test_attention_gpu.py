@@ -521,6 +521,7 @@ def test_tiled_output_rejects_a_head_stride_other_than_d():
     (8, 2, 64, 300, 64, "random"),         # no common run
     (8, 8, 128, 230, 40, "holes"),         # rows without any node slot, and causal rows
     (8, 2, 128, 320, 100, "nan"),          # NaN / inf K and V in slots that later rows alone may see
+    (8, 2, 64, 700, 33, "nan"),            # the same in a segment of 704 slots
     (8, 2, 64, 1000, 100, "random"),       # 1024 slots: the longest segment node_stream takes
     (8, 2, 32, 500, 64, "open32k"),        # 512 slots: its longest at head_dim 32
     (8, 2, 32, 530, 33, "causal"),         # 544 slots: gathered
