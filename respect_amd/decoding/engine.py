@@ -212,6 +212,13 @@ class Decoder:
         the prompt segment and [P, P + NN) the node segment; msk [T, NN] uint8
         (row t may attend to node slot j).  Returns fp32 logits [T, V].
         """
+        y = self._layers(ids, slots, positions, cache, P, msk, NN)
+        return self._linear(y.data_ptr(), _lib.RSPX_TILED, int(ids.shape[0]), self.t_lm_head, out_dtype=torch.float32)
+
+    def _layers(self, ids, slots, positions, cache, P: int, msk, NN: int, kv_only: bool = False) -> torch.Tensor | None:
+        """forward's layers: the final normalised rows [T, H] in the tiled layout.
+        ``kv_only``: only the K/V of the tokens is wanted; the last layer stops
+        once it has written them, and None is returned."""
         cfg = self.cfg
         L = _lib.lib()
         dev = self.device
@@ -241,6 +248,8 @@ class Decoder:
                 qkvp, S, lay.q_norm.data_ptr(), lay.k_norm.data_ptr(), cos.data_ptr(),
                 sin.data_ptr(), cos.stride(0), slots32.data_ptr(), cache.cap, ck.data_ptr(), ck.stride(0), ck.stride(1),
                 cv.data_ptr(), cv.stride(0), cv.stride(1), qo.data_ptr(), T, HQ, HK, D, cfg.eps, s))
+            if kv_only and li + 1 == len(self.layers):
+                return None
             trie_attn(qo.permute(1, 0, 2), ck[:, :P], cv[:, :P], ck[:, P:P + NN], cv[:, P:P + NN], msk,
                       self.sm_scale, out=att, workspace=ws_attn, out_tiled=True)
             hp, S = self._partials(att.data_ptr(), TILED, T, lay.tout)
@@ -263,27 +272,32 @@ class Decoder:
             _lib.check("rspx_add_rmsnorm_partials", L.rspx_add_rmsnorm_partials(
                 x.data_ptr(), Hd, hp, S, nxt.data_ptr(), x.data_ptr(), Hd, y.data_ptr(), TILED,
                 T, Hd, cfg.eps, s))
-        return self._linear(y.data_ptr(), TILED, T, self.t_lm_head, out_dtype=torch.float32)
+        return y
 
     # ------------------------------------------------------------------ prompt
     @torch.no_grad()
     def prefill(self, ids: torch.Tensor, cache, chunk: int = 512) -> torch.Tensor:
         """Fill cache slots [0, len(ids)) with the prompt's KV, ``chunk`` tokens per
         forward: a chunk sees the earlier chunks as its prompt segment and
-        itself causally as its node segment.  Returns the last row's logits."""
+        itself causally as its node segment.  Returns the last row's logits [1, V]:
+        the vocabulary projection runs for that row alone, and earlier chunks end
+        with the last layer's K/V."""
         n = int(ids.shape[0])
         if n > cache.cap:
             raise ValueError(f"prefill: {n} prompt tokens exceed the cache's {cache.cap} slots")
         dev = self.device
-        logits = None
+        last = None
         for c0 in range(0, n, chunk):
             c1 = min(n, c0 + chunk)
             T = c1 - c0
             NN = -(-T // 32) * 32
             msk = torch.tril(torch.ones(T, NN, dtype=torch.uint8, device=dev))
             pos = torch.arange(c0, c1, device=dev)
-            logits = self.forward(ids[c0:c1], pos.to(torch.int32), pos, cache, c0, msk, NN)
-        return logits[-1:]
+            y = self._layers(ids[c0:c1], pos.to(torch.int32), pos, cache, c0, msk, NN, kv_only=c1 < n)
+            if c1 == n:   # row T - 1 of the tiled rows (RSPX_TILED): elements 32 b + 8 g + e at [b, g, e]
+                m = T - 1
+                last = y.view(-1, self.cfg.hidden // 32, 4, 4, 16, 8)[m // 64, :, m % 64 // 16, :, m % 16].reshape(1, -1)
+        return self._linear(last.data_ptr(), last.stride(0), 1, self.t_lm_head, out_dtype=torch.float32)
 
     # ------------------------------------------------------------------ graphs
     def graphed(self, cache, P: int, T: int, NN: int) -> "GraphedForward":
