@@ -581,13 +581,24 @@ __global__ __launch_bounds__(256) void reduce_kernel(const float* part, int S, i
 // Any shape outside gemm_kernel's (N % 16 != 0 or K % 256 != 0): one chain
 // of v_mfma_f32_16x16x32_bf16 over the 32-wide k-blocks of K in increasing k,
 // rounded once -- an order fixed by K alone, so a row's bits never depend on
-// M.  Workgroup = 4 waves on adjacent 16-column groups of a 64-column tile,
-// times one 64-row tile (MT row tiles of 16).  Operands go from memory
-// straight into the MFMA registers through bounded buffer loads: rows past M,
-// columns past N and k past K get an out-of-range offset and read as zero, so
-// they add exact zeros to the chain.  V16 (every row 16-byte aligned, K % 8
-// == 0): a lane's 8 consecutive k come in one 16-byte load, else in eight
-// 2-byte loads; both give the same operand values.
+// M.  Workgroup = 64 CT columns (4 waves of CT 16-column tiles) times 16 MT rows.
+//
+// What bounded it: one k-block at a time from memory into the MFMA registers, a
+// memory latency per k-block, and every wave reading all of X by itself.  Now W
+// fragments go into a ring of registers 3 rounds of KB k-blocks ahead, and X is
+// shared: the waves load a round's fragments 3 rounds ahead, one part each, and
+// put them into one of two LDS buffers a round before use.  X passes through
+// registers, not direct-to-LDS loads, because a lane's 8 k may start at any 2-byte
+// address and end past K.  No load reaches past a row's K elements and none sits
+// under a branch (a load under one makes the compiler drain all before it): a
+// group that K cuts, or a round past K, loads the row's last 8 elements.  What K
+// leaves past its whole rounds is taken once at the end, such a group shifted into
+// place with zeros past K, so that it adds exact zeros to the chain.  Rows past M and columns past N read the last row or column;
+// their results are not stored.
+//
+// 77 x 4864 x 896: 21.3 -> 8.0 us (1.1 TB/s of 9.6 MB); 23 x 9976 x 6596, rows not
+// 16-byte aligned: 304 -> 39.6 us (3.3 TB/s); 512 x 9976 x 6596: 3.10 -> 0.192 ms
+// (350 TFLOP/s); 1024 x 5504 x 4416: 469 -> 118 us (422 TFLOP/s).
 struct AnyArgs {
   const uint16_t* x; int64_t sx;  // [M, K]
   const uint16_t* w; int64_t sw;  // [N, K]
@@ -595,70 +606,189 @@ struct AnyArgs {
   int M, N, K, out_fp32;
 };
 
-// The MFMA operand of one lane: row `row` (element offset roff from the
-// descriptor's base; ok = the row exists), k .. k + 7.
-template <bool V16>
-__device__ __forceinline__ u32x4 any_frag(__amdgpu_buffer_rsrc_t r, int roff, bool ok, int k, int K) {
-  if constexpr (V16) {
-    return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, ok && k < K ? (roff + k) * 2 : kOOB, 0, 0));
-  } else {
-    uint32_t h[8];
+// The 16 bytes at p, any 2-byte address (one instruction on this target).
+__device__ __forceinline__ u32x4 any_load(const uint16_t* p) {
+  u32x4 v;
+  __builtin_memcpy(&v, p, 16);
+  return v;
+}
+
+// Elements k .. k + 7 of a row, zero past K, from v = the 8 elements at min(k, K - 8).
+__device__ __forceinline__ u32x4 any_cut(u32x4 v, int k, int K) {
+  const int s = max(0, k + 8 - K);   // elements past K
+  if (s & 1) {
 #pragma unroll
-    for (int j = 0; j < 8; ++j)
-      h[j] = __builtin_amdgcn_raw_buffer_load_b16(r, ok && k + j < K ? (roff + k + j) * 2 : kOOB, 0, 0);
-    return u32x4{h[0] | (h[1] << 16), h[2] | (h[3] << 16), h[4] | (h[5] << 16), h[6] | (h[7] << 16)};
+    for (int i = 0; i < 4; ++i) v[i] = (v[i] >> 16) | (i < 3 ? v[i + 1 < 4 ? i + 1 : 3] << 16 : 0u);
+  }
+  u32x4 o;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    uint32_t x = 0u;
+#pragma unroll
+    for (int j = i; j < 4; ++j) x = j - i == s >> 1 ? v[j] : x;
+    o[i] = x;
+  }
+  return o;
+}
+
+template <int MT, int CT> constexpr int any_kb() { return CT * MT >= 16 ? 1 : CT == 1 && MT <= 2 ? 4 : 2; }   // k-blocks of a round
+
+template <int MT, int CT>
+__global__ __launch_bounds__(256, 2) void gemm_any_kernel(AnyArgs A, int units, int mtiles) {
+  constexpr int KB = any_kb<MT, CT>();
+  constexpr int NC = KB * MT;           // 1 KB X fragments of a round
+  constexpr int XL = (NC + 3) / 4;      // fragments a wave loads per round
+  __shared__ __attribute__((aligned(16))) char xs[2 * XL * 4 * 1024];
+  const int lane = __lane_id();
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int n16 = lane & 15, g4 = lane >> 4;
+  const int j = blockIdx.x >> 3;        // as gemm_wide_kernel: the row tiles of a column slice on one XCD
+  const int nt = (blockIdx.x & 7) + 8 * (j / mtiles), mt = j % mtiles;
+  if (nt >= units) return;
+  const int col = nt * 64 * CT + 16 * CT * w, row0 = mt * 16 * MT;
+  const int K = A.K, nkb = (K + 31) >> 5, nr = K / (32 * KB);   // nr: whole rounds
+
+  const uint16_t* wp[CT];
+#pragma unroll
+  for (int c = 0; c < CT; ++c) wp[c] = A.w + (int64_t)min(col + 16 * c + n16, A.N - 1) * A.sw;
+  const uint16_t* xp[XL];
+  int xk[XL];                           // k of the lane's fragment jj (w + 4 jj: k-block c / MT, row tile c % MT)
+#pragma unroll
+  for (int jj = 0; jj < XL; ++jj) {
+    const int c = w + 4 * jj;
+    xp[jj] = A.x + (int64_t)min(row0 + 16 * (c % MT) + n16, A.M - 1) * A.sx;
+    xk[jj] = c < NC ? 32 * (c / MT) + 8 * g4 : 0x40000000;   // past any K: zeros
+  }
+  lds_char_t* xl = (lds_char_t*)xs;
+  typedef __attribute__((address_space(3))) u32x4 lds_u32x4_t;
+  f32x4 acc[MT][CT];
+#pragma unroll
+  for (int t = 0; t < MT; ++t)
+#pragma unroll
+    for (int c = 0; c < CT; ++c) acc[t][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+  u32x4 wf[4][KB][CT], xr[2][XL];
+
+  auto load_w = [&](int r, u32x4 (&f)[KB][CT]) {
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+      for (int c = 0; c < CT; ++c) f[kb][c] = any_load(wp[c] + min(32 * (KB * r + kb) + 8 * g4, K - 8));
+    asm volatile("" ::: "memory");   // the loads stay in this order, so the waits for them are exact
+  };
+  auto load_x = [&](int r, u32x4 (&f)[XL]) {
+#pragma unroll
+    for (int jj = 0; jj < XL; ++jj) f[jj] = any_load(xp[jj] + min(32 * KB * r + xk[jj], K - 8));
+    asm volatile("" ::: "memory");
+  };
+  auto put_x = [&](int r, const u32x4 (&f)[XL]) {
+#pragma unroll
+    for (int jj = 0; jj < XL; ++jj)
+      *(lds_u32x4_t*)(xl + ((r & 1) * XL * 4 + w + 4 * jj) * 1024 + 16 * lane) = f[jj];
+  };
+  auto compute = [&](int r, int n, const u32x4 (&f)[KB][CT]) {   // the round's first n k-blocks
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) {
+      if (kb >= n) break;
+      u32x4 xf[MT];
+#pragma unroll
+      for (int t = 0; t < MT; ++t)
+        xf[t] = *(const lds_u32x4_t*)(xl + ((r & 1) * XL * 4 + kb * MT + t) * 1024 + 16 * lane);
+#pragma unroll
+      for (int t = 0; t < MT; ++t)
+#pragma unroll
+        for (int c = 0; c < CT; ++c)
+          acc[t][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, f[kb][c]),
+                                                              __builtin_bit_cast(bf16x8, xf[t]), acc[t][c], 0, 0, 0);
+    }
+  };
+  load_x(0, xr[0]);
+  load_w(0, wf[0]);
+  load_x(1, xr[1]);
+  load_w(1, wf[1]);
+  put_x(0, xr[0]);
+  load_x(2, xr[0]);
+  load_w(2, wf[2]);
+  int r0 = 0;
+  for (; r0 + 4 <= nr; r0 += 4) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int r = r0 + u;
+      raw_barrier();   // round r's X is in LDS; every wave is done with round r - 1's buffer
+      put_x(r + 1, xr[(u + 1) & 1]);
+      load_x(r + 3, xr[(u + 1) & 1]);
+      load_w(r + 3, wf[(u + 3) & 3]);
+      compute(r, KB, wf[u]);
+    }
+  }
+  // Up to three more whole rounds, already requested (a way out of the middle of
+  // the loop would blur its waits).
+#pragma unroll
+  for (int u = 0; u < 3; ++u) {
+    if (r0 + u >= nr) break;
+    raw_barrier();
+    put_x(r0 + u + 1, xr[(u + 1) & 1]);
+    compute(r0 + u, KB, wf[u]);
+  }
+  if (KB * nr < nkb) {
+    // What is left of K, less than a round.
+    load_x(nr, xr[0]);
+    load_w(nr, wf[0]);
+#pragma unroll
+    for (int jj = 0; jj < XL; ++jj) xr[0][jj] = any_cut(xr[0][jj], 32 * KB * nr + xk[jj], K);
+    raw_barrier();   // every wave is done with the buffer
+    put_x(nr, xr[0]);
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+      for (int c = 0; c < CT; ++c) wf[0][kb][c] = any_cut(wf[0][kb][c], 32 * (KB * nr + kb) + 8 * g4, K);
+    raw_barrier();
+    compute(nr, nkb - KB * nr, wf[0]);
+  }
+  // acc[t][c][e] = D[column 16 c + 4 g4 + e][row 16 t + n16] of the wave's tiles.
+#pragma unroll
+  for (int t = 0; t < MT; ++t) {
+    const int m = row0 + 16 * t + n16;
+    if (m >= A.M) continue;
+#pragma unroll
+    for (int c = 0; c < CT; ++c)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int n = col + 16 * c + 4 * g4 + e;
+        if (n >= A.N) continue;
+        if (A.out_fp32)
+          static_cast<float*>(A.out)[(int64_t)m * A.so + n] = acc[t][c][e];
+        else
+          static_cast<uint16_t*>(A.out)[(int64_t)m * A.so + n] = f32_to_bf16_rne(acc[t][c][e]);
+      }
   }
 }
 
-template <int MT, bool V16>
-__global__ __launch_bounds__(256) void gemm_any_kernel(AnyArgs A) {
-  const int lane = __lane_id(), wv = threadIdx.x >> 6;
-  const int n16 = lane & 15, g4 = lane >> 4;
-  const int n0 = blockIdx.x * 64 + wv * 16, m0 = blockIdx.y * kRows;
-  if (n0 >= A.N) return;  // whole wave; no barriers below
-  const int nw = min(16, A.N - n0), mw = min(kRows, A.M - m0);
-  // Descriptors start at the wave's first column and the tile's first row,
-  // so every offset fits 31 bits (the host checks 64 rows of x and 16 of w).
-  const __amdgpu_buffer_rsrc_t rw = rsrc(A.w + (int64_t)n0 * A.sw, ((int64_t)(nw - 1) * A.sw + A.K) * 2);
-  const __amdgpu_buffer_rsrc_t rx = rsrc(A.x + (int64_t)m0 * A.sx, ((int64_t)(mw - 1) * A.sx + A.K) * 2);
-  const bool wok = n16 < nw;
-  const int woff = n16 * (int)A.sw;
-  int xoff[MT];
-  bool xok[MT];
+// K < 8: no row holds a 16-byte group.  One 16 x 16 tile per wave, its elements
+// loaded one by one into the single k-block of the chain.
+__global__ __launch_bounds__(64) void gemm_small_k_kernel(AnyArgs A, int ntiles) {
+  const int lane = __lane_id(), n16 = lane & 15, g4 = lane >> 4;
+  const int n0 = 16 * (int)(blockIdx.x % ntiles);
+  const int64_t m0 = 16 * (int64_t)(blockIdx.x / ntiles);
+  u32x4 wf = {0u, 0u, 0u, 0u}, xf = wf;
+  if (g4 == 0) {
 #pragma unroll
-  for (int t = 0; t < MT; ++t) {
-    xok[t] = 16 * t + n16 < mw;
-    xoff[t] = (16 * t + n16) * (int)A.sx;
-  }
-  f32x4 acc[MT];
-#pragma unroll
-  for (int t = 0; t < MT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const int nkb = (A.K + 31) >> 5;
-  for (int kb = 0; kb < nkb; ++kb) {
-    const int k = 32 * kb + 8 * g4;
-    const u32x4 wf = any_frag<V16>(rw, woff, wok, k, A.K);
-    u32x4 xf[MT];
-#pragma unroll
-    for (int t = 0; t < MT; ++t) xf[t] = any_frag<V16>(rx, xoff[t], xok[t], k, A.K);
-#pragma unroll
-    for (int t = 0; t < MT; ++t)
-      acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wf), __builtin_bit_cast(bf16x8, xf[t]),
-                                                       acc[t], 0, 0, 0);
-  }
-  // acc[t][e] = D[column 4 g4 + e][row 16 t + n16] of the wave's tile.
-#pragma unroll
-  for (int t = 0; t < MT; ++t) {
-    const int m = m0 + 16 * t + n16;
-    if (m >= A.M) continue;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int n = n0 + 4 * g4 + e;
-      if (n >= A.N) continue;
-      if (A.out_fp32)
-        static_cast<float*>(A.out)[(int64_t)m * A.so + n] = acc[t][e];
-      else
-        static_cast<uint16_t*>(A.out)[(int64_t)m * A.so + n] = f32_to_bf16_rne(acc[t][e]);
+    for (int j = 0; j < 7; ++j) {
+      if (j >= A.K) break;
+      if (n0 + n16 < A.N) wf[j / 2] |= (uint32_t)A.w[(int64_t)(n0 + n16) * A.sw + j] << (16 * (j & 1));
+      if (m0 + n16 < A.M) xf[j / 2] |= (uint32_t)A.x[(m0 + n16) * A.sx + j] << (16 * (j & 1));
     }
+  }
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wf), __builtin_bit_cast(bf16x8, xf), acc, 0, 0,
+                                                0);
+  const int64_t m = m0 + n16;
+  if (m >= A.M) return;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const int n = n0 + 4 * g4 + e;
+    if (n >= A.N) continue;
+    if (A.out_fp32) static_cast<float*>(A.out)[m * A.so + n] = acc[e];
+    else static_cast<uint16_t*>(A.out)[m * A.so + n] = f32_to_bf16_rne(acc[e]);
   }
 }
 
@@ -745,6 +875,26 @@ static int reduce_launch(const gemm::Args& a, hipStream_t s) {
   return hipGetLastError() == hipSuccess ? RSPX_OK : RSPX_ELAUNCH;
 }
 
+// Column tiles per wave of gemm_wide_kernel and gemm_any_kernel, 4, 4 - step, ..:
+// the least time for the busiest CU, workgroups per CU times a workgroup's time for
+// its 16 ct columns per wave (tiles: row tiles times K chunks).  Narrower waves read
+// each X fragment for fewer MFMAs, so ct = 1 .. 4 cost 14 : 24 : 31 : 40 and not
+// 1 : 2 : 3 : 4 (512 rows, o projection [4096, 4096]: 33.1 / 27.5 / 32.6 / 23.0 us
+// at ct = 1 .. 4 with 4 / 2 / 2 / 1 workgroups per CU; 512 rows, gate/up
+// [24576, 4096]: 144.8 / 115.8 / 103.3 / 116.7 us with 6 / 3 / 2 / 2; 128 rows,
+// q/k/v [6144, 4096]: 20.1 / 16.5 / 19.3 / 22.2 us with 2 / 1 / 1 / 1; 512 rows,
+// [9976, 6596]: 216 / 259 / - / 192 us with 3 / 2 / - / 1).
+static int columns_per_wave(int N, int64_t tiles, int step) {
+  static const int cost[5] = {0, 14, 24, 31, 40};
+  int ct = 4;
+  int64_t best = 0;
+  for (int c = 4; c >= 1; c = c > step || c == 1 ? c - step : 1) {
+    const int64_t t = ((int64_t)((N + 64 * c - 1) / (64 * c)) * tiles + 255) / 256 * cost[c];
+    if (c == 4 || t < best) { ct = c; best = t; }
+  }
+  return ct;
+}
+
 // 31-bit byte offsets inside a 128-row tile of x and a wave's 64 rows of w.
 static bool wide_fits(const gemm::Args& a) {
   return (a.x_tiled || (int64_t)128 * a.sx * 2 < (1ll << 30)) && (a.sw == kTiled || (int64_t)64 * a.sw * 2 < (1ll << 30)) &&
@@ -755,20 +905,7 @@ static int wide_launch(const gemm::Args& a, hipStream_t s) {
   // Row tiles of at most 128 rows, all of the same height.
   const int mtiles = (a.M + 127) / 128;
   const int mt = ((a.M + mtiles - 1) / mtiles + 15) / 16;
-  // Column tiles per wave: the least time for the busiest CU, workgroups per CU
-  // times a workgroup's time for its 16 ct columns per wave.  Narrower waves read
-  // each X fragment for fewer MFMAs, so ct = 1 .. 4 cost 14 : 24 : 31 : 40 and not
-  // 1 : 2 : 3 : 4 (512 rows, o projection [4096, 4096]: 33.1 / 27.5 / 32.6 / 23.0 us
-  // at ct = 1 .. 4 with 4 / 2 / 2 / 1 workgroups per CU; 512 rows, gate/up
-  // [24576, 4096]: 144.8 / 115.8 / 103.3 / 116.7 us with 6 / 3 / 2 / 2; 128 rows,
-  // q/k/v [6144, 4096]: 20.1 / 16.5 / 19.3 / 22.2 us with 2 / 1 / 1 / 1).
-  static const int cost[5] = {0, 14, 24, 31, 40};
-  int ct = 4;
-  int64_t best = 0;
-  for (int c = 4; c >= 1; --c) {
-    const int64_t t = ((int64_t)((a.N + 64 * c - 1) / (64 * c)) * a.S * mtiles + 255) / 256 * cost[c];
-    if (c == 4 || t < best) { ct = c; best = t; }
-  }
+  const int ct = columns_per_wave(a.N, a.S * mtiles, 1);
   const int64_t units = (int64_t)((a.N + 64 * ct - 1) / (64 * ct)) * a.S;
   const int64_t wgs = (units + 7) / 8 * 8 * mtiles;
   if (wgs > 0x7fffffff) return RSPX_EUNSUPPORTED;
@@ -803,8 +940,9 @@ static int linear_launch(const void* x, int64_t sx, const void* w, int64_t sw, v
   a.silu = silu;
   a.x_tiled = sx == kTiled;
   a.out_tiled = silu && so == kTiled;
-  if (M > gemm::kRows && wide_fits(a)) return wide_launch(a, s);
   const int MTILES = (M + gemm::kRows - 1) / gemm::kRows;
+  if (MTILES > 65535) return RSPX_EUNSUPPORTED;
+  if (M > gemm::kRows && wide_fits(a)) return wide_launch(a, s);
   // 8 waves (128 columns) share each X round between twice the columns; worth
   // it while the grid keeps >= 192 workgroups, and for the widest layers
   // (the vocabulary head) only when the X block is large (many rows).
@@ -817,7 +955,6 @@ static int linear_launch(const void* x, int64_t sx, const void* w, int64_t sw, v
   const int waves = (N % 96 == 0 && wg8 < 256 && wg6 >= 256 && wg6 <= 512) ? 6
                     : (wg8 >= 192 && (M >= 32 || wg8 < 1024)) ? 8 : 4;
   const int NT = (N + 16 * waves - 1) / (16 * waves);
-  if (MTILES > 65535) return RSPX_EUNSUPPORTED;
   const int mt = (MTILES > 1 || M >= 64) ? 4 : (M + 15) / 16;  // row tiles per 64-row tile
   // X-resident blocks pay where X is large against each block's W slice and
   // the grid is one wave of 6- or 8-wave blocks (q/k/v [64 x 4096] .
@@ -888,20 +1025,41 @@ static int linear_any(const void* x, int64_t sx, const void* w, int64_t sw, void
   // 31-bit byte offsets inside one 64-row tile of x and one 16-row slice of w.
   if (((int64_t)gemm::kRows * sx + K) * 2 >= (1ll << 31) - 64 || ((int64_t)16 * sw + K) * 2 >= (1ll << 31) - 64)
     return RSPX_EUNSUPPORTED;
-  const int64_t gx = (N + 63) / 64, gy = (M + gemm::kRows - 1) / gemm::kRows;
-  if (gy > 65535) return RSPX_EUNSUPPORTED;
+  if ((M + gemm::kRows - 1) / gemm::kRows > 65535) return RSPX_EUNSUPPORTED;
   gemm::AnyArgs a{static_cast<const uint16_t*>(x), sx, static_cast<const uint16_t*>(w), sw, out, so, M, N, K,
                   out_fp32 ? 1 : 0};
-  const bool v16 = K % 8 == 0 && sx % 8 == 0 && sw % 8 == 0 && al(x, 16) && al(w, 16);
-  const int mt = M >= gemm::kRows ? 4 : (M + 15) / 16;
-  const dim3 g((unsigned)gx, (unsigned)gy), b(256);
-#define RSPX_ANY_MT(V)                                                                   \
-  if (mt == 4) hipLaunchKernelGGL((gemm::gemm_any_kernel<4, V>), g, b, 0, s, a);         \
-  else if (mt == 3) hipLaunchKernelGGL((gemm::gemm_any_kernel<3, V>), g, b, 0, s, a);    \
-  else if (mt == 2) hipLaunchKernelGGL((gemm::gemm_any_kernel<2, V>), g, b, 0, s, a);    \
-  else hipLaunchKernelGGL((gemm::gemm_any_kernel<1, V>), g, b, 0, s, a);
-  if (v16) { RSPX_ANY_MT(true) }
-  else { RSPX_ANY_MT(false) }
+  if (K < 8) {
+    const int64_t tiles = (int64_t)((N + 15) / 16) * ((M + 15) / 16);
+    if (tiles > 0x7fffffff) return RSPX_EUNSUPPORTED;
+    hipLaunchKernelGGL(gemm::gemm_small_k_kernel, dim3((unsigned)tiles), dim3(64), 0, s, a, (N + 15) / 16);
+    return hipGetLastError() == hipSuccess ? RSPX_OK : RSPX_ELAUNCH;
+  }
+  // Row tiles of 1, 2, 4, 6 or 8 16-row tiles and 1, 2 or 4 column tiles a wave
+  // (columns_per_wave); where that leaves CUs without a workgroup, lower row tiles
+  // while the grid stays within one workgroup per CU (77 x 4864 x 896: 12.1 -> 8.0
+  // us, 64 x 5000 x 2600: 25.9 -> 18.3; up to two per CU: 10.7, 26.6).
+  const int mtiles = (M + 127) / 128, rows = (M + mtiles - 1) / mtiles;
+  const int ct = columns_per_wave(N, mtiles, 2);
+  const int64_t units = (N + 64 * ct - 1) / (64 * ct);
+  int mt = rows <= 16 ? 1 : rows <= 32 ? 2 : rows <= 64 ? 4 : rows <= 96 ? 6 : 8;
+  auto row_tiles = [&](int t) { return (M + 16 * t - 1) / (16 * t); };
+  while (ct == 1 && mt > 1 && units * row_tiles(mt == 6 ? 4 : mt / 2) <= 256) mt = mt == 6 ? 4 : mt / 2;
+  const int64_t mtl = row_tiles(mt);
+  const int64_t wgs = (units + 7) / 8 * 8 * mtl;
+  if (wgs > 0x7fffffff) return RSPX_EUNSUPPORTED;
+  const dim3 g((unsigned)wgs), b(256);
+#define RSPX_ANY(MTV, CTV) \
+  hipLaunchKernelGGL((gemm::gemm_any_kernel<MTV, CTV>), g, b, 0, s, a, (int)units, (int)mtl);
+#define RSPX_ANY_MT(CTV)                                \
+  if (mt == 1) { RSPX_ANY(1, CTV) }                     \
+  else if (mt == 2) { RSPX_ANY(2, CTV) }                \
+  else if (mt == 4) { RSPX_ANY(4, CTV) }                \
+  else if (mt == 6) { RSPX_ANY(6, CTV) }                \
+  else { RSPX_ANY(8, CTV) }
+  if (ct == 1) { RSPX_ANY_MT(1) }
+  else if (ct == 2) { RSPX_ANY_MT(2) }
+  else { RSPX_ANY_MT(4) }
+#undef RSPX_ANY
 #undef RSPX_ANY_MT
   return hipGetLastError() == hipSuccess ? RSPX_OK : RSPX_ELAUNCH;
 }

@@ -460,3 +460,33 @@ def test_linear_many_rows(M, N, K):
                                                               N // 2, m1 - m0, N, K, s))
             return o
         assert torch.equal(silu(0, M), torch.cat([silu(i, min(M, i + 64)) for i in range(0, M, 64)]))
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 1, 1), (5, 40, 7), (17, 30, 8), (1, 65, 9), (16, 64, 63), (33, 129, 64),
+                                   (64, 100, 65), (97, 300, 127), (128, 272, 129), (129, 4100, 200), (40, 16500, 96),
+                                   (300, 9000, 72)])
+def test_linear_any_shape_edges(M, N, K):
+    """Outside N % 16 == 0, K % 256 == 0: K below one load, below a round, whole rounds with and
+    without a rest, every row and column tile height and width; the accumulation bound in fp32,
+    the bits of calls on single rows, and operands at 2-byte addresses whose rows end where the
+    allocation ends."""
+    from respect_amd import _lib
+    from respect_amd.kernels.gemm import linear
+    print(f"[linear any edges] M={M} N={N} K={K}", flush=True)
+    x, w = _xw(M * 3 + N + K, M, N, K)
+    xd, wd = _dev(x), _dev(w)
+    f32 = linear(xd, wd, out_dtype=torch.float32)
+    ex = G.linear_exact(x, w)
+    assert np.all(np.abs(f32.cpu().numpy().astype(np.float64) - ex) <= G.linear_error_bound(x, w) + 1e-30)
+    assert torch.equal(linear(xd, wd), f32.to(torch.bfloat16))
+    for m in sorted({0, M // 2, M - 1}):
+        assert torch.equal(linear(xd[m:m + 1], wd, out_dtype=torch.float32), f32[m:m + 1])
+    L, s = _lib.lib(), _lib.stream_ptr(xd.device)
+    xb = torch.empty(1 + M * K, device="cuda", dtype=torch.bfloat16)
+    wb = torch.empty(1 + N * K, device="cuda", dtype=torch.bfloat16)
+    xb[1:], wb[1:] = xd.reshape(-1), wd.reshape(-1)
+    ob = torch.full((M, N), float("nan"), device="cuda")
+    _lib.check("rspx_linear", L.rspx_linear(xb.data_ptr() + 2, K, wb.data_ptr() + 2, K, ob.data_ptr(), N, M, N, K, 1,
+                                            None, 0, s))
+    torch.cuda.synchronize()
+    assert torch.equal(ob, f32)
