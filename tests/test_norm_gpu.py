@@ -344,3 +344,44 @@ def test_silu_mul_any_width(rows, F, off):
     assert torch.isnan(y[:, F].float()).all()
     aligned = silu_mul(_dev(gu[:, :F]), _dev(gu[:, F:]))
     assert torch.equal(y[:, :F], aligned)
+
+
+@pytest.mark.parametrize("rows,F", [(1, 8), (3, 2056), (342, 12288), (1025, 4104)])
+def test_silu_mul_eight_elements(rows, F):
+    """Widths and alignments at which a thread takes eight elements: the bits of the
+    two- and one-element forms (the same values at addresses only those take), and of
+    contiguous halves as of a packed gate/up tensor; infinities and NaN among them."""
+    from respect_amd import _lib
+    from respect_amd.system.fused import silu_mul
+    print(f"[silu_mul] rows={rows} F={F}", flush=True)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(rows)
+    gu = torch.randn(rows, 2 * F, generator=g, device="cuda").to(torch.bfloat16)
+    gu[0, :4] = torch.tensor([float("inf"), -float("inf"), float("nan"), -200.0], device="cuda")
+    bits = lambda t: t.contiguous().view(torch.int16)   # noqa: E731
+    out = silu_mul(gu[:, :F], gu[:, F:])
+    assert torch.equal(bits(silu_mul(gu[:, :F].contiguous(), gu[:, F:].contiguous())), bits(out))
+    L, s = _lib.lib(), _lib.stream_ptr(gu.device)
+    for off in (1, 2):   # elements past a 16-byte boundary: one and two elements per thread
+        buf = torch.zeros(rows * 2 * F + off, device="cuda", dtype=torch.bfloat16)
+        buf[off:] = gu.reshape(-1)
+        y = torch.empty(rows, F, device="cuda", dtype=torch.bfloat16)
+        p = buf.data_ptr() + 2 * off
+        _lib.check("rspx_silu_mul", L.rspx_silu_mul(p, 2 * F, p + 2 * F, 2 * F, y.data_ptr(), F, rows, F, s))
+        assert torch.equal(bits(y), bits(out))
+
+
+@pytest.mark.parametrize("B,H,L", [(1, 1, 1), (1, 32, 513), (1, 7, 2350), (2, 9, 1000)])
+def test_rope_heads_per_thread(B, H, L):
+    """Four heads per thread, H no multiple of four and L none of 16: bit for bit PyTorch's bf16
+    element-wise ops, from both orders of heads and tokens in memory."""
+    from respect_amd.system.fused import rope
+    print(f"[rope] B={B} H={H} L={L}", flush=True)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(L)
+    x = torch.randn(B, L, H, 128, generator=g, device="cuda").to(torch.bfloat16).transpose(1, 2)
+    cos, sin = (torch.randn(B, L, 128, generator=g, device="cuda").to(torch.bfloat16) for _ in range(2))
+    out = rope(x, cos, sin)
+    assert torch.equal(rope(x.contiguous(), cos, sin), out)
+    rot = torch.cat((-x[..., 64:], x[..., :64]), dim=-1)
+    assert torch.equal(x * cos[:, None] + rot * sin[:, None], out)
