@@ -401,8 +401,8 @@ __global__ __launch_bounds__(64 * W) void gemm_kernel(Args A) {
   for (int t = 0; t < MT; ++t) store_tile(A, s, row0 + 16 * t + n16, col + 4 * g4, acc[t]);
 }
 
-// More than 64 rows: workgroup = (64 CT output columns, chunk s, 16 MT rows), 4
-// waves of CT 16-column tiles, every wave over all MT row tiles.  The same MFMA
+// Many rows: workgroup = (16 W CT output columns, chunk s, 16 MT rows), W waves of
+// CT 16-column tiles, every wave over all MT row tiles.  The same MFMA
 // chain per element as gemm_kernel, in the same k order: the same bits.
 //
 // What bounds it: at one 16-column tile per wave (gemm_kernel) a k-block's X
@@ -414,21 +414,23 @@ __global__ __launch_bounds__(64 * W) void gemm_kernel(Args A) {
 // ahead, one barrier per round: the barrier that publishes round r's X also says
 // that every wave is done with round r - 1, whose buffer then takes round r + 3.
 //
-// Tiles of one 64 CT-column slice and chunk follow each other on one XCD
+// Tiles of one column slice and chunk follow each other on one XCD
 // (workgroups are dealt round-robin over the 8 XCDs), so its L2 reads the slice of
 // W from memory once for all row tiles.
 //
 // 512 rows, q/k/v [6144, 4096], o [4096, 4096], gate/up [24576, 4096] and down
 // [4096, 12288]: 35.6 / 23.0 / 103 / 49 us (0.72 / 0.75 / 1.0 / 1.05 PFLOP/s)
-// instead of 77.7 / 44.9 / 257 / 132 us in 64-row tiles of gemm_kernel.
+// instead of 77.7 / 44.9 / 257 / 132 us in 64-row tiles of gemm_kernel.  At 33 .. 64
+// rows (CT = 1) its gain is the deeper X ring and the single barrier per round; use_wide
+// has the figures.
 constexpr int kWideRing = 4;    // rounds of X in LDS and of W in registers
 template <int CT> constexpr int wide_kb() { return CT >= 3 ? 1 : 2; }   // k-blocks of a round
 
-template <int MT, int CT, bool WT>
-__global__ __launch_bounds__(256, 2) void gemm_wide_kernel(Args A, int units, int mtiles) {
+template <int MT, int CT, int W, bool WT>
+__global__ __launch_bounds__(64 * W, 2) void gemm_wide_kernel(Args A, int units, int mtiles) {
   constexpr int KB = wide_kb<CT>();
   constexpr int NC = KB * MT;             // 1 KB X chunks of a round
-  constexpr int XL = (NC + 3) / 4;        // chunks a wave requests per round (those past NC read nothing)
+  constexpr int XL = (NC + W - 1) / W;    // chunks a wave requests per round (those past NC read nothing)
   constexpr int WL = KB * CT;             // W loads of a wave per round
   constexpr int WKB = WT ? 1024 : 64;     // bytes between a lane's consecutive k-blocks of W
   static_assert(2 * (XL + WL) < 64 && kWideRing == 4 && 256 % (32 * KB * kWideRing) == 0, "vmcnt range");
@@ -441,13 +443,13 @@ __global__ __launch_bounds__(256, 2) void gemm_wide_kernel(Args A, int units, in
   const int unit = (blockIdx.x & 7) + 8 * (j / mtiles), mt = j % mtiles;
   if (unit >= units) return;
   const int s = unit % A.S, nt = unit / A.S;
-  const int col = nt * 64 * CT + 16 * CT * w;   // this wave's first column
+  const int col = 16 * CT * (nt * W + w);       // this wave's first column
   const int row0 = mt * 16 * MT;
   const int k0 = s * A.KC;
   const int nr = A.KC / (32 * KB);              // a multiple of kWideRing: KC % 256 == 0
   const int ncol = min(CT, (A.N - col + 15) / 16);   // column tiles of this wave inside N (may be <= 0)
 
-  // X: lane offset of the wave's chunk jj of a round: c = w + 4 jj, k-block
+  // X: lane offset of the wave's chunk jj of a round: c = w + W jj, k-block
   // c / MT, row tile c % MT.
   const int mrows = min(16 * MT, A.M - row0);
   const int t0 = row0 / 16;                      // first 16-row tile
@@ -458,7 +460,7 @@ __global__ __launch_bounds__(256, 2) void gemm_wide_kernel(Args A, int units, in
   int xo[XL];
 #pragma unroll
   for (int jj = 0; jj < XL; ++jj) {
-    const int c = w + 4 * jj, kb = c / MT, t = c % MT;
+    const int c = w + W * jj, kb = c / MT, t = c % MT;
     int o;
     if (A.x_tiled) {
       const int T = t0 + t;
@@ -495,7 +497,7 @@ __global__ __launch_bounds__(256, 2) void gemm_wide_kernel(Args A, int units, in
             u32x4, __builtin_amdgcn_raw_buffer_load_b128(rw, woff + c * wcol + WKB * (KB * rr + kb), 0, 0));
 #pragma unroll
     for (int jj = 0; jj < XL; ++jj) {
-      const int c = w + 4 * jj;
+      const int c = w + W * jj;
       x_dma16(rx, xo[jj] + xkb * KB * rr, xl + (c < NC ? slot * NC + c : kWideRing * NC) * 1024);
     }
     asm volatile("" ::: "memory");
@@ -875,24 +877,30 @@ static int reduce_launch(const gemm::Args& a, hipStream_t s) {
   return hipGetLastError() == hipSuccess ? RSPX_OK : RSPX_ELAUNCH;
 }
 
-// Column tiles per wave of gemm_wide_kernel and gemm_any_kernel, 4, 4 - step, ..:
-// the least time for the busiest CU, workgroups per CU times a workgroup's time for
-// its 16 ct columns per wave (tiles: row tiles times K chunks).  Narrower waves read
-// each X fragment for fewer MFMAs, so ct = 1 .. 4 cost 14 : 24 : 31 : 40 and not
+// Waves of a workgroup and 16-column tiles per wave, for gemm_wide_kernel and (any)
+// gemm_any_kernel: the least time for the busiest CU, workgroups per CU times a
+// workgroup's time (tiles: row tiles times K chunks).  Narrower waves read each X
+// fragment for fewer MFMAs, so 1 .. 4 column tiles cost 14 : 24 : 31 : 40 and not
 // 1 : 2 : 3 : 4 (512 rows, o projection [4096, 4096]: 33.1 / 27.5 / 32.6 / 23.0 us
-// at ct = 1 .. 4 with 4 / 2 / 2 / 1 workgroups per CU; 512 rows, gate/up
-// [24576, 4096]: 144.8 / 115.8 / 103.3 / 116.7 us with 6 / 3 / 2 / 2; 128 rows,
-// q/k/v [6144, 4096]: 20.1 / 16.5 / 19.3 / 22.2 us with 2 / 1 / 1 / 1; 512 rows,
-// [9976, 6596]: 216 / 259 / - / 192 us with 3 / 2 / - / 1).
-static int columns_per_wave(int N, int64_t tiles, int step) {
-  static const int cost[5] = {0, 14, 24, 31, 40};
-  int ct = 4;
-  int64_t best = 0;
-  for (int c = 4; c >= 1; c = c > step || c == 1 ? c - step : 1) {
-    const int64_t t = ((int64_t)((N + 64 * c - 1) / (64 * c)) * tiles + 255) / 256 * cost[c];
-    if (c == 4 || t < best) { ct = c; best = t; }
+// at 1 .. 4 with 4 / 2 / 2 / 1 workgroups per CU; 512 rows, gate/up [24576, 4096]:
+// 144.8 / 115.8 / 103.3 / 116.7 us with 6 / 3 / 2 / 2; 128 rows, q/k/v [6144, 4096]:
+// 20.1 / 16.5 / 19.3 / 22.2 us with 2 / 1 / 1 / 1; 512 rows, [9976, 6596]: 216 / 259
+// / - / 192 us with 3 / 2 / - / 1).  Six waves of one tile (96 columns, 22) fill the
+// chip with one workgroup per CU where 64 columns take two and 128 leave CUs idle:
+// gate/up at 64 rows 37.2 us instead of 47.0 (4 x 1) and 40.2 (4 x 2), at 128 rows 45.6
+// instead of 61.0 and 50.3.
+struct WaveTile { int waves, ct; };
+static WaveTile wave_tile(int N, int64_t tiles, bool any) {
+  static const struct { WaveTile t; int cost; } kTiles[] = {{{4, 4}, 40}, {{4, 3}, 31}, {{4, 2}, 24}, {{6, 1}, 22}, {{4, 1}, 14}};
+  WaveTile best{4, 4};
+  int64_t t_best = -1;
+  for (const auto& c : kTiles) {
+    if (any && (c.t.ct == 3 || c.t.waves == 6)) continue;
+    const int cols = 16 * c.t.waves * c.t.ct;
+    const int64_t t = ((int64_t)((N + cols - 1) / cols) * tiles + 255) / 256 * c.cost;
+    if (t_best < 0 || t < t_best) { best = c.t; t_best = t; }
   }
-  return ct;
+  return best;
 }
 
 // 31-bit byte offsets inside a 128-row tile of x and a wave's 64 rows of w.
@@ -901,29 +909,53 @@ static bool wide_fits(const gemm::Args& a) {
          (int64_t)a.K * 384 < (1ll << 30);
 }
 
-static int wide_launch(const gemm::Args& a, hipStream_t s) {
-  // Row tiles of at most 128 rows, all of the same height.
-  const int mtiles = (a.M + 127) / 128;
+// Whether gemm_wide_kernel runs the call.  Always above 64 rows.  For 33 .. 64 rows
+// where waves of one column tile make one workgroup for most CUs and its chunk has
+// eight rounds or more: q/k/v [6144, 4096], o [4096, 4096], gate/up [24576, 4096] and
+// down [4096, 12288] with tiled W at 64 rows 12.3 / 9.1 / 37.2 / 20.7 us instead of
+// 13.7 / 10.3 / 39.7 / 23.3 in gemm_kernel, at 48 rows 11.7 / 8.6 / 36.1 / 19.6
+// instead of 12.1 / 9.6 / 36.9 / 21.8, at 32 rows 11.4 / 8.3 / 35.7 / 19.0 and 11.2 /
+// 8.5 / 36.1 / 19.3.  gemm_kernel keeps more bytes of W in flight per wave, which
+// counts in short chunks and small grids ([4096, 1024], four rounds, 64 rows: 5.1
+// against 5.3; [1024, 3072], 64 workgroups, 48 rows: 5.9 / 6.1), and shares X between
+// 128 columns in large ones (vocabulary [151936, 4096]: 239 / 252).
+static bool use_wide(const gemm::Args& a, WaveTile t) {
+  if (!wide_fits(a) || a.M <= 32) return false;
+  if (a.M > gemm::kRows) return true;
+  const int cols = 16 * t.waves;
+  const int64_t wgs = (int64_t)((a.N + cols - 1) / cols) * a.S;
+  return t.ct == 1 && a.KC >= 512 && wgs > 128 && wgs <= 256;
+}
+
+static int wide_launch(const gemm::Args& a, WaveTile wt, int mtiles, hipStream_t s) {
   const int mt = ((a.M + mtiles - 1) / mtiles + 15) / 16;
-  const int ct = columns_per_wave(a.N, a.S * mtiles, 1);
-  const int64_t units = (int64_t)((a.N + 64 * ct - 1) / (64 * ct)) * a.S;
+  const int cols = 16 * wt.waves * wt.ct;
+  const int64_t units = (int64_t)((a.N + cols - 1) / cols) * a.S;
   const int64_t wgs = (units + 7) / 8 * 8 * mtiles;
   if (wgs > 0x7fffffff) return RSPX_EUNSUPPORTED;
-  const dim3 g((unsigned)wgs), b(256);
-#define RSPX_WIDE(MTV, CTV)                                                                                        \
+  const dim3 g((unsigned)wgs), b(64 * wt.waves);
+#define RSPX_WIDE(MTV, CTV, WV)                                                                                    \
   if (a.sw == kTiled)                                                                                              \
-    hipLaunchKernelGGL((gemm::gemm_wide_kernel<MTV, CTV, true>), g, b, 0, s, a, (int)units, mtiles);               \
-  else hipLaunchKernelGGL((gemm::gemm_wide_kernel<MTV, CTV, false>), g, b, 0, s, a, (int)units, mtiles);
+    hipLaunchKernelGGL((gemm::gemm_wide_kernel<MTV, CTV, WV, true>), g, b, 0, s, a, (int)units, mtiles);           \
+  else hipLaunchKernelGGL((gemm::gemm_wide_kernel<MTV, CTV, WV, false>), g, b, 0, s, a, (int)units, mtiles);
+#define RSPX_WIDE_1(MTV)                                 \
+  if (wt.waves == 6) { RSPX_WIDE(MTV, 1, 6) }            \
+  else { RSPX_WIDE(MTV, 1, 4) }
 #define RSPX_WIDE_CT(MTV)                                \
-  if (ct == 4) { RSPX_WIDE(MTV, 4) }                     \
-  else if (ct == 3) { RSPX_WIDE(MTV, 3) }                \
-  else if (ct == 2) { RSPX_WIDE(MTV, 2) }                \
-  else { RSPX_WIDE(MTV, 1) }
-  if (mt == 8) { RSPX_WIDE_CT(8) }
-  else if (mt == 7) { RSPX_WIDE_CT(7) }
-  else if (mt == 6) { RSPX_WIDE_CT(6) }
-  else { RSPX_WIDE_CT(5) }
+  if (wt.ct == 4) { RSPX_WIDE(MTV, 4, 4) }               \
+  else if (wt.ct == 3) { RSPX_WIDE(MTV, 3, 4) }          \
+  else if (wt.ct == 2) { RSPX_WIDE(MTV, 2, 4) }          \
+  else { RSPX_WIDE_1(MTV) }
+  switch (mt) {
+    case 8: RSPX_WIDE_CT(8) break;
+    case 7: RSPX_WIDE_CT(7) break;
+    case 6: RSPX_WIDE_CT(6) break;
+    case 5: RSPX_WIDE_CT(5) break;
+    case 4: RSPX_WIDE_1(4) break;   // at most 64 rows: use_wide's one-tile waves
+    default: RSPX_WIDE_1(3) break;
+  }
 #undef RSPX_WIDE_CT
+#undef RSPX_WIDE_1
 #undef RSPX_WIDE
   return reduce_launch(a, s);
 }
@@ -942,7 +974,10 @@ static int linear_launch(const void* x, int64_t sx, const void* w, int64_t sw, v
   a.out_tiled = silu && so == kTiled;
   const int MTILES = (M + gemm::kRows - 1) / gemm::kRows;
   if (MTILES > 65535) return RSPX_EUNSUPPORTED;
-  if (M > gemm::kRows && wide_fits(a)) return wide_launch(a, s);
+  // gemm_wide_kernel: row tiles of at most 128 rows, all of the same height.
+  const int mtiles = (M + 127) / 128;
+  const WaveTile wt = wave_tile(N, (int64_t)S * mtiles, false);
+  if (use_wide(a, wt)) return wide_launch(a, wt, mtiles, s);
   // 8 waves (128 columns) share each X round between twice the columns; worth
   // it while the grid keeps >= 192 workgroups, and for the widest layers
   // (the vocabulary head) only when the X block is large (many rows).
@@ -1035,11 +1070,11 @@ static int linear_any(const void* x, int64_t sx, const void* w, int64_t sw, void
     return hipGetLastError() == hipSuccess ? RSPX_OK : RSPX_ELAUNCH;
   }
   // Row tiles of 1, 2, 4, 6 or 8 16-row tiles and 1, 2 or 4 column tiles a wave
-  // (columns_per_wave); where that leaves CUs without a workgroup, lower row tiles
+  // (wave_tile); where that leaves CUs without a workgroup, lower row tiles
   // while the grid stays within one workgroup per CU (77 x 4864 x 896: 12.1 -> 8.0
   // us, 64 x 5000 x 2600: 25.9 -> 18.3; up to two per CU: 10.7, 26.6).
   const int mtiles = (M + 127) / 128, rows = (M + mtiles - 1) / mtiles;
-  const int ct = columns_per_wave(N, mtiles, 2);
+  const int ct = wave_tile(N, mtiles, true).ct;
   const int64_t units = (N + 64 * ct - 1) / (64 * ct);
   int mt = rows <= 16 ? 1 : rows <= 32 ? 2 : rows <= 64 ? 4 : rows <= 96 ? 6 : 8;
   auto row_tiles = [&](int t) { return (M + 16 * t - 1) / (16 * t); };

@@ -422,10 +422,12 @@ def test_linear_silu_tiled_w(M):
 
 @pytest.mark.parametrize("M,N,K", [(65, 16, 256), (80, 272, 512), (81, 64, 256), (96, 4112, 256), (112, 1040, 768),
                                    (113, 4096, 1024), (127, 12304, 512), (128, 6144, 256), (129, 528, 1280),
-                                   (257, 8208, 256), (513, 4096, 512)])
+                                   (257, 8208, 256), (513, 4096, 512),
+                                   (33, 16416, 512), (48, 4000, 2048), (49, 20512, 512), (64, 6128, 2048),
+                                   (97, 24560, 256)])   # 33 .. 64 rows: one column tile per wave; 6 waves
 def test_linear_many_rows(M, N, K):
-    """More than 64 rows (row tiles of 80 .. 128 rows, 1 .. 4 column tiles per wave, ragged last
-    tiles): the bits of 64-row calls from row-major and tiled operands, in bf16, fp32, chunk
+    """More than 32 rows (row tiles of 48 .. 128 rows, 1 .. 4 column tiles per wave, ragged last
+    tiles): the bits of 32-row calls from row-major and tiled operands, in bf16, fp32, chunk
     partials and the SwiGLU epilogue, and the parity bound of test_linear_parity_bf16."""
     from _tiled import to_tiled
     from respect_amd import _lib
@@ -435,7 +437,7 @@ def test_linear_many_rows(M, N, K):
     xd, wd = _dev(x), _dev(w)
     wt = tile_weight(wd)
     for dt in (torch.bfloat16, torch.float32):
-        ref = torch.cat([linear(xd[i:i + 64], wd, out_dtype=dt) for i in range(0, M, 64)])
+        ref = torch.cat([linear(xd[i:i + 32], wd, out_dtype=dt) for i in range(0, M, 32)])
         assert torch.equal(linear(xd, wd, out_dtype=dt), ref)
         assert torch.equal(linear(xd, wt, out_dtype=dt), ref)
     ex = G.linear_exact(x, w)
@@ -459,7 +461,7 @@ def test_linear_many_rows(M, N, K):
             _lib.check("rspx_linear_silu", L.rspx_linear_silu(xa.data_ptr(), K, wt.data_ptr(), T, o.data_ptr(),
                                                               N // 2, m1 - m0, N, K, s))
             return o
-        assert torch.equal(silu(0, M), torch.cat([silu(i, min(M, i + 64)) for i in range(0, M, 64)]))
+        assert torch.equal(silu(0, M), torch.cat([silu(i, min(M, i + 32)) for i in range(0, M, 32)]))
 
 
 @pytest.mark.parametrize("M,N,K", [(1, 1, 1), (5, 40, 7), (17, 30, 8), (1, 65, 9), (16, 64, 63), (33, 129, 64),
