@@ -1,4 +1,5 @@
-"""ctypes binding of ``librespect_amd.so`` (the C ABI declared in include/respect_amd.h).
+"""ctypes binding of ``librespect_amd.so`` (the C ABI declared in include/respect_amd.h),
+and ``calls()``, the native form of the wrappers' common case (csrc/calls.cpp).
 
 torch is imported before the library is opened: the library then binds to the
 HIP runtime torch already loaded (same SONAME), so torch's streams and device
@@ -113,6 +114,20 @@ def lib() -> ctypes.CDLL:
     return _lib
 
 
+_calls = None
+
+
+def calls():
+    """The extension module ``_calls`` built beside the library; its functions return None
+    for a call that they leave to the Python wrapper."""
+    global _calls
+    if _calls is None:
+        lib()   # the library itself, with its message if it is not built
+        from . import _calls as mod
+        _calls = mod
+    return _calls
+
+
 def strerror(code: int) -> str:
     return lib().rspx_strerror(code).decode()
 
@@ -120,6 +135,13 @@ def strerror(code: int) -> str:
 def check(fn: str, code: int) -> None:
     if code != 0:
         raise RspxError(fn, code)
+
+
+def result(fn: str, y):
+    """What a function of ``calls()`` returned, unless that is a status: then raise it."""
+    if y.__class__ is int:
+        check(fn, y)
+    return y
 
 
 def stream_ptr(device: torch.device) -> int:

@@ -51,6 +51,33 @@ def sources() -> list[Path]:
 
 
 TRACE_LIB = PKG / "librespect_amd_trace.so"
+CALLS_SRC = CSRC / "calls.cpp"
+CALLS_LIB = PKG / "_calls.so"
+
+
+def build_calls(verbose: bool = False) -> Path:
+    """Compile ``csrc/calls.cpp`` (host code: torch tensors to C-ABI calls) into the
+    extension module ``_calls.so`` beside the library it calls."""
+    import sysconfig
+    from torch.utils import cpp_extension as ext
+    cxx = shutil.which("g++") or "g++"
+    tmp = CALLS_LIB.with_suffix(".so.tmp")
+    rocm = Path(hipcc()).resolve().parent.parent
+    cmd = [cxx, "-O2", "-std=c++17", "-fPIC", "-shared", "-w", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM", "-I", str(INCLUDE),
+           "-isystem", str(rocm / "include")]
+    for p in [*ext.include_paths(), sysconfig.get_paths()["include"]]:
+        cmd += ["-isystem", p]
+    cmd += [str(CALLS_SRC), "-o", str(tmp), "-L", str(PKG), f"-l:{LIB.name}", "-Wl,-rpath,$ORIGIN"]
+    for p in ext.library_paths():
+        cmd += ["-L", p]
+    cmd += ["-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python"]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError("g++ failed on calls.cpp:\n" + r.stdout + r.stderr)
+    os.replace(tmp, CALLS_LIB)
+    return CALLS_LIB
 
 
 def build(verbose: bool = False, jobs: int = 8, trace: bool = False) -> Path:
@@ -112,4 +139,5 @@ if __name__ == "__main__":
         print(build(verbose="-v" in sys.argv, trace=True))
     else:
         print(build(verbose="-v" in sys.argv))
+        print(build_calls(verbose="-v" in sys.argv))
         print(build_bench_floor(verbose="-v" in sys.argv))

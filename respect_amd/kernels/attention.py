@@ -30,6 +30,10 @@ def trie_attn(q, kp, vp, kn, vn, msk, sm_scale=None, out=None, rows_per_wave: in
     a per-stream scratch buffer).  ``out_tiled``: ``out`` is a flat bf16 buffer
     of at least ceil(M / 64) 64 H D elements that receives the [M, H D] result
     in the tiled activation layout (RSPX_TILED) instead of [H, M, D]."""
+    if out is None and workspace is None and rows_per_wave == 0 and launches == 0 and not out_tiled:
+        y = _lib.calls().trie_attn(q, kp, vp, kn, vn, msk, sm_scale, _lib._WORKSPACES, "attn")
+        if y is not None:
+            return _lib.result("rspx_trie_attn", y)
     H, M, D = q.shape
     HK, P, D2 = kp.shape
     NN = kn.shape[1]

@@ -66,6 +66,13 @@ def tile_weight(w: torch.Tensor) -> TiledWeight:
 def linear(x, w, BM=32, BN=128, BK=64, num_warps=4, num_stages=2, out_dtype=None, out=None, workspace=None):
     """x (M, K) @ w (N, K)^T -> (M, N). Bias is handled by the caller.  ``workspace``:
     optional uint8 GPU tensor of at least rspx_linear_workspace_bytes bytes."""
+    if out is None and workspace is None and (out_dtype is None or out_dtype in (torch.bfloat16, torch.float32)):
+        tiled = w.__class__ is TiledWeight
+        N, K = w.shape if tiled else (0, 0)
+        y = _lib.calls().linear(x, w.buf if tiled else w, N, K, tiled, out_dtype is torch.float32, _lib._WORKSPACES,
+                                "linear")
+        if y is not None:
+            return _lib.result("rspx_linear", y)
     if x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16:
         raise TypeError("linear: bf16 x and w are required")
     out_dtype = out_dtype or x.dtype

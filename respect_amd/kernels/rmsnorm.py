@@ -16,6 +16,9 @@ from ._tensor import as_kernel_input
 
 def rmsnorm(x, w, eps):
     """x [..., N] bf16, w [N] bf16 -> bf16 tensor shaped like x."""
+    y = _lib.calls().rmsnorm(x, w, eps)
+    if y is not None:
+        return _lib.result("rspx_rmsnorm", y)
     shape = x.shape
     N = shape[-1]
     if w.numel() != N:

@@ -17,6 +17,9 @@ from ..kernels._tensor import as_kernel_input
 
 def rope(x, cos, sin):
     """q*cos + rotate_half(q)*sin.  x [B,H,L,D], cos/sin [B,L,D] -> [B,H,L,D] bf16."""
+    y = _lib.calls().rope(x, cos, sin)
+    if y is not None:
+        return _lib.result("rspx_rope", y)
     if x.dtype != torch.bfloat16 or cos.dtype != torch.bfloat16 or sin.dtype != torch.bfloat16:
         raise TypeError("rope: respect_amd builds the bf16 path only")
     B, H, L, D = x.shape
@@ -35,6 +38,9 @@ def rope(x, cos, sin):
 
 def silu_mul(g, u):
     """silu(g) * u for bf16 tensors of the same shape (views into a packed gate/up are fine)."""
+    y = _lib.calls().silu_mul(g, u)
+    if y is not None:
+        return _lib.result("rspx_silu_mul", y)
     if g.dtype != torch.bfloat16 or u.dtype != torch.bfloat16:
         raise TypeError("silu_mul: respect_amd builds the bf16 path only")
     if g.shape != u.shape:
@@ -68,6 +74,9 @@ def qk_norm_rope(q, k, wq, wk, eps, cos, sin):
     each token's position) -> (q_out [T, HQ, D], k_out [T, HK, D]).  Bitwise
     equal to ``rope(rmsnorm(q, wq, eps), ...)`` and the same for k.
     """
+    y = _lib.calls().qk_norm_rope(q, k, wq, wk, eps, cos, sin)
+    if y is not None:
+        return _lib.result("rspx_qk_norm_rope", y)
     T, HQ, D = q.shape
     HK = k.shape[1]
     q = as_kernel_input(q, "q")
@@ -93,6 +102,9 @@ def rmsnorm_qk_norm_rope(x, w, eps, q, k, wq, wk, qk_eps, cos, sin):
     launch -> (y, q_out, k_out), bitwise the two calls' results.  x [..., N] with N % 8 == 0
     and N <= 16384; the rest as qk_norm_rope.  No counterpart in the reference (two
     launches there): for a caller with both inputs ready."""
+    y = _lib.calls().rmsnorm_qk_norm_rope(x, w, eps, q, k, wq, wk, qk_eps, cos, sin)
+    if y is not None:
+        return _lib.result("rspx_rmsnorm_qk_norm_rope", y)
     N = x.shape[-1]
     if w.numel() != N:
         raise ValueError(f"rmsnorm_qk_norm_rope: w has {w.numel()} elements for rows of {N}")
@@ -154,6 +166,9 @@ def _square(xs):
 
 def add_sq(r, h):
     """x = r + h (bf16, rounded once) and x.float() ** 2; both [rows, n]."""
+    y = _lib.calls().add_sq(r, h)
+    if y is not None:
+        return _lib.result("rspx_add_sq", y)
     if r.shape != h.shape:
         raise ValueError("add_sq: r and h must have the same shape")
     rs, hs = _bf16_rows(r, "r"), _bf16_rows(h, "h")
@@ -174,6 +189,9 @@ def norm_from(xs, sq, w, eps):
     if not (sq.is_cuda and sq.device == xs.device) or tuple(sq.shape) != (M, N) or tuple(w.shape) != (N,):
         raise ValueError("norm_from: sq must be [M, N] and w [N], on the device of xs")
     var = sq.mean(-1).contiguous()
+    y = _lib.calls().norm_apply(xs, var, w, eps)
+    if y is not None:
+        return _lib.result("rspx_norm_apply", y)
     xs = as_kernel_input(xs.contiguous(), "xs")
     w = as_kernel_input(w.contiguous(), "w")
     y = torch.empty((M, N), device=xs.device, dtype=torch.bfloat16)
@@ -192,6 +210,9 @@ def rmsnorm(x, w, eps):
 def rope_vision(x, cos, sin):
     """One tensor of apply_rotary_pos_emb_vision: x [L, NH, D] bf16, cos/sin [L, D];
     computed in float32, returned in bf16."""
+    y = _lib.calls().rope_vision(x, cos, sin)
+    if y is not None:
+        return _lib.result("rspx_rope_vision", y)
     if x.dtype != torch.bfloat16:
         raise TypeError("rope_vision: respect_amd builds the bf16 path only")
     L, NH, D = x.shape

@@ -1,0 +1,93 @@
+"""The native form of the wrappers' common case (respect_amd/_calls, csrc/calls.cpp): which
+calls it takes, and that it and the Python wrappers' own path give the same results."""
+import pytest
+import torch
+
+
+def test_calls_leaves_what_it_does_not_take():
+    """CPU tensors, other dtypes, non-tensors and wrong argument counts come back as None, so
+    that the Python wrapper decides (on the CPU: no kernel is called)."""
+    from respect_amd import _lib
+    if not _lib.LIB_PATH.exists():
+        pytest.skip("librespect_amd.so not built")
+    c = _lib.calls()
+    x = torch.zeros(4, 16, dtype=torch.bfloat16)
+    assert c.silu_mul(x, x) is None and c.silu_mul(x) is None and c.silu_mul(1, "a") is None
+    assert c.rmsnorm(x, x[0], 1e-6) is None and c.rmsnorm(x.float(), x[0], 1e-6) is None
+    assert c.linear(x, x, 0, 0, False, False, {}, "linear") is None
+    assert c.trie_attn(x, x, x, x, x, x, None, {}, "attn") is None
+    assert c.rope(x, x, x) is None and c.add_sq(x, x) is None and c.rope_vision(x, x, x) is None
+    assert c.norm_apply(x, x, x, 1e-6) is None and c.qk_norm_rope(x, x, x, x, 1e-6, x, x) is None
+    assert c.rmsnorm_qk_norm_rope(x, x, 1e-6, x, x, x, x, 1e-6, x, x) is None
+
+
+@pytest.mark.gpu
+def test_calls_equal_the_wrappers_own_path(monkeypatch):
+    """Each wrapper with and without the native call: equal results, shapes and dtypes, for the
+    layouts the native call takes and for views, paddings and dtypes it leaves to Python."""
+    from respect_amd import _lib
+    from respect_amd.kernels.attention import fused_attn_hyb
+    from respect_amd.kernels.gemm import linear, tile_weight
+    from respect_amd.kernels.rmsnorm import rmsnorm
+    from respect_amd.system import fused as F
+
+    class Leave:
+        def __getattr__(self, name):
+            return lambda *a: None
+
+    g = torch.Generator(device="cuda")
+    g.manual_seed(1)
+
+    def r(*s, dtype=torch.bfloat16):
+        return torch.randn(*s, generator=g, device="cuda").to(dtype)
+
+    x, w, w2 = r(2, 5, 512), r(512), r(768, 512)
+    q, k, wq = r(7, 4, 128), r(7, 2, 128), r(128)
+    cos, sin = r(7, 128), r(7, 128)
+    gu = r(7, 2048)
+    kp, kn = r(2, 40, 64), r(2, 32, 64)
+    qa, msk = r(4, 9, 64), torch.ones(9, 32, dtype=torch.bool, device="cuda").tril()
+    xr = r(1, 9, 4, 128)
+    tw = tile_weight(w2)
+    fns = [
+        lambda: F.silu_mul(gu[:, :1024], gu[:, 1024:]),
+        lambda: F.silu_mul(gu[0, :1024], gu[0, 1024:]),
+        lambda: F.silu_mul(gu[:, 1:1001], gu[:, 1001:2001]),
+        lambda: rmsnorm(x, w, 1e-6),
+        lambda: rmsnorm(q[:, 1:3], wq, 1e-5),
+        lambda: rmsnorm(x[..., :500], w[:500], 1e-6),
+        lambda: F.qk_norm_rope(q, k, wq, wq, 1e-6, cos, sin),
+        lambda: F.rmsnorm_qk_norm_rope(x, w, 1e-6, q, k, wq, wq, 1e-5, cos, sin),
+        lambda: F.rmsnorm_qk_norm_rope(x, w, 1e-6, q, k, wq, wq, 1e-5, cos[:, None], sin[:, None]),
+        lambda: linear(x, w2),
+        lambda: linear(x, w2, out_dtype=torch.float32),
+        lambda: linear(x[0, 1:], tw),
+        lambda: linear(x[..., :100], w2[:, :100]),
+        lambda: linear(r(70, 512) * 0 + x[0, :1], torch.nn.Parameter(w2)),
+        lambda: fused_attn_hyb(qa, kp, kp, kn, kn, msk),
+        lambda: fused_attn_hyb(qa, kp, kp, kn, kn, msk.to(torch.uint8), 0.1),
+        lambda: fused_attn_hyb(qa, kp, kp, kn, kn, msk.to(torch.int32), 0.1),
+        lambda: F.rope(xr.transpose(1, 2), cos[None, :7].expand(1, 7, 128).repeat(1, 2, 1)[:, :9],
+                       sin[None, :7].repeat(1, 2, 1)[:, :9]),
+        lambda: F.add_sq(x[0], x[1]),
+        lambda: F.norm_from(x[0], x[0].float() ** 2, w, 1e-6),
+        lambda: F.rope_vision(q, cos.float(), sin.float()),
+        lambda: F.rope_vision(q, cos, sin),
+    ]
+    for i, fn in enumerate(fns):
+        print(f"[calls] {i}", flush=True)
+        a = fn()
+        with monkeypatch.context() as m:
+            m.setattr(_lib, "calls", lambda: Leave())
+            b = fn()
+        for u, v in zip(a if isinstance(a, tuple) else (a,), b if isinstance(b, tuple) else (b,)):
+            assert u.dtype == v.dtype and u.shape == v.shape and torch.equal(u, v), i
+    # errors are the wrappers' own
+    with pytest.raises(TypeError):
+        F.silu_mul(gu.float(), gu.float())
+    with pytest.raises(ValueError):
+        F.silu_mul(gu, gu[:, :1024])
+    with pytest.raises(TypeError):
+        linear(x.float(), w2)
+    with pytest.raises(ValueError):
+        fused_attn_hyb(qa, kp, kp, kn, kn, msk[:, :16])
