@@ -418,23 +418,31 @@ __global__ __launch_bounds__(64 * W) void gemm_kernel(Args A) {
 // (workgroups are dealt round-robin over the 8 XCDs), so its L2 reads the slice of
 // W from memory once for all row tiles.
 //
+// Row-major operands: an operand tile of 16 rows is 64 bytes of each, half a cache
+// line, and the loads of a round took twice the line requests of the tiled layouts.
+// With two k-blocks a round every load takes 8 rows of 128 bytes instead; x goes
+// to LDS in swizzled 16-byte pieces, w is put on its lanes by two DPP moves per
+// register pair.  x and w row-major, 128 rows: q/k/v 20.4 -> 16.7 us, o 17.4 -> 12.9,
+// gate/up 65.2 -> 51, down 46.9 -> 32.1 (tiled 15.6 / 11.9 / 45.8 / 27.1); 512 rows,
+// gate/up 177 -> 133.  Three column tiles then hold two rounds only (four would not
+// fit the registers): half as far ahead, but 132.6 instead of 176.0 us there, where a
+// CU has two workgroups; a lone one gains nothing with tiled w (160 rows, gate/up:
+// 65.6 us against 59.4), so it keeps the single k-block rounds.
+//
 // 512 rows, q/k/v [6144, 4096], o [4096, 4096], gate/up [24576, 4096] and down
-// [4096, 12288]: 35.6 / 23.0 / 103 / 49 us (0.72 / 0.75 / 1.0 / 1.05 PFLOP/s)
+// [4096, 12288], tiled: 35.6 / 23.0 / 103 / 49 us (0.72 / 0.75 / 1.0 / 1.05 PFLOP/s)
 // instead of 77.7 / 44.9 / 257 / 132 us in 64-row tiles of gemm_kernel.  At 33 .. 64
 // rows (CT = 1) its gain is the deeper X ring and the single barrier per round; use_wide
 // has the figures.
-constexpr int kWideRing = 4;    // rounds of X in LDS and of W in registers
-template <int CT> constexpr int wide_kb() { return CT >= 3 ? 1 : 2; }   // k-blocks of a round
-
-template <int MT, int CT, int W, bool WT>
+// KB: k-blocks of a round.  RING: rounds of X in LDS and of W in registers.
+template <int MT, int CT, int W, bool WT, int KB, int RING>
 __global__ __launch_bounds__(64 * W, 2) void gemm_wide_kernel(Args A, int units, int mtiles) {
-  constexpr int KB = wide_kb<CT>();
   constexpr int NC = KB * MT;             // 1 KB X chunks of a round
   constexpr int XL = (NC + W - 1) / W;    // chunks a wave requests per round (those past NC read nothing)
   constexpr int WL = KB * CT;             // W loads of a wave per round
   constexpr int WKB = WT ? 1024 : 64;     // bytes between a lane's consecutive k-blocks of W
-  static_assert(2 * (XL + WL) < 64 && kWideRing == 4 && 256 % (32 * KB * kWideRing) == 0, "vmcnt range");
-  __shared__ __attribute__((aligned(16))) char xs[(kWideRing * NC + 1) * 1024];   // the last KB takes chunks past NC
+  static_assert((RING - 2) * (XL + WL) < 64, "vmcnt range");
+  __shared__ __attribute__((aligned(16))) char xs[(RING * NC + 1) * 1024];   // the last KB takes chunks past NC
   const int lane = __lane_id();
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int n16 = lane & 15, g4 = lane >> 4;
@@ -446,11 +454,14 @@ __global__ __launch_bounds__(64 * W, 2) void gemm_wide_kernel(Args A, int units,
   const int col = 16 * CT * (nt * W + w);       // this wave's first column
   const int row0 = mt * 16 * MT;
   const int k0 = s * A.KC;
-  const int nr = A.KC / (32 * KB);              // a multiple of kWideRing: KC % 256 == 0
+  const int nr = A.KC / (32 * KB);              // a multiple of RING (the host checks it)
   const int ncol = min(CT, (A.N - col + 15) / 16);   // column tiles of this wave inside N (may be <= 0)
 
-  // X: lane offset of the wave's chunk jj of a round: c = w + W jj, k-block
-  // c / MT, row tile c % MT.
+  // X: lane offset of the wave's chunk jj of a round, c = w + W jj: of row tile t =
+  // c % MT the k-block kb = c / MT (tiled x: one operand tile), or, row-major x, the
+  // rows 8 kb .. + 7 over both k-blocks of the round, 128 bytes each, whose 16-byte
+  // pieces take XOR-swizzled places so that the fragment reads below hit all banks.
+  // It lands at KB of tile t: (t KB + kb) 1 KB.
   const int mrows = min(16 * MT, A.M - row0);
   const int t0 = row0 / 16;                      // first 16-row tile
   const __amdgpu_buffer_rsrc_t rx =
@@ -465,8 +476,10 @@ __global__ __launch_bounds__(64 * W, 2) void gemm_wide_kernel(Args A, int units,
     if (A.x_tiled) {
       const int T = t0 + t;
       o = (((T >> 2) - (t0 >> 2)) * (A.K >> 5) + (k0 >> 5) + kb) * 4096 + (T & 3) * 1024 + 16 * lane;
+    } else if constexpr (KB == 2) {
+      o = 2 * (16 * t + 8 * kb + (lane >> 3)) * (int)A.sx + 16 * ((lane & 7) ^ (4 * kb + g4));
     } else {
-      o = 2 * ((16 * t + n16) * (int)A.sx + 8 * g4) + 64 * kb;
+      o = 2 * ((16 * t + n16) * (int)A.sx + 8 * g4);
     }
     xo[jj] = c < NC && 16 * t < mrows ? o : kOOBRow;
   }
@@ -475,7 +488,11 @@ __global__ __launch_bounds__(64 * W, 2) void gemm_wide_kernel(Args A, int units,
                 ncol > 0 ? (int64_t)(ncol - 1) * (A.K * 32 + 2 * kWSlabPad) + A.KC * 32 : 0)
          : rsrc(A.w + (int64_t)(ncol > 0 ? col : 0) * A.sw + k0,
                 ncol > 0 ? 2 * ((int64_t)(16 * ncol - 1) * A.sw + A.KC) : 0);
-  const int woff = WT ? 16 * lane : 2 * (n16 * (int)A.sw + 8 * g4);
+  // Row-major w, two k-blocks a round: load j takes the rows 8 j .. + 7 over both,
+  // 128 bytes each; w_operands puts the pieces on their lanes.
+  constexpr bool WL2 = !WT && KB == 2;
+  const int woff = WT ? 16 * lane
+                   : WL2 ? 2 * (n16 & 7) * (int)A.sw + 16 * (4 * (n16 >> 3) + g4) : 2 * (n16 * (int)A.sw + 8 * g4);
   const int wcol = WT ? A.K * 32 + 2 * kWSlabPad : 32 * (int)A.sw;   // bytes between column tiles
 
   lds_char_t* xl = (lds_char_t*)xs;
@@ -484,9 +501,9 @@ __global__ __launch_bounds__(64 * W, 2) void gemm_wide_kernel(Args A, int units,
   for (int t = 0; t < MT; ++t)
 #pragma unroll
     for (int c = 0; c < CT; ++c) acc[t][c] = f32x4{0.f, 0.f, 0.f, 0.f};
-  u32x4 wf[kWideRing][KB][CT];
+  u32x4 wf[RING][KB][CT];
 
-  // Round rr's W into ring slot rr % 4, then its X chunks: with X issued last, a
+  // Round rr's W into ring slot rr % RING, then its X chunks: with X issued last, a
   // count that covers round rr's X covers its W too.
   auto issue = [&](int rr, u32x4 (&wr)[KB][CT], int slot) {
 #pragma unroll
@@ -494,22 +511,42 @@ __global__ __launch_bounds__(64 * W, 2) void gemm_wide_kernel(Args A, int units,
 #pragma unroll
       for (int kb = 0; kb < KB; ++kb)
         wr[kb][c] = __builtin_bit_cast(
-            u32x4, __builtin_amdgcn_raw_buffer_load_b128(rw, woff + c * wcol + WKB * (KB * rr + kb), 0, 0));
+            u32x4, __builtin_amdgcn_raw_buffer_load_b128(rw, woff + c * wcol + (WL2 ? 128 * rr + 16 * kb * (int)A.sw : WKB * (KB * rr + kb)), 0, 0));
 #pragma unroll
     for (int jj = 0; jj < XL; ++jj) {
       const int c = w + W * jj;
-      x_dma16(rx, xo[jj] + xkb * KB * rr, xl + (c < NC ? slot * NC + c : kWideRing * NC) * 1024);
+      x_dma16(rx, xo[jj] + xkb * KB * rr, xl + (c < NC ? slot * NC + (c % MT) * KB + c / MT : RING * NC) * 1024);
     }
     asm volatile("" ::: "memory");
   };
+  // Fragment (kb, t): lane (n16, g4) reads row n16, 16-byte piece 4 kb + g4.
+  int xr[KB];
+#pragma unroll
+  for (int kb = 0; kb < KB; ++kb)
+    xr[kb] = KB == 1 || A.x_tiled ? 1024 * kb + 16 * lane : 128 * n16 + 16 * ((4 * kb + g4) ^ (n16 >> 1));
+  // Loads j = 0, 1 of row-major w hold, on lane (n16, g4), row 8 j + n16 % 8, piece
+  // 4 (n16 / 8) + g4; operand kb takes row n16, piece 4 kb + g4: half of each 16
+  // lanes from its own register, half from the other's lane n16 + 8 (mod 16).
+  auto w_operands = [&](u32x4& w0, u32x4& w1) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int a = (int)w0[i], b = (int)w1[i];
+      w0[i] = (uint32_t)__builtin_amdgcn_update_dpp(a, b, 0x128, 0xf, 0xc, false);   // row_ror:8, lanes 8 .. 15
+      w1[i] = (uint32_t)__builtin_amdgcn_update_dpp(b, a, 0x128, 0xf, 0x3, false);   // row_ror:8, lanes 0 .. 7
+    }
+  };
   // The X fragments of a k-block are read two row tiles ahead of their MFMAs.
-  auto compute = [&](const u32x4 (&wr)[KB][CT], int slot) {
+  auto compute = [&](u32x4 (&wr)[KB][CT], int slot) {
+    if constexpr (WL2) {
+#pragma unroll
+      for (int c = 0; c < CT; ++c) w_operands(wr[0][c], wr[KB - 1][c]);
+    }
 #pragma unroll
     for (int kb = 0; kb < KB; ++kb) {
       u32x4 xf[MT];
 #pragma unroll
       for (int t = 0; t < MT; ++t)
-        xf[t] = *(const __attribute__((address_space(3))) u32x4*)(xl + (slot * NC + kb * MT + t) * 1024 + 16 * lane);
+        xf[t] = *(const __attribute__((address_space(3))) u32x4*)(xl + (slot * NC + t * KB) * 1024 + xr[kb]);
 #pragma unroll
       for (int t = 0; t < MT; ++t)
 #pragma unroll
@@ -526,31 +563,25 @@ __global__ __launch_bounds__(64 * W, 2) void gemm_wide_kernel(Args A, int units,
   };
   constexpr int PER = XL + WL;   // loads a wave issues per round
 #pragma unroll
-  for (int r = 0; r < kWideRing - 1; ++r) issue(r, wf[r], r);
+  for (int r = 0; r < RING - 1; ++r) issue(r, wf[r], r);
   int r = 0;
-  for (; r + kWideRing < nr; r += kWideRing) {
+  for (; r + RING < nr; r += RING) {
 #pragma unroll
-    for (int u = 0; u < kWideRing; ++u) {
-      RSPX_VMW(2 * PER);   // round r + u has landed (this wave's part)
+    for (int u = 0; u < RING; ++u) {
+      vm_wait_n((RING - 2) * PER);   // round r + u has landed (this wave's part)
       raw_barrier();       // every wave's part, and every wave is done with round r + u - 1
-      issue(r + u + kWideRing - 1, wf[(u + kWideRing - 1) % kWideRing], (u + kWideRing - 1) % kWideRing);
+      issue(r + u + RING - 1, wf[(u + RING - 1) % RING], (u + RING - 1) % RING);
       compute(wf[u], u);
     }
   }
-  // The last four rounds: one more to request.
-  RSPX_VMW(2 * PER);
-  raw_barrier();
-  issue(r + 3, wf[3], 3);
-  compute(wf[0], 0);
-  RSPX_VMW(2 * PER);
-  raw_barrier();
-  compute(wf[1], 1);
-  RSPX_VMW(PER);
-  raw_barrier();
-  compute(wf[2], 2);
-  RSPX_VMW(0);
-  raw_barrier();
-  compute(wf[3], 3);
+  // The last RING rounds: one more to request.
+#pragma unroll
+  for (int u = 0; u < RING; ++u) {
+    vm_wait_n((RING - 1 - (u > 0 ? u : 1)) * PER);
+    raw_barrier();
+    if (u == 0) issue(r + RING - 1, wf[RING - 1], RING - 1);
+    compute(wf[u], u);
+  }
 #pragma unroll
   for (int c = 0; c < CT; ++c)
     if (c < ncol)
@@ -877,7 +908,7 @@ static int reduce_launch(const gemm::Args& a, hipStream_t s) {
   return hipGetLastError() == hipSuccess ? RSPX_OK : RSPX_ELAUNCH;
 }
 
-// Waves of a workgroup and 16-column tiles per wave, for gemm_wide_kernel and (any)
+// Waves of a workgroup and 16-column tiles per wave, for gemm_wide_kernel and
 // gemm_any_kernel: the least time for the busiest CU, workgroups per CU times a
 // workgroup's time (tiles: row tiles times K chunks).  Narrower waves read each X
 // fragment for fewer MFMAs, so 1 .. 4 column tiles cost 14 : 24 : 31 : 40 and not
@@ -889,15 +920,24 @@ static int reduce_launch(const gemm::Args& a, hipStream_t s) {
 // chip with one workgroup per CU where 64 columns take two and 128 leave CUs idle:
 // gate/up at 64 rows 37.2 us instead of 47.0 (4 x 1) and 40.2 (4 x 2), at 128 rows 45.6
 // instead of 61.0 and 50.3.
+//
+// Row-major w costs more the more column tiles a wave has (4 do not fit its two
+// k-blocks a round, and two workgroups per CU hide its shallower ring), so there the
+// costs are 15 : 24 : 36 and 21 for six waves, a lone workgroup 1.2 of its share (512
+// rows, gate/up: 132.6 us at 4 x 3, 138.1 at 4 x 2, 153.4 at 6 x 1; 256 rows: 102.0 /
+// 94.9 / 84.6; 512 rows, o: 40.4 / 30.9 / 38.4, 36.1 at 4 x 1, 33.6 at 4 x 4).
 struct WaveTile { int waves, ct; };
-static WaveTile wave_tile(int N, int64_t tiles, bool any) {
-  static const struct { WaveTile t; int cost; } kTiles[] = {{{4, 4}, 40}, {{4, 3}, 31}, {{4, 2}, 24}, {{6, 1}, 22}, {{4, 1}, 14}};
-  WaveTile best{4, 4};
+enum class TileFor { kTiledW, kRowsW, kAny };
+static WaveTile wave_tile(int N, int64_t tiles, TileFor use) {
+  static const struct { WaveTile t; int cost, cost_rows; } kTiles[] = {
+      {{4, 4}, 40, 0}, {{4, 3}, 31, 36}, {{4, 2}, 24, 24}, {{6, 1}, 22, 21}, {{4, 1}, 14, 15}};
+  WaveTile best{4, 1};
   int64_t t_best = -1;
   for (const auto& c : kTiles) {
-    if (any && (c.t.ct == 3 || c.t.waves == 6)) continue;
+    if (use == TileFor::kAny ? c.t.ct == 3 || c.t.waves == 6 : use == TileFor::kRowsW && c.t.ct == 4) continue;
     const int cols = 16 * c.t.waves * c.t.ct;
-    const int64_t t = ((int64_t)((N + cols - 1) / cols) * tiles + 255) / 256 * c.cost;
+    const int64_t n = ((int64_t)((N + cols - 1) / cols) * tiles + 255) / 256;   // workgroups of the busiest CU
+    const int64_t t = use == TileFor::kRowsW ? (n > 1 ? 5 * n : 6) * c.cost_rows : n * c.cost;
     if (t_best < 0 || t < t_best) { best = c.t; t_best = t; }
   }
   return best;
@@ -909,53 +949,72 @@ static bool wide_fits(const gemm::Args& a) {
          (int64_t)a.K * 384 < (1ll << 30);
 }
 
-// Whether gemm_wide_kernel runs the call.  Always above 64 rows.  For 33 .. 64 rows
-// where waves of one column tile make one workgroup for most CUs and its chunk has
+// Whether gemm_wide_kernel runs the call.  Always above 64 rows, except that tiled
+// operands whose chunk is one round of gemm_kernel stay there while neither grid is
+// large ([4096, 1024]: 96 rows 5.3 us against 5.6, 128 rows 5.8 / 6.4; [576, 512],
+// 1024 rows 4.8 / 5.5; but [6144, 1024], 96 rows 8.7 / 7.5).  For 33 .. 64 rows where waves of one column tile make one workgroup for most CUs and its chunk has
 // eight rounds or more: q/k/v [6144, 4096], o [4096, 4096], gate/up [24576, 4096] and
-// down [4096, 12288] with tiled W at 64 rows 12.3 / 9.1 / 37.2 / 20.7 us instead of
+// down [4096, 12288], tiled, at 64 rows 12.3 / 9.1 / 37.2 / 20.7 us instead of
 // 13.7 / 10.3 / 39.7 / 23.3 in gemm_kernel, at 48 rows 11.7 / 8.6 / 36.1 / 19.6
 // instead of 12.1 / 9.6 / 36.9 / 21.8, at 32 rows 11.4 / 8.3 / 35.7 / 19.0 and 11.2 /
-// 8.5 / 36.1 / 19.3.  gemm_kernel keeps more bytes of W in flight per wave, which
-// counts in short chunks and small grids ([4096, 1024], four rounds, 64 rows: 5.1
-// against 5.3; [1024, 3072], 64 workgroups, 48 rows: 5.9 / 6.1), and shares X between
-// 128 columns in large ones (vocabulary [151936, 4096]: 239 / 252).
+// 8.5 / 36.1 / 19.3; row-major at 64 rows 13.1 / 9.8 / 44.5 / 25.4 instead of 16.3 /
+// 11.7 / 47.6 / 28.1.  Tiled x with row-major w is the slower one there (gate/up, 48
+// rows: 43.6 / 40.6).  gemm_kernel keeps more bytes of W in flight per wave, which
+// counts in short chunks and small grids ([4096, 1024], 64 rows: 5.1 against 5.3;
+// [1024, 3072], 64 workgroups, 48 rows: 5.9 / 6.1), and shares X between 128 columns
+// in large ones (vocabulary [151936, 4096]: 239 / 252).
 static bool use_wide(const gemm::Args& a, WaveTile t) {
   if (!wide_fits(a) || a.M <= 32) return false;
-  if (a.M > gemm::kRows) return true;
+  const bool w_tiled = a.sw == kTiled;
   const int cols = 16 * t.waves;
-  const int64_t wgs = (int64_t)((a.N + cols - 1) / cols) * a.S;
-  return t.ct == 1 && a.KC >= 512 && wgs > 128 && wgs <= 256;
+  const int64_t wgs = (int64_t)((a.N + cols - 1) / cols) * a.S;   // of one row tile
+  if (a.M > gemm::kRows) {
+    const bool one_round = a.KC == gemm::kRoundK && a.x_tiled && w_tiled;
+    return !(one_round && t.ct == 1 && t.waves == 4 && wgs * ((a.M + gemm::kRows - 1) / gemm::kRows) <= 512);
+  }
+  return t.ct == 1 && a.KC >= 512 && wgs > 128 && wgs <= 256 && (w_tiled || !a.x_tiled);
 }
 
 static int wide_launch(const gemm::Args& a, WaveTile wt, int mtiles, hipStream_t s) {
-  const int mt = ((a.M + mtiles - 1) / mtiles + 15) / 16;
   const int cols = 16 * wt.waves * wt.ct;
   const int64_t units = (int64_t)((a.N + cols - 1) / cols) * a.S;
+  // Lower row tiles while the grid stays within one workgroup per CU ([1024, 3072],
+  // tiled / row-major, 128 rows: 7.0 / 11.7 us in one tile, 4.7 / 6.1 in four).
+  if (wt.ct == 1 && units < 256) mtiles = max(mtiles, min((int)(256 / units), (a.M + 31) / 32));
+  const int mt = ((a.M + mtiles - 1) / mtiles + 15) / 16;
+  mtiles = (a.M + 16 * mt - 1) / (16 * mt);
   const int64_t wgs = (units + 7) / 8 * 8 * mtiles;
   if (wgs > 0x7fffffff) return RSPX_EUNSUPPORTED;
   const dim3 g((unsigned)wgs), b(64 * wt.waves);
-#define RSPX_WIDE(MTV, CTV, WV)                                                                                    \
-  if (a.sw == kTiled)                                                                                              \
-    hipLaunchKernelGGL((gemm::gemm_wide_kernel<MTV, CTV, WV, true>), g, b, 0, s, a, (int)units, mtiles);           \
-  else hipLaunchKernelGGL((gemm::gemm_wide_kernel<MTV, CTV, WV, false>), g, b, 0, s, a, (int)units, mtiles);
+  const bool w_tiled = a.sw == kTiled;
+#define RSPX_WIDE(MTV, CTV, WV, WTV, KBV, RV) \
+  hipLaunchKernelGGL((gemm::gemm_wide_kernel<MTV, CTV, WV, WTV, KBV, RV>), g, b, 0, s, a, (int)units, mtiles)
+#define RSPX_WIDE_12(MTV, CTV, WV)                  \
+  if (w_tiled) RSPX_WIDE(MTV, CTV, WV, true, 2, 4); \
+  else RSPX_WIDE(MTV, CTV, WV, false, 2, 4);
 #define RSPX_WIDE_1(MTV)                                 \
-  if (wt.waves == 6) { RSPX_WIDE(MTV, 1, 6) }            \
-  else { RSPX_WIDE(MTV, 1, 4) }
-#define RSPX_WIDE_CT(MTV)                                \
-  if (wt.ct == 4) { RSPX_WIDE(MTV, 4, 4) }               \
-  else if (wt.ct == 3) { RSPX_WIDE(MTV, 3, 4) }          \
-  else if (wt.ct == 2) { RSPX_WIDE(MTV, 2, 4) }          \
+  if (wt.waves == 6) { RSPX_WIDE_12(MTV, 1, 6) }         \
+  else { RSPX_WIDE_12(MTV, 1, 4) }
+#define RSPX_WIDE_CT(MTV)                                                      \
+  if (wt.ct == 4) RSPX_WIDE(MTV, 4, 4, true, 1, 4);   /* tiled w only */       \
+  else if (wt.ct == 3) {                                                       \
+    if (!w_tiled) RSPX_WIDE(MTV, 3, 4, false, 2, 2);                           \
+    else if (!a.x_tiled && wgs > 256) RSPX_WIDE(MTV, 3, 4, true, 2, 2);        \
+    else RSPX_WIDE(MTV, 3, 4, true, 1, 4);                                     \
+  } else if (wt.ct == 2) { RSPX_WIDE_12(MTV, 2, 4) }                           \
   else { RSPX_WIDE_1(MTV) }
   switch (mt) {
     case 8: RSPX_WIDE_CT(8) break;
     case 7: RSPX_WIDE_CT(7) break;
     case 6: RSPX_WIDE_CT(6) break;
     case 5: RSPX_WIDE_CT(5) break;
-    case 4: RSPX_WIDE_1(4) break;   // at most 64 rows: use_wide's one-tile waves
-    default: RSPX_WIDE_1(3) break;
+    case 4: RSPX_WIDE_1(4) break;   // one-tile waves: use_wide's rule, or lower row tiles
+    case 3: RSPX_WIDE_1(3) break;
+    default: RSPX_WIDE_1(2) break;
   }
 #undef RSPX_WIDE_CT
 #undef RSPX_WIDE_1
+#undef RSPX_WIDE_12
 #undef RSPX_WIDE
   return reduce_launch(a, s);
 }
@@ -976,7 +1035,7 @@ static int linear_launch(const void* x, int64_t sx, const void* w, int64_t sw, v
   if (MTILES > 65535) return RSPX_EUNSUPPORTED;
   // gemm_wide_kernel: row tiles of at most 128 rows, all of the same height.
   const int mtiles = (M + 127) / 128;
-  const WaveTile wt = wave_tile(N, (int64_t)S * mtiles, false);
+  const WaveTile wt = wave_tile(N, (int64_t)S * mtiles, sw == kTiled ? TileFor::kTiledW : TileFor::kRowsW);
   if (use_wide(a, wt)) return wide_launch(a, wt, mtiles, s);
   // 8 waves (128 columns) share each X round between twice the columns; worth
   // it while the grid keeps >= 192 workgroups, and for the widest layers
@@ -1074,7 +1133,7 @@ static int linear_any(const void* x, int64_t sx, const void* w, int64_t sw, void
   // while the grid stays within one workgroup per CU (77 x 4864 x 896: 12.1 -> 8.0
   // us, 64 x 5000 x 2600: 25.9 -> 18.3; up to two per CU: 10.7, 26.6).
   const int mtiles = (M + 127) / 128, rows = (M + mtiles - 1) / mtiles;
-  const int ct = wave_tile(N, mtiles, true).ct;
+  const int ct = wave_tile(N, mtiles, TileFor::kAny).ct;
   const int64_t units = (N + 64 * ct - 1) / (64 * ct);
   int mt = rows <= 16 ? 1 : rows <= 32 ? 2 : rows <= 64 ? 4 : rows <= 96 ? 6 : 8;
   auto row_tiles = [&](int t) { return (M + 16 * t - 1) / (16 * t); };

@@ -424,7 +424,9 @@ def test_linear_silu_tiled_w(M):
                                    (113, 4096, 1024), (127, 12304, 512), (128, 6144, 256), (129, 528, 1280),
                                    (257, 8208, 256), (513, 4096, 512),
                                    (33, 16416, 512), (48, 4000, 2048), (49, 20512, 512), (64, 6128, 2048),
-                                   (97, 24560, 256)])   # 33 .. 64 rows: one column tile per wave; 6 waves
+                                   (97, 24560, 256),    # 33 .. 64 rows: one column tile per wave; 6 waves
+                                   (130, 1040, 768), (100, 80, 1536),   # lower row tiles in a small grid
+                                   (140, 12304, 1024), (400, 12304, 512), (129, 24592, 512)])   # three tiles, two
 def test_linear_many_rows(M, N, K):
     """More than 32 rows (row tiles of 48 .. 128 rows, 1 .. 4 column tiles per wave, ragged last
     tiles): the bits of 32-row calls from row-major and tiled operands, in bf16, fp32, chunk
@@ -446,14 +448,17 @@ def test_linear_many_rows(M, N, K):
     L, s, T = _lib.lib(), _lib.stream_ptr(xd.device), _lib.RSPX_TILED
     xt = to_tiled(xd, fill=float("nan"))
     S = L.rspx_linear_splits(N, K)
-    parts = [torch.full((S, M, N), float("nan"), device="cuda") for _ in range(3)]
-    for p, xa, sx, wa in ((parts[0], xd, K, wd), (parts[1], xt, T, wd), (parts[2], xt, T, wt)):
+    parts = [torch.full((S, M, N), float("nan"), device="cuda") for _ in range(4)]
+    xw, ww = (torch.full((r, K + 24), float("nan"), device="cuda", dtype=torch.bfloat16) for r in (M, N))
+    xw[:, :K], ww[:, :K] = xd, wd          # rows apart, NaN between them
+    for p, xa, sx, wa in ((parts[0], xd, K, wd), (parts[1], xt, T, wd), (parts[2], xt, T, wt),
+                          (parts[3], xw, K + 24, ww)):
         _lib.check("rspx_linear_partials", L.rspx_linear_partials(xa.data_ptr(), sx, wa.data_ptr(), wa.stride(0),
                                                                   p.data_ptr(), M, N, K, s))
     acc = parts[0][0]
     for c in range(1, S):
         acc = acc + parts[0][c]
-    assert torch.equal(acc, ref) and torch.equal(parts[0], parts[1]) and torch.equal(parts[0], parts[2])
+    assert torch.equal(acc, ref) and all(torch.equal(parts[0], p) for p in parts[1:])
     if S == 1 and N % 32 == 0:
         def silu(m0, m1):
             o = torch.empty(m1 - m0, N // 2, device="cuda", dtype=torch.bfloat16)
