@@ -178,9 +178,11 @@ def bench_attn(args) -> dict:
     return res
 
 
-# One call is one fused_kernel launch when its grid fits on the device at once,
-# else prompt_kernel then node_merge_kernel.
-ATTN_KERNELS = ("rspx::fused_kernel", "rspx::prompt_kernel", "rspx::node_merge_kernel")
+# One call is one fused_kernel launch when its grid fits on the device at once
+# (fused_pair_kernel for up to twice that), else prompt_pair_kernel, then
+# node_block_kernel or node_merge_kernel (D = 256: fused2_kernel, prompt_kernel).
+ATTN_KERNELS = ("rspx::fused_kernel", "rspx::fused_pair_kernel", "rspx::fused2_kernel", "rspx::prompt_kernel",
+                "rspx::prompt_pair_kernel", "rspx::node_merge_kernel", "rspx::node_block_kernel")
 COPY_KERNEL = "__amd_rocclr_copyBuffer"
 PROBE_COPY_BYTES = 1 << 28   # the probe's device copy: 256 MiB read + 256 MiB written
 

@@ -101,9 +101,9 @@ const char* rspx_version(void);
  * NN <= 4096 (the node-slot limit of the reference dispatcher, NMAX).
  *
  * Launches: one (prompt groups, node partials and merge in one kernel whose
- * workgroups wait for each other; used when the grid, or half of it with two
- * row blocks per workgroup, fits on the device at once) or two (prompt
- * groups, then node partials and merge).  All give the same bits.
+ * workgroups wait for each other; used when the grid, or half of it with twice
+ * the rows per workgroup, fits on the device at once) or two (prompt groups,
+ * then node partials and merge).  All give the same bits.
  *
  * rows_per_wave: 0 = automatic (one 16-row tile per wave when that grid
  * fits on the device at once, e.g. 1-token calls; two otherwise), else 1 or
@@ -271,9 +271,9 @@ int rspx_silu_mul(const void* g, int64_t sg, const void* u, int64_t su, void* y,
  * 16-byte aligned; sx may be RSPX_TILED, and so may sw: w is then in the
  * tiled weight layout rspx_linear_tile_weight writes (same results, bit for
  * bit).  Any M, N, K (the reference's kernel masks every edge,
- * gemm.py:19-27): with N % 16 == 0 and K % 256 == 0 the streaming kernel
- * runs; any other (N, K) runs one bounded-load MFMA chain per output tile,
- * row-major operands only (RSPX_EUNSUPPORTED for RSPX_TILED), 2-byte
+ * gemm.py:19-27): with N % 16 == 0 and K % 256 == 0 the streaming
+ * kernels run; any other (N, K) runs one MFMA chain over bounded loads per
+ * output tile, row-major operands only (RSPX_EUNSUPPORTED for RSPX_TILED), 2-byte
  * alignment (4-byte for an fp32 out), row strides below 2^24 elements.
  *
  * Reduction order: K is cut into rspx_linear_splits(N, K) equal chunks (a

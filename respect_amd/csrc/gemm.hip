@@ -11,7 +11,8 @@
 //   ((c0 + c1) + c2) + ..., then rounded once to the output type.
 // So a row's output bits do not depend on how many rows the call carries.
 //
-// Work split: workgroup = (16 W output columns, chunk s, 64-row tile), W = 4,
+// Work split (gemm_kernel: few rows; gemm_wide_kernel takes calls of many, with
+// its own comment): workgroup = (16 W output columns, chunk s, 64-row tile), W = 4,
 // 6 or 8 waves of 16 columns each (the host picks W per shape for speed; the
 // chunk count S comes from 64-column tiles whatever W is, so W never changes
 // a bit of the result).  W -- the large operand, read exactly once -- goes
@@ -26,7 +27,8 @@
 // x may also come in the tiled layout (row stride RSPX_TILED, tiled_offset in
 // common.h): a 64-row block's k-block is then four 1 KB operand tiles, and
 // each direct-to-LDS load copies one whole tile instead of 16 rows x 64 B
-// (gate/up [64 x 4096] . [24576 x 4096]^T on MI355X: 46 instead of 53 us).
+// (gemm_kernel, gate/up [64 x 4096] . [24576 x 4096]^T on MI355X: 46 instead of 53
+// us; gemm_wide_kernel loads row-major x in whole lines: 37.2 and 37.3).
 // The LDS image, and so every result bit, is the same in both layouts.  The
 // SwiGLU epilogue can write its output tiled for the next layer.
 //
@@ -41,8 +43,8 @@
 // loads its MFMA A operand (row n % 16, k 8 g .. 8 g + 7) as 16 contiguous
 // bytes of one 1 KB tile.  The TCP (vector L1) then handles one 8 KB piece per
 // wave and round instead of 16 rows of 512 bytes on 16 pages (q/k/v, o,
-// gate/up, down at 64 rows: 14.1 / 10.4 / 40.2 / 23.4 us instead of 14.6 /
-// 11.1 / 42.0 / 24.6; one row 11.0 / 7.9 / 34.9 / 18.7 instead of 11.3 / 8.5 /
+// gate/up, down at 64 rows, tiled x: 12.3 / 9.1 / 37.2 / 20.7 us instead of 13.2 /
+// 9.9 / 43.6 / 24.2; one row 11.0 / 7.9 / 34.9 / 18.7 instead of 11.3 / 8.5 /
 // 34.4 / 19.5).  The same bits as the row-major W.
 
 #include "common.h"
