@@ -422,29 +422,33 @@ __global__ __launch_bounds__(64 * W) void gemm_kernel(Args A) {
 //
 // Row-major operands: an operand tile of 16 rows is 64 bytes of each, half a cache
 // line, and the loads of a round took twice the line requests of the tiled layouts.
-// With two k-blocks a round every load takes 8 rows of 128 bytes instead; x goes
-// to LDS in swizzled 16-byte pieces, w is put on its lanes by two DPP moves per
-// register pair.  x and w row-major, 128 rows: q/k/v 20.4 -> 16.7 us, o 17.4 -> 12.9,
-// gate/up 65.2 -> 51, down 46.9 -> 32.1 (tiled 15.6 / 11.9 / 45.8 / 27.1); 512 rows,
-// gate/up 177 -> 133.  Three column tiles then hold two rounds only (four would not
-// fit the registers): half as far ahead, but 132.6 instead of 176.0 us there, where a
-// CU has two workgroups; a lone one gains nothing with tiled w (160 rows, gate/up:
-// 65.6 us against 59.4), so it keeps the single k-block rounds.
+// Over pairs of k-blocks every load takes 8 rows of 128 bytes instead; x goes to LDS
+// in swizzled 16-byte pieces, w is put on its lanes by two DPP moves per register
+// pair.  x and w row-major, 128 rows: q/k/v 20.4 -> 16.7 us, o 17.4 -> 12.9, gate/up
+// 65.2 -> 51, down 46.9 -> 32.1 (tiled 15.6 / 11.9 / 45.8 / 27.1); 512 rows, gate/up
+// 177 -> 133.  Three column tiles of row-major w hold two rounds only (four would not
+// fit the registers): half as far ahead, but 132.6 instead of 176.0 us there.  With
+// tiled w three and four column tiles keep single k-block rounds of W beside pairs of
+// X: row-major x then costs nothing (512 rows, down 50.8 us against 51.9 tiled, 61.9
+// with half lines; 1024 rows, gate/up 184 against 178 and 223).
 //
 // 512 rows, q/k/v [6144, 4096], o [4096, 4096], gate/up [24576, 4096] and down
 // [4096, 12288], tiled: 35.6 / 23.0 / 103 / 49 us (0.72 / 0.75 / 1.0 / 1.05 PFLOP/s)
 // instead of 77.7 / 44.9 / 257 / 132 us in 64-row tiles of gemm_kernel.  At 33 .. 64
 // rows (CT = 1) its gain is the deeper X ring and the single barrier per round; use_wide
 // has the figures.
-// KB: k-blocks of a round.  RING: rounds of X in LDS and of W in registers.
+// KB: k-blocks of a round of W, RING: rounds of W in registers.  X comes in pairs of
+// k-blocks: one a round (KB = 2, RING of them in LDS), or one every other round (KB =
+// 1, four in LDS, one barrier per pair).
 template <int MT, int CT, int W, bool WT, int KB, int RING>
 __global__ __launch_bounds__(64 * W, 2) void gemm_wide_kernel(Args A, int units, int mtiles) {
-  constexpr int NC = KB * MT;             // 1 KB X chunks of a round
-  constexpr int XL = (NC + W - 1) / W;    // chunks a wave requests per round (those past NC read nothing)
+  constexpr int NC = 2 * MT;              // 1 KB X chunks of a pair
+  constexpr int XL = (NC + W - 1) / W;    // chunks a wave requests per pair (those past NC read nothing)
   constexpr int WL = KB * CT;             // W loads of a wave per round
   constexpr int WKB = WT ? 1024 : 64;     // bytes between a lane's consecutive k-blocks of W
-  static_assert((RING - 2) * (XL + WL) < 64, "vmcnt range");
-  __shared__ __attribute__((aligned(16))) char xs[(RING * NC + 1) * 1024];   // the last KB takes chunks past NC
+  constexpr int XRING = KB == 2 ? RING : 4;
+  static_assert((KB == 2 || RING == 4) && (RING - 2) * (XL + WL) < 64 && XL + 2 * WL < 64, "vmcnt range");
+  __shared__ __attribute__((aligned(16))) char xs[(XRING * NC + 1) * 1024];   // the last KB takes chunks past NC
   const int lane = __lane_id();
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int n16 = lane & 15, g4 = lane >> 4;
@@ -459,11 +463,11 @@ __global__ __launch_bounds__(64 * W, 2) void gemm_wide_kernel(Args A, int units,
   const int nr = A.KC / (32 * KB);              // a multiple of RING (the host checks it)
   const int ncol = min(CT, (A.N - col + 15) / 16);   // column tiles of this wave inside N (may be <= 0)
 
-  // X: lane offset of the wave's chunk jj of a round, c = w + W jj: of row tile t =
+  // X: lane offset of the wave's chunk jj of a pair, c = w + W jj: of row tile t =
   // c % MT the k-block kb = c / MT (tiled x: one operand tile), or, row-major x, the
-  // rows 8 kb .. + 7 over both k-blocks of the round, 128 bytes each, whose 16-byte
-  // pieces take XOR-swizzled places so that the fragment reads below hit all banks.
-  // It lands at KB of tile t: (t KB + kb) 1 KB.
+  // rows 8 kb .. + 7 over both k-blocks, 128 bytes each, whose 16-byte pieces take
+  // XOR-swizzled places so that the fragment reads below hit all banks.  It lands in
+  // the (2 t + kb)-th KB of the pair's slot.
   const int mrows = min(16 * MT, A.M - row0);
   const int t0 = row0 / 16;                      // first 16-row tile
   const __amdgpu_buffer_rsrc_t rx =
@@ -478,10 +482,8 @@ __global__ __launch_bounds__(64 * W, 2) void gemm_wide_kernel(Args A, int units,
     if (A.x_tiled) {
       const int T = t0 + t;
       o = (((T >> 2) - (t0 >> 2)) * (A.K >> 5) + (k0 >> 5) + kb) * 4096 + (T & 3) * 1024 + 16 * lane;
-    } else if constexpr (KB == 2) {
-      o = 2 * (16 * t + 8 * kb + (lane >> 3)) * (int)A.sx + 16 * ((lane & 7) ^ (4 * kb + g4));
     } else {
-      o = 2 * ((16 * t + n16) * (int)A.sx + 8 * g4);
+      o = 2 * (16 * t + 8 * kb + (lane >> 3)) * (int)A.sx + 16 * ((lane & 7) ^ (4 * kb + g4));
     }
     xo[jj] = c < NC && 16 * t < mrows ? o : kOOBRow;
   }
@@ -505,27 +507,29 @@ __global__ __launch_bounds__(64 * W, 2) void gemm_wide_kernel(Args A, int units,
     for (int c = 0; c < CT; ++c) acc[t][c] = f32x4{0.f, 0.f, 0.f, 0.f};
   u32x4 wf[RING][KB][CT];
 
-  // Round rr's W into ring slot rr % RING, then its X chunks: with X issued last, a
-  // count that covers round rr's X covers its W too.
-  auto issue = [&](int rr, u32x4 (&wr)[KB][CT], int slot) {
+  auto issue_w = [&](int rr, u32x4 (&wr)[KB][CT]) {
 #pragma unroll
     for (int c = 0; c < CT; ++c)
 #pragma unroll
       for (int kb = 0; kb < KB; ++kb)
         wr[kb][c] = __builtin_bit_cast(
-            u32x4, __builtin_amdgcn_raw_buffer_load_b128(rw, woff + c * wcol + (WL2 ? 128 * rr + 16 * kb * (int)A.sw : WKB * (KB * rr + kb)), 0, 0));
+            u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                       rw, woff + c * wcol + (WL2 ? 128 * rr + 16 * kb * (int)A.sw : WKB * (KB * rr + kb)), 0, 0));
+    asm volatile("" ::: "memory");
+  };
+  auto issue_x = [&](int pair, int slot) {
 #pragma unroll
     for (int jj = 0; jj < XL; ++jj) {
       const int c = w + W * jj;
-      x_dma16(rx, xo[jj] + xkb * KB * rr, xl + (c < NC ? slot * NC + (c % MT) * KB + c / MT : RING * NC) * 1024);
+      x_dma16(rx, xo[jj] + xkb * 2 * pair, xl + (c < NC ? slot * NC + (c % MT) * 2 + c / MT : XRING * NC) * 1024);
     }
     asm volatile("" ::: "memory");
   };
   // Fragment (kb, t): lane (n16, g4) reads row n16, 16-byte piece 4 kb + g4.
-  int xr[KB];
+  int xr[2];
 #pragma unroll
-  for (int kb = 0; kb < KB; ++kb)
-    xr[kb] = KB == 1 || A.x_tiled ? 1024 * kb + 16 * lane : 128 * n16 + 16 * ((4 * kb + g4) ^ (n16 >> 1));
+  for (int kb = 0; kb < 2; ++kb)
+    xr[kb] = A.x_tiled ? 1024 * kb + 16 * lane : 128 * n16 + 16 * ((4 * kb + g4) ^ (n16 >> 1));
   // Loads j = 0, 1 of row-major w hold, on lane (n16, g4), row 8 j + n16 % 8, piece
   // 4 (n16 / 8) + g4; operand kb takes row n16, piece 4 kb + g4: half of each 16
   // lanes from its own register, half from the other's lane n16 + 8 (mod 16).
@@ -538,7 +542,7 @@ __global__ __launch_bounds__(64 * W, 2) void gemm_wide_kernel(Args A, int units,
     }
   };
   // The X fragments of a k-block are read two row tiles ahead of their MFMAs.
-  auto compute = [&](u32x4 (&wr)[KB][CT], int slot) {
+  auto compute = [&](u32x4 (&wr)[KB][CT], int slot, int kb0) {
     if constexpr (WL2) {
 #pragma unroll
       for (int c = 0; c < CT; ++c) w_operands(wr[0][c], wr[KB - 1][c]);
@@ -548,7 +552,7 @@ __global__ __launch_bounds__(64 * W, 2) void gemm_wide_kernel(Args A, int units,
       u32x4 xf[MT];
 #pragma unroll
       for (int t = 0; t < MT; ++t)
-        xf[t] = *(const __attribute__((address_space(3))) u32x4*)(xl + (slot * NC + t * KB) * 1024 + xr[kb]);
+        xf[t] = *(const __attribute__((address_space(3))) u32x4*)(xl + (slot * NC + 2 * t) * 1024 + xr[kb0 + kb]);
 #pragma unroll
       for (int t = 0; t < MT; ++t)
 #pragma unroll
@@ -563,26 +567,67 @@ __global__ __launch_bounds__(64 * W, 2) void gemm_wide_kernel(Args A, int units,
       if (t + 3 < MT * KB) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
     }
   };
-  constexpr int PER = XL + WL;   // loads a wave issues per round
+  if constexpr (KB == 2) {
+    // Round rr's W into ring slot rr % RING, then its X: with X issued last, a count
+    // that covers round rr's X covers its W too.
+    auto issue = [&](int rr, int slot) {
+      issue_w(rr, wf[slot]);
+      issue_x(rr, slot);
+    };
+    constexpr int PER = XL + WL;   // loads a wave issues per round
 #pragma unroll
-  for (int r = 0; r < RING - 1; ++r) issue(r, wf[r], r);
-  int r = 0;
-  for (; r + RING < nr; r += RING) {
+    for (int r = 0; r < RING - 1; ++r) issue(r, r);
+    int r = 0;
+    for (; r + RING < nr; r += RING) {
+#pragma unroll
+      for (int u = 0; u < RING; ++u) {
+        vm_wait_n((RING - 2) * PER);   // round r + u has landed (this wave's part)
+        raw_barrier();       // every wave's part, and every wave is done with round r + u - 1
+        issue(r + u + RING - 1, (u + RING - 1) % RING);
+        compute(wf[u], u, 0);
+      }
+    }
+    // The last RING rounds: one more to request.
 #pragma unroll
     for (int u = 0; u < RING; ++u) {
-      vm_wait_n((RING - 2) * PER);   // round r + u has landed (this wave's part)
-      raw_barrier();       // every wave's part, and every wave is done with round r + u - 1
-      issue(r + u + RING - 1, wf[(u + RING - 1) % RING], (u + RING - 1) % RING);
-      compute(wf[u], u);
+      vm_wait_n((RING - 1 - (u > 0 ? u : 1)) * PER);
+      raw_barrier();
+      if (u == 0) issue(r + RING - 1, RING - 1);
+      compute(wf[u], u, 0);
     }
-  }
-  // The last RING rounds: one more to request.
+  } else {
+    // W three rounds ahead, X two pairs ahead.  Round r waits until what was issued
+    // after its W is all that is in flight: rounds r - 2 and r - 1 issued W, the even
+    // one of them X before it.  X of pair r / 2 is older than W of round r.
+    issue_x(0, 0);
+    issue_w(0, wf[0]);
+    issue_x(1, 1);
+    issue_w(1, wf[1]);
+    issue_w(2, wf[2]);
+    int r = 0;
+    for (; r + 8 < nr; r += 8) {
 #pragma unroll
-  for (int u = 0; u < RING; ++u) {
-    vm_wait_n((RING - 1 - (u > 0 ? u : 1)) * PER);
-    raw_barrier();
-    if (u == 0) issue(r + RING - 1, wf[RING - 1], RING - 1);
-    compute(wf[u], u);
+      for (int u = 0; u < 8; ++u) {
+        vm_wait_n(XL + 2 * WL);
+        if (u % 2 == 0) {
+          raw_barrier();   // every wave's part of the pair, and every wave is done with the pair before
+          issue_x((r + u) / 2 + 2, (u / 2 + 2) % 4);
+        }
+        issue_w(r + u + 3, wf[(u + 3) % 4]);
+        compute(wf[u % 4], u / 2, u % 2);
+      }
+    }
+    // The last eight rounds request up to their end.
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      vm_wait_n(u < 5 ? XL + 2 * WL : (7 - u) * WL);
+      if (u % 2 == 0) {
+        raw_barrier();
+        if (u + 4 < 8) issue_x((r + u) / 2 + 2, (u / 2 + 2) % 4);
+      }
+      if (u + 3 < 8) issue_w(r + u + 3, wf[(u + 3) % 4]);
+      compute(wf[u % 4], u / 2, u % 2);
+    }
   }
 #pragma unroll
   for (int c = 0; c < CT; ++c)
@@ -1001,7 +1046,6 @@ static int wide_launch(const gemm::Args& a, WaveTile wt, int mtiles, hipStream_t
   if (wt.ct == 4) RSPX_WIDE(MTV, 4, 4, true, 1, 4);   /* tiled w only */       \
   else if (wt.ct == 3) {                                                       \
     if (!w_tiled) RSPX_WIDE(MTV, 3, 4, false, 2, 2);                           \
-    else if (!a.x_tiled && wgs > 256) RSPX_WIDE(MTV, 3, 4, true, 2, 2);        \
     else RSPX_WIDE(MTV, 3, 4, true, 1, 4);                                     \
   } else if (wt.ct == 2) { RSPX_WIDE_12(MTV, 2, 4) }                           \
   else { RSPX_WIDE_1(MTV) }
