@@ -74,11 +74,19 @@ bool rows_of(const Tensor& t, int64_t& m, int64_t& n, int64_t& stride) {
 
 bool fits_int(int64_t v) { return v >= 0 && v <= 0x7fffffff; }
 
+// The C-ABI call without the GIL.  f also asks torch for pointers and the stream, which
+// may throw (a tensor without readable memory): the destructor takes the GIL back first.
+struct NoGil {
+  PyThreadState* state = PyEval_SaveThread();
+  NoGil() = default;
+  NoGil(const NoGil&) = delete;
+  ~NoGil() { PyEval_RestoreThread(state); }
+};
+
 template <class F>
 int call(F&& f) {
-  int rc;
-  Py_BEGIN_ALLOW_THREADS rc = f();
-  Py_END_ALLOW_THREADS return rc;
+  NoGil no_gil;
+  return f();
 }
 
 PyObject* wrap(Tensor&& t) { return THPVariable_Wrap(std::move(t)); }

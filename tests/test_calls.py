@@ -91,3 +91,28 @@ def test_calls_equal_the_wrappers_own_path(monkeypatch):
         linear(x.float(), w2)
     with pytest.raises(ValueError):
         fused_attn_hyb(qa, kp, kp, kn, kn, msk[:, :16])
+
+
+@pytest.mark.gpu
+def test_calls_raise_where_torch_refuses_the_memory():
+    """An output whose memory torch refuses to hand out (an allocation made under a dispatch
+    mode that fakes it) is an ordinary error from inside the native call, and the thread
+    holds the interpreter afterwards: later calls work."""
+    from torch.utils._python_dispatch import TorchDispatchMode
+    from respect_amd.kernels.gemm import linear
+    from respect_amd.system import fused as F
+
+    class NoMemory(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            r = func(*args, **(kwargs or {}))
+            if func is torch.ops.aten.empty.memory_format:
+                torch._C._set_throw_on_mutable_data_ptr(r)
+            return r
+
+    x, w = (torch.randn(n, 512, device="cuda").bfloat16() for n in (4, 2048))
+    want = F.silu_mul(x, x)
+    y = linear(x, w)
+    for fn in (lambda: F.silu_mul(x, x), lambda: linear(x, w)):
+        with pytest.raises(RuntimeError, match="data pointer"), NoMemory():
+            fn()
+    assert torch.equal(F.silu_mul(x, x), want) and torch.equal(linear(x, w), y)
