@@ -1384,7 +1384,10 @@ __device__ __forceinline__ void node_task(const TrieAttnArgs& A, int g, int p0, 
       vrow1 = st + rr1 * RB;
       vsw0 = vswz<D>(rr0);
       vsw1 = vswz<D>(rr1);
-      __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0): K fragments and this wave's stage rows
+      // vmcnt(0): K fragments and this wave's stage rows.  The wait is no memory barrier for
+      // the compiler, and the V reads below carry no wait of their own (lds_read_tr).
+      __builtin_amdgcn_s_waitcnt(0x0F70);
+      asm volatile("" ::: "memory");
       // Scores (the chain of node_scores: the same bits as the resident form).
 #pragma unroll
       for (int kb = 0; kb < 2; ++kb) {

@@ -393,21 +393,25 @@ def test_one_and_two_launches_equal(which):
     assert _status(c, ws) == 0
 
 
-@pytest.mark.parametrize("shape", ["8b", "d64"])
+@pytest.mark.parametrize("shape", ["8b", "d64", "d256"])
 def test_one_and_two_pass_node_segments_equal(shape):
     """The same trie and committed slots in a node segment of 128 and 192 slots (two and
     three chunks of K and V resident), of 256 slots (the extra slots masked out; V resident,
-    scores from K fragments loaded into registers), of 384 slots (streamed: a score pass
-    whose scores stay in LDS, then V gathered by rank) and of 1024 / 512 slots (streamed past
-    the kept-score limit: the scores recomputed from K gathered by rank) give the same
-    bits, through one and two launches."""
-    args = {"8b": (11, 32, 8, 128, 3072, 4, 24, 0, 16, 64), "d64": (7, 16, 2, 64, 3086, 3, 9, 0, 6, None)}[shape]
+    scores from K fragments loaded into registers), of 384 and 1024 slots (node_stream: the
+    scores stay in LDS, V in chunks, the ranks past the common run gathered) and of 1088 and
+    1536 slots (gathered: the scores recomputed from K, and V staged, by rank) give the same
+    bits, through one and two launches.  At head_dim 256 one chunk is resident and every
+    longer segment is gathered."""
+    args = {"8b": (11, 32, 8, 128, 3072, 4, 24, 0, 16, 64), "d64": (7, 16, 2, 64, 3086, 3, 9, 0, 6, None),
+            "d256": (19, 8, 2, 256, 700, 3, 9, 0, 6, None)}[shape]
     kw = {"kv_scale": 128 ** -0.5} if shape == "8b" else {}
-    base = 40 if shape == "8b" else 90
+    base = {"8b": 40, "d64": 90, "d256": 12}[shape]
     short = gen.attn_case(*args, base=base, **kw)
-    assert 64 < short.kn.shape[1] <= 128
+    lo, hi = (0, 64) if shape == "d256" else (64, 128)
+    assert lo < short.kn.shape[1] <= hi
     ref = _run(short, launches=2)
-    for step in (192, 256, 384, 1024 if shape == "8b" else 512):
+    for step in (192, 256, 384, 512, 1024, 1088, 1536):
+        print(f"[segments] {shape} NN={step}", flush=True)
         long = gen.attn_case(*args, base=base, nn_step=step, **kw)
         assert long.kn.shape[1] == step and np.array_equal(long.msk[:, :short.kn.shape[1]], short.msk)
         for launches in (1, 2):
