@@ -348,19 +348,20 @@ def _status(case, ws):
 
 
 @pytest.mark.parametrize("which", ["cfg1", "cfg2", "base37", "base100", "n64b40", "long", "gqa2", "d64",
-                                   "d64b90", "n128b70", "n72", "n100b30", "n192p512", "n256p512", "n512p256"])
+                                   "d64b90", "n128b70", "n72", "n100b30", "n192p512", "n256p512", "n512p256",
+                                   "d256", "d256m36"])
 def test_one_and_two_launches_equal(which):
     """The one-kernel path (prompt groups, node partials and merge with workgroups
     waiting on per-row-block counters) and the two-kernel path give the same
     bits; the counters are back at zero after each call (repeat calls on one
     workspace stay equal) and no wait ran out.  base100 / n64b40 / d64b90 put
     65-128 slots in the node segment (two chunks, loaded whole by both paths); long /
-    n128b70 have 512 rows per kv head, two row blocks per workgroup in one launch;
-    n72 / n100b30 (288 / 400 rows, 5 / 7 row blocks) leave the last workgroups of
-    that launch a single block.  n192p512 / n256p512 / n512p256 take the two-block
-    launch with 4 / 4 / 2 key groups, where each workgroup merges 2 x 64 / NG
-    consecutive rows of one block (a resident, a V-resident and a streamed node
-    segment; 32 and 64 merge rows need two and four node batches)."""
+    n128b70 have 512 rows per kv head, 128-row blocks in one launch; n72 / n100b30
+    (288 / 400 rows) leave the last of them partly empty.  n192p512 / n256p512 /
+    n512p256 take that launch with 4 / 4 / 2 key groups, where each workgroup merges
+    32 / 32 / 64 rows (a resident, a V-resident and a streamed node segment; two and
+    four node batches).  d256 / d256m36 have 8 and 5 32-row blocks at head_dim 256: two
+    blocks per workgroup, one after the other, the last workgroups of d256m36 one."""
     from respect_amd import _lib
     c = {"cfg1": gen.cfg1, "cfg2": gen.cfg2, "base37": lambda: gen.cfg2(seed=4, base=37),
          "base100": lambda: gen.cfg2(seed=4, base=100),
@@ -376,7 +377,9 @@ def test_one_and_two_launches_equal(which):
                                           base=30),
          "n192p512": lambda: gen.attn_case(16, 32, 8, 128, 512, 12, 16, 0, 0, 192, kv_scale=128 ** -0.5),
          "n256p512": lambda: gen.attn_case(17, 32, 8, 128, 512, 16, 16, 0, 0, 256, kv_scale=128 ** -0.5),
-         "n512p256": lambda: gen.attn_case(18, 32, 8, 128, 256, 16, 32, 0, 0, 512, kv_scale=128 ** -0.5)}[which]()
+         "n512p256": lambda: gen.attn_case(18, 32, 8, 128, 256, 16, 32, 0, 0, 512, kv_scale=128 ** -0.5),
+         "d256": lambda: gen.attn_case(9, 32, 8, 256, 3072, 4, 24, 0, 16, 64, kv_scale=256 ** -0.5),
+         "d256m36": lambda: gen.attn_case(20, 32, 8, 256, 3072, 3, 16, 0, 6, 36, kv_scale=256 ** -0.5)}[which]()
     print(f"[one/two launches] {which} NN={c.kn.shape[1]}", flush=True)
     H, M, D = c.q.shape
     HK, P, _ = c.kp.shape
@@ -388,7 +391,7 @@ def test_one_and_two_launches_equal(which):
     assert _status(c, ws) == 0
     for o in ones + [auto]:
         assert torch.equal(o, two)
-    for rpw in (1, 2):
+    for rpw in (1, 2) if D <= 128 else (1,):
         assert torch.equal(_run(c, launches=1, rows_per_wave=rpw, workspace=ws), two)
     assert _status(c, ws) == 0
 
@@ -436,7 +439,7 @@ def test_one_launch_workspace_shared_by_shapes():
     assert _status(cases[0], ws) == 0
 
 
-@pytest.mark.parametrize("which", ["cfg2", "cfg1", "n128", "one"])
+@pytest.mark.parametrize("which", ["cfg2", "cfg1", "n128", "one", "d256"])
 def test_wait_that_gives_up_poisons_its_rows(which):
     """One-launch path with the counter wait forced to give up at once (the spin limit
     lowered through the test hook, so every workgroup still exits normally): every row
@@ -446,10 +449,12 @@ def test_wait_that_gives_up_poisons_its_rows(which):
     counters were left at zero)."""
     from respect_amd import _lib
     c = {"cfg2": lambda: gen.cfg2(seed=6), "cfg1": gen.cfg1,
-         # 512 rows per kv head: two row blocks per workgroup in the one-launch path
+         # 512 rows per kv head: 128-row blocks in the one-launch path
          "n128": lambda: gen.attn_case(9, 32, 8, 128, 3072, 8, 32, 0, 32, 128, kv_scale=128 ** -0.5),
          # one query row (4 rows per kv head, one row tile per wave)
-         "one": lambda: gen.path_case(gen.cfg2(seed=6), 5)}[which]()
+         "one": lambda: gen.path_case(gen.cfg2(seed=6), 5),
+         # 8 32-row blocks of 8 kv heads and 8 key groups: two blocks per workgroup in one launch
+         "d256": lambda: gen.attn_case(9, 32, 8, 256, 3072, 4, 24, 0, 16, 64, kv_scale=256 ** -0.5)}[which]()
     H, M, D = c.q.shape
     HK, P, _ = c.kp.shape
     L = _lib.lib()

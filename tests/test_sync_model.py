@@ -1,6 +1,9 @@
 """Host-side model of the one-launch attention's cross-workgroup protocol
-(respect_amd/csrc/trie_attn.hip: count_partial, block_tail, fused_kernel,
-fused2_kernel), run on the CPU under many random schedules.
+(respect_amd/csrc/trie_attn.hip: count_partial, block_tail and the kernels that
+use them), run on the CPU under many random schedules.  fused_kernel and
+fused_pair_kernel (the same with 128-row blocks) follow it as it stands;
+fused2_kernel, which takes two row blocks per workgroup at head_dim 256, is the
+model's ``two``.
 
 Each workgroup (g, rb, q) of a row block of NG workgroups:
   0. reads the block's counter at its start (`old`, before its own add);
