@@ -65,7 +65,9 @@ extern "C" {
 /* Human-readable text for an RSPX_* code (static storage). */
 const char* rspx_strerror(int code);
 
-/* Library version, e.g. "respect_amd 0.1.0 gfx950". */
+/* Library version.  The last number goes up with every change of a signature in this
+ * header: code compiled against another one compares it before its first call. */
+#define RSPX_VERSION "respect_amd 0.1.0 gfx950 abi 1"
 const char* rspx_version(void);
 
 /* ---------------------------------------------------------------- attention

@@ -9,6 +9,7 @@ built, every kernel call raises.
 from __future__ import annotations
 
 import ctypes
+import warnings
 from pathlib import Path
 
 import torch  # noqa: F401  (loads the HIP runtime the library will share)
@@ -117,13 +118,32 @@ def lib() -> ctypes.CDLL:
 _calls = None
 
 
+class _NoCalls:
+    """Stands for ``_calls`` where only the library is built: every call is left to the wrapper."""
+
+    def __getattr__(self, name):
+        return lambda *args: None
+
+
 def calls():
     """The extension module ``_calls`` built beside the library; its functions return None
-    for a call that they leave to the Python wrapper."""
+    for a call that they leave to the Python wrapper.  Without the module every call is
+    (the same kernels, 10 to 20 us more host time each); one compiled for another version
+    of the library or of torch raises."""
     global _calls
     if _calls is None:
-        lib()   # the library itself, with its message if it is not built
-        from . import _calls as mod
+        version = lib().rspx_version().decode()   # the library itself, with its message if it is not built
+        try:
+            from . import _calls as mod
+        except ImportError as e:
+            warnings.warn(f"respect_amd._calls: {e}; kernel calls go through the slower Python wrappers until "
+                          "`python -m respect_amd.build` has built it", RuntimeWarning, stacklevel=2)
+            mod = _NoCalls()
+        else:
+            if mod.VERSION != version or mod.TORCH != torch.__version__.split("+")[0]:
+                raise RuntimeError(
+                    f"respect_amd._calls was built for {mod.VERSION!r} and torch {mod.TORCH}, but the library is "
+                    f"{version!r} and torch {torch.__version__}; run `python -m respect_amd.build`")
         _calls = mod
     return _calls
 

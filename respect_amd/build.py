@@ -2,7 +2,9 @@
 
 The library is one C-ABI ``.so`` (no torch types in any signature) compiled from
 every ``respect_amd/csrc/*.hip`` file.  It is written next to this file so that
-it travels with the source tree; ``python -m respect_amd.build`` rebuilds it.
+it travels with the source tree, and beside it the extension module ``_calls``
+(csrc/calls.cpp) for the Python and torch that run this; ``python -m
+respect_amd.build`` rebuilds both.
 """
 from __future__ import annotations
 
@@ -10,6 +12,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 import tempfile
 from pathlib import Path
 
@@ -52,13 +55,13 @@ def sources() -> list[Path]:
 
 TRACE_LIB = PKG / "librespect_amd_trace.so"
 CALLS_SRC = CSRC / "calls.cpp"
-CALLS_LIB = PKG / "_calls.so"
+# The interpreter's own suffix: another Python's build is not picked up.
+CALLS_LIB = PKG / ("_calls" + sysconfig.get_config_var("EXT_SUFFIX"))
 
 
 def build_calls(verbose: bool = False) -> Path:
     """Compile ``csrc/calls.cpp`` (host code: torch tensors to C-ABI calls) into the
-    extension module ``_calls.so`` beside the library it calls."""
-    import sysconfig
+    extension module ``_calls`` beside the library it calls."""
     from torch.utils import cpp_extension as ext
     cxx = shutil.which("g++") or "g++"
     tmp = CALLS_LIB.with_suffix(".so.tmp")
@@ -77,11 +80,13 @@ def build_calls(verbose: bool = False) -> Path:
     if r.returncode != 0:
         raise RuntimeError("g++ failed on calls.cpp:\n" + r.stdout + r.stderr)
     os.replace(tmp, CALLS_LIB)
+    (PKG / "_calls.so").unlink(missing_ok=True)   # the module's earlier name
     return CALLS_LIB
 
 
 def build(verbose: bool = False, jobs: int = 8, trace: bool = False) -> Path:
-    """Compile every kernel source and link ``librespect_amd.so`` (always rebuilds).
+    """Compile every kernel source and link ``librespect_amd.so``, then ``_calls`` against
+    it (always rebuilds).
     ``trace``: the measurement variant ``librespect_amd_trace.so`` instead, built with
     -DRSPX_PHASE_TRACE (the one-launch attention records per-wave phase timestamps,
     read back by rspx_trie_attn_phase_trace; ``bench.py --phase-trace``)."""
@@ -115,6 +120,8 @@ def build(verbose: bool = False, jobs: int = 8, trace: bool = False) -> Path:
         if r.returncode != 0:
             raise RuntimeError("link failed:\n" + r.stdout + r.stderr)
         os.replace(tmp, lib_out)
+    if not trace:
+        build_calls(verbose)
     return lib_out
 
 
@@ -139,5 +146,4 @@ if __name__ == "__main__":
         print(build(verbose="-v" in sys.argv, trace=True))
     else:
         print(build(verbose="-v" in sys.argv))
-        print(build_calls(verbose="-v" in sys.argv))
         print(build_bench_floor(verbose="-v" in sys.argv))

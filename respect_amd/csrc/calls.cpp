@@ -17,6 +17,7 @@
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/version.h>
 
 #include "respect_amd.h"
 
@@ -388,4 +389,12 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_calls", nullptr, -1, methods, nul
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__calls() { return PyModule_Create(&module); }
+// VERSION and TORCH: what the module was compiled against, for respect_amd._lib to compare.
+PyMODINIT_FUNC PyInit__calls() {
+  PyObject* m = PyModule_Create(&module);
+  if (m && (PyModule_AddStringConstant(m, "VERSION", RSPX_VERSION) || PyModule_AddStringConstant(m, "TORCH", TORCH_VERSION))) {
+    Py_DECREF(m);
+    return nullptr;
+  }
+  return m;
+}

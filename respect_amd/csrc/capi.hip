@@ -15,4 +15,4 @@ extern "C" const char* rspx_strerror(int code) {
   }
 }
 
-extern "C" const char* rspx_version(void) { return "respect_amd 0.1.0 gfx950"; }
+extern "C" const char* rspx_version(void) { return RSPX_VERSION; }

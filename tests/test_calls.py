@@ -21,6 +21,37 @@ def test_calls_leaves_what_it_does_not_take():
     assert c.rmsnorm_qk_norm_rope(x, x, 1e-6, x, x, x, x, 1e-6, x, x) is None
 
 
+def test_calls_missing_or_of_another_build(monkeypatch):
+    """Without the extension module the wrappers take their own path, with one warning; a module
+    compiled for another library or torch raises instead of being called."""
+    import sys
+    import types
+    import respect_amd
+    from respect_amd import _lib
+    from respect_amd.system import fused as F
+    if not _lib.LIB_PATH.exists():
+        pytest.skip("librespect_amd.so not built")
+    version, tv = _lib.lib().rspx_version().decode(), torch.__version__.split("+")[0]
+    x = torch.zeros(4, 16, dtype=torch.bfloat16)
+    with monkeypatch.context() as m:
+        m.setattr(_lib, "_calls", None)
+        m.delattr(respect_amd, "_calls", raising=False)
+        m.setitem(sys.modules, "respect_amd._calls", None)   # the import fails
+        with pytest.warns(RuntimeWarning, match="respect_amd.build"):
+            assert _lib.calls().silu_mul(x, x) is None
+        with pytest.raises(RuntimeError, match="GPU tensor"):
+            F.silu_mul(x, x)                                 # the wrapper's own checks
+    for v, t in ((version + "0", tv), (version, "1.0.0")):
+        with monkeypatch.context() as m:
+            mod = types.SimpleNamespace(VERSION=v, TORCH=t)
+            m.setattr(_lib, "_calls", None)
+            m.setattr(respect_amd, "_calls", mod, raising=False)
+            m.setitem(sys.modules, "respect_amd._calls", mod)
+            with pytest.raises(RuntimeError, match="respect_amd.build"):
+                _lib.calls()
+    assert _lib.calls().VERSION == version
+
+
 @pytest.mark.gpu
 def test_calls_equal_the_wrappers_own_path(monkeypatch):
     """Each wrapper with and without the native call: equal results, shapes and dtypes, for the
