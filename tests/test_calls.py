@@ -55,7 +55,8 @@ def test_calls_missing_or_of_another_build(monkeypatch):
 @pytest.mark.gpu
 def test_calls_equal_the_wrappers_own_path(monkeypatch):
     """Each wrapper with and without the native call: equal results, shapes and dtypes, for the
-    layouts the native call takes and for views, paddings and dtypes it leaves to Python."""
+    layouts the native call takes (it does take them) and for views, paddings and dtypes it
+    leaves to Python."""
     from respect_amd import _lib
     from respect_amd.kernels.attention import fused_attn_hyb
     from respect_amd.kernels.gemm import linear, tile_weight
@@ -80,39 +81,69 @@ def test_calls_equal_the_wrappers_own_path(monkeypatch):
     qa, msk = r(4, 9, 64), torch.ones(9, 32, dtype=torch.bool, device="cuda").tril()
     xr = r(1, 9, 4, 128)
     tw = tile_weight(w2)
-    fns = [
+    taken = [
         lambda: F.silu_mul(gu[:, :1024], gu[:, 1024:]),
         lambda: F.silu_mul(gu[0, :1024], gu[0, 1024:]),
-        lambda: F.silu_mul(gu[:, 1:1001], gu[:, 1001:2001]),
         lambda: rmsnorm(x, w, 1e-6),
-        lambda: rmsnorm(q[:, 1:3], wq, 1e-5),
-        lambda: rmsnorm(x[..., :500], w[:500], 1e-6),
         lambda: F.qk_norm_rope(q, k, wq, wq, 1e-6, cos, sin),
         lambda: F.rmsnorm_qk_norm_rope(x, w, 1e-6, q, k, wq, wq, 1e-5, cos, sin),
-        lambda: F.rmsnorm_qk_norm_rope(x, w, 1e-6, q, k, wq, wq, 1e-5, cos[:, None], sin[:, None]),
         lambda: linear(x, w2),
         lambda: linear(x, w2, out_dtype=torch.float32),
         lambda: linear(x[0, 1:], tw),
-        lambda: linear(x[..., :100], w2[:, :100]),
         lambda: linear(r(70, 512) * 0 + x[0, :1], torch.nn.Parameter(w2)),
         lambda: fused_attn_hyb(qa, kp, kp, kn, kn, msk),
         lambda: fused_attn_hyb(qa, kp, kp, kn, kn, msk.to(torch.uint8), 0.1),
-        lambda: fused_attn_hyb(qa, kp, kp, kn, kn, msk.to(torch.int32), 0.1),
         lambda: F.rope(xr.transpose(1, 2), cos[None, :7].expand(1, 7, 128).repeat(1, 2, 1)[:, :9],
                        sin[None, :7].repeat(1, 2, 1)[:, :9]),
         lambda: F.add_sq(x[0], x[1]),
         lambda: F.norm_from(x[0], x[0].float() ** 2, w, 1e-6),
         lambda: F.rope_vision(q, cos.float(), sin.float()),
+    ]
+    left = [   # a copy, a dtype or a shape that the wrapper makes or converts
+        lambda: F.silu_mul(gu[:, 1:1001], gu[:, 1001:2001]),
+        lambda: rmsnorm(q[:, 1:3], wq, 1e-5),
+        lambda: rmsnorm(x[..., :500], w[:500], 1e-6),
+        lambda: F.rmsnorm_qk_norm_rope(x, w, 1e-6, q, k, wq, wq, 1e-5, cos[:, None], sin[:, None]),
+        lambda: linear(x[..., :100], w2[:, :100]),
+        lambda: fused_attn_hyb(qa, kp, kp, kn, kn, msk.to(torch.int32), 0.1),
         lambda: F.rope_vision(q, cos, sin),
     ]
-    for i, fn in enumerate(fns):
+    native = _lib.calls()
+    answers = []
+
+    class Record:
+        def __getattr__(self, name):
+            def call(*a):
+                answers.append(getattr(native, name)(*a))
+                return answers[-1]
+            return call
+
+    def taken_by(fn):
+        answers.clear()
+        with monkeypatch.context() as m:
+            m.setattr(_lib, "calls", lambda: Record())
+            y = fn()
+        assert len(answers) == 1
+        return answers[0] is not None, y
+
+    for i, fn in enumerate(taken + left):
         print(f"[calls] {i}", flush=True)
-        a = fn()
+        fn()                       # the stream's scratch is made
+        took, a = taken_by(fn)
+        assert took == (i < len(taken)), i
         with monkeypatch.context() as m:
             m.setattr(_lib, "calls", lambda: Leave())
             b = fn()
         for u, v in zip(a if isinstance(a, tuple) else (a,), b if isinstance(b, tuple) else (b,)):
             assert u.dtype == v.dtype and u.shape == v.shape and torch.equal(u, v), i
+    # a scratch that is missing or too small is made by the wrapper; the next call is taken
+    for fn, tag in ((lambda: linear(x[0], w2), "linear"), (lambda: fused_attn_hyb(qa, kp, kp, kn, kn, msk), "attn")):
+        key = next(k for k in _lib._WORKSPACES if k[2] == tag)
+        for start in ({}, {key: torch.zeros(16, dtype=torch.uint8, device="cuda")}):
+            with monkeypatch.context() as m:
+                m.setattr(_lib, "_WORKSPACES", start)
+                (first, a), (second, b) = taken_by(fn), taken_by(fn)
+            assert not first and second and torch.equal(a, b)
     # errors are the wrappers' own
     with pytest.raises(TypeError):
         F.silu_mul(gu.float(), gu.float())
