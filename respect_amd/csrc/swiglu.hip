@@ -6,17 +6,21 @@
 // of PyTorch's bf16 F.silu(g) * u.  No reduction: each element depends on its
 // own g and u only, so rows never influence each other.
 //
-// Eight bf16 per thread (16-byte loads of g and u, one 16-byte store) where cols,
-// the strides and the pointers allow it, else two (4-byte ones), else one (the
-// same values).  Grid: x = blocks along a row, y = rows (one launch per 65535
-// rows), so a thread finds its row and column without a division.  Loads and stores are
-// non-temporal: nothing is read twice, and stores not kept in L2 shorten the
-// write-back at the kernel's end.  What bounds it: one memory round trip in small
-// calls, bandwidth in large ones, where four bytes per load kept too little in
-// flight -- gate/up [3072, 2 x 12288] 53.9 us with two elements per thread, 37.5
-// with eight (6.0 TB/s), [512, 2 x 12288] 11.0 -> 8.3; the packed [64, 2 x 12288]
-// call of a 64-node step 4.6 -> 3.8, launches back to back.  g and u may be
-// strided views (e.g. the two halves of a packed [rows, 2F] gate/up).
+// Two bf16 per thread (4-byte loads of g and u, one 4-byte store), four from kWide
+// elements on, where cols, the strides and the pointers allow it, else one (the same
+// values).  Grid: x = blocks along a row, y = rows (one launch per 65535 rows), so a
+// thread finds its row and column without a division.  Stores are non-temporal: not
+// kept in L2, they shorten the write-back at the kernel's end; loads are ordinary
+// (non-temporal ones: [2048, 2 x 6144] 15.6 us instead of 13.9).  What bounds it: one
+// memory round trip in small calls, where more elements per thread only lengthen the
+// chain and leave fewer wavefronts ([64, 2 x 12288] 3.02 / 3.19 / 3.47 us with 2 / 4 / 8
+// elements, [16, 2 x 3072] 2.10 / 2.15 / 2.33, [1, 2 x 4096] 2.06 / 2.08 / 2.15); and
+// bandwidth in large ones, where four bytes per load kept too little in flight
+// ([3072, 2 x 12288] 56.2 us with 2, 40.6 with 4 (5.6 TB/s), 39.7 with 8; [2511, 2 x 2112],
+// which fills 8-element blocks badly, 8.7 / 7.7 / 10.4).  The lines cross near 1.5 M
+// elements ([512, 2 x 2816] 3.88 / 3.89, [128, 2 x 12288] 3.93 / 3.90; graph replays over
+// rotating inputs).  g and u may be strided views (e.g. the two halves of a packed
+// [rows, 2F] gate/up).
 #include "common.h"
 #include "respect_amd.h"
 
@@ -24,12 +28,11 @@ namespace rspx {
 
 __device__ __forceinline__ float swiglu1(float g, float u) { return round_bf16(silu_f32(g)) * u; }
 
-// Threads of a block: with two elements each, 512 took 2.48 us for the [64, 2 x
-// 12288] call, 256 2.54.
-constexpr int swiglu_threads(int V) { return V == 8 ? 256 : 512; }
+constexpr int swiglu_threads(int V) { return V == 4 ? 256 : 512; }
+constexpr int64_t kWide = 3 << 19;   // elements
 constexpr int kMaxGridY = 65535;
 
-// V elements per thread: 8, 2 or 1.
+// V elements per thread: 4, 2 or 1.
 template <int V>
 __global__ __launch_bounds__(swiglu_threads(V)) void silu_mul_kernel(const uint16_t* g, int64_t sg, const uint16_t* u,
                                                                      int64_t su, uint16_t* y, int64_t sy, int row0,
@@ -40,14 +43,14 @@ __global__ __launch_bounds__(swiglu_threads(V)) void silu_mul_kernel(const uint1
   if (unit >= units) return;
   const int c = unit * V;
   const int row = row0 + blockIdx.y;
-  if constexpr (V == 8) {
-    const u32x4 gw = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(g + row * sg + c));
-    const u32x4 uw = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(u + row * su + c));
-    u32x4 o;
+  if constexpr (V == 4) {
+    const u32x2 gw = *reinterpret_cast<const u32x2*>(g + row * sg + c);
+    const u32x2 uw = *reinterpret_cast<const u32x2*>(u + row * su + c);
+    u32x2 o;
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < 2; ++i)
       o[i] = pack_bf16x2(swiglu1(bf16_lo(gw[i]), bf16_lo(uw[i])), swiglu1(bf16_hi(gw[i]), bf16_hi(uw[i])));
-    __builtin_nontemporal_store(o, reinterpret_cast<u32x4*>(y + row * sy + c));
+    __builtin_nontemporal_store(o, reinterpret_cast<u32x2*>(y + row * sy + c));
   } else if constexpr (V == 2) {
     const uint32_t gw = *reinterpret_cast<const uint32_t*>(g + row * sg + c);
     const uint32_t uw = *reinterpret_cast<const uint32_t*>(u + row * su + c);
@@ -72,7 +75,7 @@ extern "C" int rspx_silu_mul(const void* g, int64_t sg, const void* u, int64_t s
   auto fits = [&](int v) {
     return cols % v == 0 && al(g, 2 * v) && al(u, 2 * v) && al(y, 2 * v) && sg % v == 0 && su % v == 0 && sy % v == 0;
   };
-  const int v = fits(8) ? 8 : fits(2) ? 2 : 1;
+  const int v = (int64_t)rows * cols >= kWide && fits(4) ? 4 : fits(2) ? 2 : 1;
   const int units = cols / v;
   const unsigned bx = (unsigned)((units + swiglu_threads(v) - 1) / swiglu_threads(v));
   const hipStream_t s = static_cast<hipStream_t>(stream);
@@ -82,7 +85,7 @@ extern "C" int rspx_silu_mul(const void* g, int64_t sg, const void* u, int64_t s
   for (int row0 = 0; row0 < rows; row0 += kMaxGridY) {   // one launch per 65535 rows
     const dim3 grid(bx, (unsigned)min(rows - row0, kMaxGridY));
     const dim3 b(swiglu_threads(v));
-    if (v == 8) hipLaunchKernelGGL(silu_mul_kernel<8>, grid, b, 0, s, G, sg, U, su, Y, sy, row0, units);
+    if (v == 4) hipLaunchKernelGGL(silu_mul_kernel<4>, grid, b, 0, s, G, sg, U, su, Y, sy, row0, units);
     else if (v == 2) hipLaunchKernelGGL(silu_mul_kernel<2>, grid, b, 0, s, G, sg, U, su, Y, sy, row0, units);
     else hipLaunchKernelGGL(silu_mul_kernel<1>, grid, b, 0, s, G, sg, U, su, Y, sy, row0, units);
   }

@@ -346,11 +346,13 @@ def test_silu_mul_any_width(rows, F, off):
     assert torch.equal(y[:, :F], aligned)
 
 
-@pytest.mark.parametrize("rows,F", [(1, 8), (3, 2056), (342, 12288), (1025, 4104)])
-def test_silu_mul_eight_elements(rows, F):
-    """Widths and alignments at which a thread takes eight elements: the bits of the
-    two- and one-element forms (the same values at addresses only those take), and of
-    contiguous halves as of a packed gate/up tensor; infinities and NaN among them."""
+@pytest.mark.parametrize("rows,F", [(1, 8), (3, 2056), (342, 12288), (1025, 4104), (383, 4104), (384, 4096),
+                                    (1537, 1028), (1537, 1030)])
+def test_silu_mul_wide_forms(rows, F):
+    """Sizes on both sides of 1.5 M elements, from where a thread takes four of them, and widths
+    that are no multiple of four: the bits of the two- and one-element forms (the same values
+    at addresses only those take), and of contiguous halves as of a packed gate/up tensor;
+    infinities and NaN among them."""
     from respect_amd import _lib
     from respect_amd.system.fused import silu_mul
     print(f"[silu_mul] rows={rows} F={F}", flush=True)
