@@ -287,17 +287,46 @@ __device__ __forceinline__ void rope_vec(const float* xv, const float* cs, const
 
 // RoPE for D = 128: x [B, H, L, D] (any strides, D contiguous), cos/sin
 // [B, L, D] with row stride scl and batch stride scb; y [B, H, L, D] contiguous.
-// A thread takes one position's 16-byte unit of HB heads, so its cos/sin are read
-// once for them, HB loads are in flight instead of one, and where the heads of a
-// token lie side by side (a projection's output seen as [B, H, L, D]) a workgroup
-// reads whole KB pieces.  Grid: x = 16 positions each, y = groups of HB heads, z =
-// batch: no index divisions.  Bound by bandwidth (q of a 3072-token prompt, 32
-// heads: 11.9 us with one unit per thread, 9.2 with four, 5.5 TB/s) or, in small
-// calls, by the launch (64 tokens: 6.3 -> 4.5 us, launches back to back).
-constexpr int kRopeHeads = 4;
+// 16 lanes per (b, h, l) row.  For calls below kRopeWide rows and short sequences: one
+// memory round trip, with every lane at work whatever H and L are (8 tokens of 4
+// heads, 1.89 us; in 16-position, four-head workgroups 2.49).
 __global__ __launch_bounds__(256) void rope_kernel(const uint16_t* x, int64_t sxb, int64_t sxh, int64_t sxl,
                                                    const uint16_t* cosb, const uint16_t* sinb, int64_t scb,
-                                                   int64_t scl, uint16_t* y, int H, int L) {
+                                                   int64_t scl, uint16_t* y, int B, int H, int L) {
+  constexpr int D = 128;
+  const int gid = blockIdx.x * 256 + threadIdx.x;
+  const int rowid = gid >> 4;      // (b, h, l) row
+  const int sub = gid & 15;
+  const int nrows = B * H * L;
+  if (rowid >= nrows) return;      // 16-lane groups leave together
+  const int l = rowid % L;
+  const int h = (rowid / L) % H;
+  const int b = rowid / (L * H);
+  float xv[8], cs[8], sn[8], o[8];
+  unpack8(*reinterpret_cast<const u32x4*>(x + b * sxb + h * sxh + (int64_t)l * sxl + sub * 8), xv);
+  unpack8(*reinterpret_cast<const u32x4*>(cosb + b * scb + (int64_t)l * scl + sub * 8), cs);
+  unpack8(*reinterpret_cast<const u32x4*>(sinb + b * scb + (int64_t)l * scl + sub * 8), sn);
+  rope_vec(xv, cs, sn, sub, o);
+  *reinterpret_cast<u32x4*>(y + (int64_t)rowid * D + sub * 8) = pack8(o);
+}
+
+// The same for many rows.  A thread takes one position's 16-byte unit of HB heads, so
+// its cos/sin are read once for them, HB loads are in flight instead of one, and where
+// the heads of a token lie side by side (a projection's output seen as [B, H, L, D]) a
+// workgroup reads whole KB pieces.  Grid: x = 16 positions each, y = groups of HB heads,
+// z = batch: no index divisions.  Bound by bandwidth: q of a 3072-token prompt, 32
+// heads, 13.1 us in rope_kernel, 11.2 here; of 2200 tokens 9.9 / 8.4, 1024 tokens 5.66 /
+// 4.72, 512 tokens 3.76 / 3.69, 300 tokens 3.30 / 3.48, so the line lies at 16384 rows; 128
+// batches of 17 tokens, half of the lanes idle, 10.06 / 10.18 (graph replays over rotating
+// inputs).  Stores are non-temporal; a following attention call that reads them takes the
+// same time as after cached ones (512 tokens after 2560 keys, both calls: 84.4 / 84.3 us;
+// 3072 tokens: 805.1 / 805.3).
+constexpr int kRopeHeads = 4;
+constexpr int64_t kRopeWide = 16384;   // rows
+constexpr int kRopeWideTokens = 64;    // the last group of 16 positions leaves at most a fifth of the lanes idle
+__global__ __launch_bounds__(256) void rope_heads_kernel(const uint16_t* x, int64_t sxb, int64_t sxh, int64_t sxl,
+                                                         const uint16_t* cosb, const uint16_t* sinb, int64_t scb,
+                                                         int64_t scl, uint16_t* y, int H, int L) {
   constexpr int D = 128, HB = kRopeHeads;
   const int l = blockIdx.x * 16 + (threadIdx.x >> 4), sub = threadIdx.x & 15;
   const int h0 = blockIdx.y * HB, b = blockIdx.z;
@@ -768,21 +797,26 @@ extern "C" int rspx_rope(const void* x, int64_t sxb, int64_t sxh, int64_t sxl, c
   if (!x || !cosb || !sinb || !y) return RSPX_EINVAL;
   if (!al16(x) || !al16(cosb) || !al16(sinb) || !al16(y) || sxb % 8 || sxh % 8 || sxl % 8 || scb % 8 || scl % 8)
     return RSPX_EALIGN;
-  if (D == 128 && rows * 16 + 255 >= 0x7fffff00) return RSPX_EUNSUPPORTED;
-  const int64_t lg = (L + 15) / 16, hg = (H + kRopeHeads - 1) / kRopeHeads;
-  if (D != 128 || hg > 65535 || B > 65535) {
+  const hipStream_t st = static_cast<hipStream_t>(stream);
+  const uint16_t *X = static_cast<const uint16_t*>(x), *C = static_cast<const uint16_t*>(cosb),
+                 *S = static_cast<const uint16_t*>(sinb);
+  uint16_t* Y = static_cast<uint16_t*>(y);
+  if (D != 128) {
     const int64_t waves = (rows + 64 / (D / 8) - 1) / (64 / (D / 8));
     if ((waves + 3) / 4 > 0x7fffffff) return RSPX_EUNSUPPORTED;
-    hipLaunchKernelGGL(rope_any_kernel, dim3((unsigned)((waves + 3) / 4)), dim3(256), 0,
-                       static_cast<hipStream_t>(stream), static_cast<const uint16_t*>(x), sxb, sxh, sxl,
-                       static_cast<const uint16_t*>(cosb), static_cast<const uint16_t*>(sinb), scb, scl,
-                       static_cast<uint16_t*>(y), B, H, L, D);
+    hipLaunchKernelGGL(rope_any_kernel, dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, st, X, sxb, sxh, sxl, C, S, scb,
+                       scl, Y, B, H, L, D);
     return hipGetLastError() == hipSuccess ? RSPX_OK : RSPX_ELAUNCH;
   }
-  hipLaunchKernelGGL(rope_kernel, dim3((unsigned)lg, (unsigned)hg, (unsigned)B), dim3(256), 0,
-                     static_cast<hipStream_t>(stream), static_cast<const uint16_t*>(x), sxb, sxh, sxl,
-                     static_cast<const uint16_t*>(cosb), static_cast<const uint16_t*>(sinb), scb, scl,
-                     static_cast<uint16_t*>(y), H, L);
+  const int64_t threads = rows * 16;
+  if (threads + 255 >= 0x7fffff00) return RSPX_EUNSUPPORTED;   // 32-bit thread indices
+  const int64_t lg = (L + 15) / 16, hg = (H + kRopeHeads - 1) / kRopeHeads;
+  if (rows >= kRopeWide && L >= kRopeWideTokens && hg <= 65535 && B <= 65535)
+    hipLaunchKernelGGL(rope_heads_kernel, dim3((unsigned)lg, (unsigned)hg, (unsigned)B), dim3(256), 0, st, X, sxb, sxh,
+                       sxl, C, S, scb, scl, Y, H, L);
+  else
+    hipLaunchKernelGGL(rope_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, st, X, sxb, sxh, sxl, C, S,
+                       scb, scl, Y, B, H, L);
   return hipGetLastError() == hipSuccess ? RSPX_OK : RSPX_ELAUNCH;
 }
 

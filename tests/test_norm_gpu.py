@@ -373,10 +373,12 @@ def test_silu_mul_wide_forms(rows, F):
         assert torch.equal(bits(y), bits(out))
 
 
-@pytest.mark.parametrize("B,H,L", [(1, 1, 1), (1, 32, 513), (1, 7, 2350), (2, 9, 1000)])
+@pytest.mark.parametrize("B,H,L", [(1, 1, 1), (1, 32, 513), (1, 7, 2350), (2, 9, 1000), (1, 32, 511), (1, 32, 512),
+                                   (4, 65, 63), (4, 65, 64), (600, 32, 1)])
 def test_rope_heads_per_thread(B, H, L):
-    """Four heads per thread, H no multiple of four and L none of 16: bit for bit PyTorch's bf16
-    element-wise ops, from both orders of heads and tokens in memory."""
+    """Four heads per thread (from 16384 rows of sequences of 64 tokens on) and one, H no
+    multiple of four and L none of 16: bit for bit PyTorch's bf16 element-wise ops, from both
+    orders of heads and tokens in memory."""
     from respect_amd.system.fused import rope
     print(f"[rope] B={B} H={H} L={L}", flush=True)
     g = torch.Generator(device="cuda")
