@@ -62,15 +62,16 @@ bool rows_of(const Tensor& t, int64_t& m, int64_t& n, int64_t& stride) {
   const int64_t d = t.dim();
   if (d < 1) return false;
   n = t.size(d - 1);
+  if (n == 0) return false;   // the wrapper refuses rows of no elements
   if (d == 2) {
     m = t.size(0);
     stride = t.stride(0);
     return t.stride(1) == 1;
   }
   if (!t.is_contiguous()) return false;
-  m = n ? t.numel() / n : 0;
+  m = t.numel() / n;
   stride = n;
-  return n > 0;
+  return true;
 }
 
 bool fits_int(int64_t v) { return v >= 0 && v <= 0x7fffffff; }
@@ -235,7 +236,7 @@ PyObject* add_sq(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (n != 2) NOT_TAKEN;
   const Tensor *r = input(a[0]), *h = input(a[1]);
   if (!r || !h || r->dim() != 2 || r->sizes() != h->sizes() || !r->is_contiguous() || !h->is_contiguous() ||
-      r->device() != h->device() || !fits_int(r->size(0)) || !fits_int(r->size(1)))
+      r->device() != h->device() || !fits_int(r->size(0)) || !fits_int(r->size(1)) || r->size(1) == 0)
     NOT_TAKEN;
   const int64_t m = r->size(0), k = r->size(1);
   Tensor x = empty_like_of(*r, {m, k}), sq = empty_like_of(*r, {m, k}, at::kFloat);

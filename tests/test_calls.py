@@ -153,6 +153,12 @@ def test_calls_equal_the_wrappers_own_path(monkeypatch):
         linear(x.float(), w2)
     with pytest.raises(ValueError):
         fused_attn_hyb(qa, kp, kp, kn, kn, msk[:, :16])
+    # rows of no elements are refused, no rows are not
+    for fn in (lambda t: F.silu_mul(t, t), lambda t: rmsnorm(t, t[0], 1e-6), lambda t: F.add_sq(t, t)):
+        with pytest.raises(RuntimeError):
+            fn(gu[:, :0])
+    assert F.silu_mul(gu[:0], gu[:0]).shape == (0, 2048) and rmsnorm(x[:0], w, 1e-6).shape == (0, 5, 512)
+    assert F.add_sq(x[0, :0], x[0, :0])[0].shape == (0, 512) and linear(x[:0], w2).shape == (0, 5, 768)
 
 
 @pytest.mark.gpu
