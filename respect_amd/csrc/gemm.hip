@@ -713,9 +713,8 @@ __device__ __forceinline__ u32x4 any_cut(u32x4 v, int k, int K) {
 
 template <int MT, int CT> constexpr int any_kb() { return CT * MT >= 16 ? 1 : CT == 1 && MT <= 2 ? 4 : 2; }   // k-blocks of a round
 
-template <int MT, int CT>
+template <int MT, int CT, int KB = any_kb<MT, CT>()>
 __global__ __launch_bounds__(256, 2) void gemm_any_kernel(AnyArgs A, int units, int mtiles) {
-  constexpr int KB = any_kb<MT, CT>();
   constexpr int NC = KB * MT;           // 1 KB X fragments of a round
   constexpr int XL = (NC + 3) / 4;      // fragments a wave loads per round
   __shared__ __attribute__((aligned(16))) char xs[2 * XL * 4 * 1024];
@@ -840,6 +839,60 @@ __global__ __launch_bounds__(256, 2) void gemm_any_kernel(AnyArgs A, int units, 
         else
           static_cast<uint16_t*>(A.out)[(int64_t)m * A.so + n] = f32_to_bf16_rne(acc[t][c][e]);
       }
+  }
+}
+
+// Short K (8 .. 32 U): nothing to pipeline, so each wave loads its W fragments and all X
+// fragments at once, straight into the MFMA registers: one memory round trip, no LDS, no
+// barriers.  Workgroup = 64 columns (4 waves of 16) times 16 MT rows; the same chain.
+template <int MT, int U>
+__global__ __launch_bounds__(256) void gemm_short_kernel(AnyArgs A) {
+  const int lane = __lane_id(), wv = threadIdx.x >> 6;
+  const int n16 = lane & 15, g4 = lane >> 4;
+  const int n0 = blockIdx.x * 64 + wv * 16, m0 = blockIdx.y * 16 * MT, K = A.K;
+  if (n0 >= A.N) return;   // whole wave; no barriers below
+  const uint16_t* wp = A.w + (int64_t)min(n0 + n16, A.N - 1) * A.sw;
+  const uint16_t* xp[MT];
+#pragma unroll
+  for (int t = 0; t < MT; ++t) xp[t] = A.x + (int64_t)min(m0 + 16 * t + n16, A.M - 1) * A.sx;
+  f32x4 acc[MT];
+#pragma unroll
+  for (int t = 0; t < MT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  u32x4 wf[U], xf[U][MT];
+#pragma unroll
+  for (int kb = 0; kb < U; ++kb) {
+    const int k = min(32 * kb + 8 * g4, K - 8);
+    wf[kb] = any_load(wp + k);
+#pragma unroll
+    for (int t = 0; t < MT; ++t) xf[kb][t] = any_load(xp[t] + k);
+  }
+#pragma unroll
+  for (int kb = 0; kb < U; ++kb) {
+    const int k = 32 * kb;
+    if (k >= K) break;
+    if (k + 32 > K) {
+      wf[kb] = any_cut(wf[kb], k + 8 * g4, K);
+#pragma unroll
+      for (int t = 0; t < MT; ++t) xf[kb][t] = any_cut(xf[kb][t], k + 8 * g4, K);
+    }
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
+      acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wf[kb]),
+                                                       __builtin_bit_cast(bf16x8, xf[kb][t]), acc[t], 0, 0, 0);
+  }
+#pragma unroll
+  for (int t = 0; t < MT; ++t) {
+    const int m = m0 + 16 * t + n16;
+    if (m >= A.M) continue;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int n = n0 + 4 * g4 + e;
+      if (n >= A.N) continue;
+      if (A.out_fp32)
+        static_cast<float*>(A.out)[(int64_t)m * A.so + n] = acc[t][e];
+      else
+        static_cast<uint16_t*>(A.out)[(int64_t)m * A.so + n] = f32_to_bf16_rne(acc[t][e]);
+    }
   }
 }
 
@@ -1174,6 +1227,32 @@ static int linear_any(const void* x, int64_t sx, const void* w, int64_t sw, void
     hipLaunchKernelGGL(gemm::gemm_small_k_kernel, dim3((unsigned)tiles), dim3(64), 0, s, a, (N + 15) / 16);
     return hipGetLastError() == hipSuccess ? RSPX_OK : RSPX_ELAUNCH;
   }
+  // Short K: gemm_short_kernel, in row tiles as high as leave a workgroup to every CU.
+  // gemm_any_kernel spends a barrier and an LDS pass on a chain of one or two memory round
+  // trips (1 x 64 x 64: 3.81 us against 1.93; 760 x 6496 x 8: 20.8 / 14.5; 10 x 96 x 128:
+  // 3.20 / 2.43; 1 x 64 x 192: 3.87 / 2.78).  Above 128 it wins with more than two row tiles,
+  // which it reads once for four waves (82 x 8256 x 192: 6.9 / 11.4; 279 x 3296 x 192: 7.3 /
+  // 11.7); from 65 to 128 with more than two it is up to 15 % ahead or behind.
+  const int nt = (N + 63) / 64;
+  int ms = min((M + 15) / 16, 4);
+  while (ms > 1 && (int64_t)nt * ((M + 16 * ms - 17) / (16 * ms - 16)) <= 256) --ms;
+  if (K <= 128 || (K <= 256 && ms <= 2)) {
+    const dim3 g((unsigned)nt, (unsigned)((M + 16 * ms - 1) / (16 * ms)));
+    const int u = (K + 31) / 32;   // k-blocks
+#define RSPX_SHORT(MTV, UV) hipLaunchKernelGGL((gemm::gemm_short_kernel<MTV, UV>), g, dim3(256), 0, s, a)
+#define RSPX_SHORT_U(MTV)           \
+  if (u <= 1) RSPX_SHORT(MTV, 1);      \
+  else if (u <= 2) RSPX_SHORT(MTV, 2); \
+  else if (u <= 4) RSPX_SHORT(MTV, 4); \
+  else RSPX_SHORT(MTV <= 2 ? MTV : 2, 8);
+    if (ms == 1) { RSPX_SHORT_U(1) }
+    else if (ms == 2) { RSPX_SHORT_U(2) }
+    else if (ms == 3) { RSPX_SHORT_U(3) }
+    else { RSPX_SHORT_U(4) }
+#undef RSPX_SHORT
+#undef RSPX_SHORT_U
+    return hipGetLastError() == hipSuccess ? RSPX_OK : RSPX_ELAUNCH;
+  }
   // Row tiles of 1, 2, 4, 6 or 8 16-row tiles and 1, 2 or 4 column tiles a wave
   // (wave_tile); where that leaves CUs without a workgroup, lower row tiles
   // while the grid stays within one workgroup per CU (77 x 4864 x 896: 12.1 -> 8.0
@@ -1196,7 +1275,14 @@ static int linear_any(const void* x, int64_t sx, const void* w, int64_t sw, void
   else if (mt == 4) { RSPX_ANY(4, CTV) }                \
   else if (mt == 6) { RSPX_ANY(6, CTV) }                \
   else { RSPX_ANY(8, CTV) }
-  if (ct == 1) { RSPX_ANY_MT(1) }
+  // One and two row tiles of one column tile take rounds of four k-blocks; of two where
+  // those come out even and the K is short, since what K leaves to the end is a memory round
+  // trip of its own (2 x 448 x 576: 5.93 us with four, 4.58 with two).
+  const bool halves = K % 128 == 64 && K <= 640;
+  if (ct == 1 && mt <= 2 && halves) {
+    if (mt == 1) hipLaunchKernelGGL((gemm::gemm_any_kernel<1, 1, 2>), g, b, 0, s, a, (int)units, (int)mtl);
+    else hipLaunchKernelGGL((gemm::gemm_any_kernel<2, 1, 2>), g, b, 0, s, a, (int)units, (int)mtl);
+  } else if (ct == 1) { RSPX_ANY_MT(1) }
   else if (ct == 2) { RSPX_ANY_MT(2) }
   else { RSPX_ANY_MT(4) }
 #undef RSPX_ANY

@@ -471,7 +471,14 @@ def test_linear_many_rows(M, N, K):
 
 @pytest.mark.parametrize("M,N,K", [(1, 1, 1), (5, 40, 7), (17, 30, 8), (1, 65, 9), (16, 64, 63), (33, 129, 64),
                                    (64, 100, 65), (97, 300, 127), (128, 272, 129), (129, 4100, 200), (40, 16500, 96),
-                                   (300, 9000, 72)])
+                                   (300, 9000, 72),
+                                   # the direct kernel: 1 .. 8 k-blocks, 1 .. 4 row tiles, and past its lines
+                                   (1, 70, 32), (40, 16500, 33), (130, 9000, 31), (50, 17000, 128), (33, 80, 129),
+                                   (32, 9000, 255), (70, 17000, 161), (5, 48, 257),
+                                   # a rest of K after 2, 3, 4, 5, ... rounds of four, two and one k-blocks
+                                   (3, 40, 300), (20, 40, 420), (7, 33, 520), (16, 100, 700), (64, 100, 270),
+                                   (60, 17000, 340), (64, 200, 400), (128, 9000, 460), (128, 16500, 265),
+                                   (128, 16500, 300), (120, 16500, 330), (128, 16500, 370)])
 def test_linear_any_shape_edges(M, N, K):
     """Outside N % 16 == 0, K % 256 == 0: K below one load, below a round, whole rounds with and
     without a rest, every row and column tile height and width; the accumulation bound in fp32,
