@@ -106,6 +106,14 @@ __device__ __forceinline__ int wg_index(const TrieAttnArgs& A, int g, int rb, in
   return g + A.HK * (rb + A.NRB * q);
 }
 
+// A.c for a product with a vector.  Loaded straight into a splat, the compiler reads it as
+// a vector with the words behind it, and then keeps a copy of them in LDS or scratch.
+__device__ __forceinline__ float score_scale(const TrieAttnArgs& A) {
+  float c = A.c;
+  asm("" : "+s"(c));
+  return c;
+}
+
 // Phase timestamps (built only with -DRSPX_PHASE_TRACE, into a separate
 // library; the product library has none of this): wave w of workgroup b
 // records the device's real-time counter (s_memrealtime, 100 MHz) at mark k
@@ -1031,10 +1039,24 @@ template <int D> struct StreamLds {
   static_assert(BATCH * TILE <= NBUF * CB, "gathered tiles fit the chunk buffers");
 };
 
-// Bytes of LDS the node phase may use (any of the layouts).
-template <int D> constexpr int node_area_bytes() {
-  const int a = NodeLds<D>::BYTES, b = VResLds<D>::BYTES, c = StreamLds<D>::SLOTS > 0 ? StreamLds<D>::BYTES : 0;
-  return a > b ? (a > c ? a : c) : (b > c ? b : c);
+// The node form of a call, chosen at launch from its node slots (the kernels' argument
+// kStream): node_stream for segments that do not stay resident and fit its score area,
+// else the resident and gathered forms.  In kernels of their own: with node_stream beside
+// the others fused_kernel<128, 2> took 223 vector registers and spilled 224 scalar ones
+// (208 and 116 without), fused_kernel<64, *> 168 and 264 (150 and 108), and every
+// node_merge_kernel<64> 98,944 bytes of LDS, one workgroup per CU (76,480, two), which
+// cost calls that never run it 2 to 6 % (16 q / 2 kv heads of 64, 4 nodes after 90 keys:
+// 15.5 us, 14.7 without; 64 rows a kv head, no prompt: 10.3 / 7.9).  Streamed calls of head_dim 32
+// and 64 take 3 to 5 % longer in the smaller kernel (3 nodes, 347 committed: 14.2 -> 15.0 us).
+template <int D> constexpr bool streams(int NN) {
+  return StreamLds<D>::SLOTS > 0 && NN > NodeLds<D>::RES * kChunk && NN > VResLds<D>::RES * kChunk &&
+         NN <= StreamLds<D>::SLOTS;
+}
+
+// Bytes of LDS the node phase of a form may use.
+template <int D, bool kStream> constexpr int node_area_bytes() {
+  if (kStream) return StreamLds<D>::BYTES;
+  return NodeLds<D>::BYTES > VResLds<D>::BYTES ? NodeLds<D>::BYTES : VResLds<D>::BYTES;
 }
 
 // Where a row's result goes: row r of kv head g is query r / GQA of head
@@ -1246,7 +1268,7 @@ __device__ __forceinline__ void node_scores(const TrieAttnArgs& A, int c0, const
     sv = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, qf[i], sv, 0, 0, 0);
   }
   // Lane (n16, g4), element j: slot 16 kt + 4 g4 + j of row p0 + n16.
-  *(lds_f32x4*)(S + (lane & 15) * SR + 16 * kt + 4 * (lane >> 4)) = sv * A.c;
+  *(lds_f32x4*)(S + (lane & 15) * SR + 16 * kt + 4 * (lane >> 4)) = sv * score_scale(A);
 }
 
 __device__ __forceinline__ float max64(float x) {
@@ -1529,10 +1551,10 @@ __device__ __forceinline__ const lds_float* node_stream(const TrieAttnArgs& A, i
                                                        int w, const bf16x8 (&qf)[D / 32]) {
   using LY = StreamLds<D>;
   constexpr int DQ = D / 32, DT = D / 16, RB = 2 * D, nw = kWavesA;
-  int lane = __lane_id();
-  asm volatile("" : "+v"(lane));   // nothing computed from it is shared with the other forms: the registers are full
+  const int lane = __lane_id();
   const int n16 = lane & 15, g4 = lane >> 4, e4 = n16 >> 2, c4 = n16 & 3;
   const int NN = A.NN, nch = (NN + kChunk - 1) / kChunk, nt = (NN + 15) / 16;
+  const float scale = score_scale(A);
   const int GQA = 1 << A.GQS, q0 = p0 >> A.GQS, ng = ((rend - 1) >> A.GQS) - q0 + 1;
   const int nrd = (rend - p0 - w + nw - 1) / nw;   // rows of this wave: p0 + w + 8 i
   lds_float* S = (lds_float*)(kv + LY::SOFF);
@@ -1592,7 +1614,7 @@ __device__ __forceinline__ const lds_float* node_stream(const TrieAttnArgs& A, i
 #pragma unroll
       for (int i = 0; i < DQ; ++i)
         sv = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, kf[u][i]), qf[i], sv, 0, 0, 0);
-      *(lds_f32x4*)(S + n16 * LY::SR + 16 * (tb + nw * u) + 4 * g4) = sv * A.c;
+      *(lds_f32x4*)(S + n16 * LY::SR + 16 * (tb + nw * u) + 4 * g4) = sv * scale;
     }
   }
   lds_barrier();   // every score is in LDS
@@ -1764,7 +1786,7 @@ __device__ __forceinline__ const lds_float* node_stream(const TrieAttnArgs& A, i
 // loads (vmcnt 0) and passed a workgroup barrier.  A resident segment the
 // caller did not issue is loaded here; a longer one streams: its maxima come
 // from a pass over K chunk by chunk, its sums from K and V gathered by rank.
-template <int D>
+template <int D, bool kStream>
 __device__ __forceinline__ const lds_float* node_rows(const TrieAttnArgs& A, int g, int p0, int rend, lds_char* kv,
                                                      int w, const NodePre<D>& pre, bool have_pre) {
   using LY = NodeLds<D>;
@@ -1791,12 +1813,9 @@ __device__ __forceinline__ const lds_float* node_rows(const TrieAttnArgs& A, int
     node_q<D>(A, g, p0, rend, qf);
   }
 
-  if constexpr (StreamLds<D>::SLOTS > 0) {
-    // 264 slots (200 committed): 20.9 us for the 64-node call with V resident, 22.4
-    // with node_stream; 500 slots: 44.7 gathered, 31.7 with node_stream.
-    if (__builtin_expect(!res && !vres && NN <= StreamLds<D>::SLOTS, 0))
-      return node_stream<D>(A, g, p0, rend, kv, w, qf);
-  }
+  // 264 slots (200 committed): 20.9 us for the 64-node call with V resident, 22.4
+  // with node_stream; 500 slots: 44.7 gathered, 31.7 with node_stream.
+  if constexpr (kStream) return node_stream<D>(A, g, p0, rend, kv, w, qf);
 
   // Maxima, mask words, allowed counts.  The first row of each group in
   // [p0, rend) records the group's mask words and count.
@@ -1880,7 +1899,7 @@ __device__ __forceinline__ const lds_float* node_rows(const TrieAttnArgs& A, int
         for (int i = 0; i < DQ; ++i)
           sv = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, kf[j][i]), qf[i], sv, 0, 0, 0);
         // Lane (n16, g4), element j: slot 16 tt + 4 g4 + j of row p0 + n16 (the chain of node_scores).
-        *(lds_f32x4*)(SV + n16 * VL::SR + 16 * tt + 4 * g4) = sv * A.c;
+        *(lds_f32x4*)(SV + n16 * VL::SR + 16 * tt + 4 * g4) = sv * score_scale(A);
       }
     }
     if (w == 0) {
@@ -1924,7 +1943,7 @@ __device__ __forceinline__ const lds_float* node_rows(const TrieAttnArgs& A, int
         for (int i = 0; i < DQ; ++i)
           sv = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, kf[i]), qf[i], sv, 0, 0, 0);
         // Lane (n16, g4), element j: slot s0 + 16 tt + 4 g4 + j of row p0 + n16.
-        *(lds_f32x4*)(SS + n16 * SRS + 16 * tt + 4 * g4) = sv * A.c;
+        *(lds_f32x4*)(SS + n16 * SRS + 16 * tt + 4 * g4) = sv * score_scale(A);
       }
       lds_barrier();
 #pragma unroll 1
@@ -2097,24 +2116,24 @@ __device__ __forceinline__ void merge_rounds(const TrieAttnArgs& A, int g, int p
 // Workgroup (g, c8): rows [8 c8, 8 c8 + 8) of kv head g, row 8 c8 + w on
 // wave w: node partial, then merge.  A node segment of at most RES chunks
 // is loaded whole up front; a longer one streams.
-template <int D>
+template <int D, bool kStream>
 __global__ __launch_bounds__(64 * kWavesA) void node_merge_kernel(TrieAttnArgs A) {
   using LY = NodeLds<D>;
   static_assert(8 <= kNodeRows, "a workgroup's rows fit the node areas");
-  __shared__ __attribute__((aligned(16))) char kv[node_area_bytes<D>()];
+  __shared__ __attribute__((aligned(16))) char kv[node_area_bytes<D, kStream>()];
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform (SGPR)
   const int RC8 = (A.R + 7) / 8;
   const int g = blockIdx.x / RC8;
   const int p0 = 8 * (blockIdx.x - g * RC8);
   const int rend = min(p0 + 8, A.R);
   NodePre<D> pre;
-  const bool pf = A.NN > 0 && A.NN <= LY::RES * kChunk;
+  const bool pf = !kStream && A.NN > 0 && A.NN <= LY::RES * kChunk;
   if (pf) {
     node_prefetch<D>(A, g, p0, rend, (lds_char*)kv, w, pre);
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's part of the segment is in LDS
     lds_barrier();                       // and every other wave's part
   }
-  const lds_float* np = node_rows<D>(A, g, p0, rend, (lds_char*)kv, w, pre, pf);
+  const lds_float* np = node_rows<D, kStream>(A, g, p0, rend, (lds_char*)kv, w, pre, pf);
   merge_rounds<D, false>(A, g, p0, rend, np, w);
 }
 
@@ -2545,16 +2564,16 @@ __device__ __forceinline__ void merge_share(const TrieAttnArgs& A, int rb, int q
 // first batch.  old: the counter before this workgroup's share
 // (counter_before), so the block is complete once the counter has moved
 // kCountUnit past the multiple of kCountUnit below it.
-template <int D, int kRT>
+template <int D, int kRT, bool kStream>
 __device__ __forceinline__ void block_tail(const TrieAttnArgs& A, char* lds, int g, int rb, int q, int r0, int rend,
                                            const NodePre<D>& pre, bool pf, int old) {
   const int lane = __lane_id();
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int* cnt = A.sync + 1 + 2 * (g * A.NRB + rb);
   const int rend0 = min(rend, r0 + kNodeRows);
-  int* gave_up = reinterpret_cast<int*>(lds + node_area_bytes<D>());  // one LDS word past the node areas
+  int* gave_up = reinterpret_cast<int*>(lds + node_area_bytes<D, kStream>());  // one LDS word past the node areas
   if (r0 < rend) {
-    const lds_float* np = node_rows<D>(A, g, r0, rend0, (lds_char*)lds, w, pre, pf);
+    const lds_float* np = node_rows<D, kStream>(A, g, r0, rend0, (lds_char*)lds, w, pre, pf);
     RSPX_MARK(12);
     if (w == 0) {
       // Bounded in time (A.deadline ticks of the constant-rate real-time
@@ -2585,7 +2604,7 @@ __device__ __forceinline__ void block_tail(const TrieAttnArgs& A, char* lds, int
     for (int b0 = rend0; b0 < rend; b0 += kNodeRows) {
       const int be = min(rend, b0 + kNodeRows);
       NodePre<D> none;
-      const lds_float* npb = node_rows<D>(A, g, b0, be, (lds_char*)lds, w, none, false);
+      const lds_float* npb = node_rows<D, kStream>(A, g, b0, be, (lds_char*)lds, w, none, false);
       if (bad) nan_rows<D>(A, g, b0, be, w);
       else merge_rounds<D, true>(A, g, b0, be, npb, w);
     }
@@ -2623,11 +2642,11 @@ __device__ __forceinline__ int counter_before(const TrieAttnArgs& A, int g, int 
   return __hip_atomic_load(A.sync + 1 + 2 * (g * A.NRB + rb), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-template <int D, int kRT>
+template <int D, int kRT, bool kStream>
 __global__ __launch_bounds__(512) void fused_kernel(TrieAttnArgs A) {
   using LY = NodeLds<D>;
   using PL = PromptLds<D, kRT>;
-  constexpr int NB = node_area_bytes<D>() + 16;
+  constexpr int NB = node_area_bytes<D, kStream>() + 16;
   constexpr int LB = PL::BYTES + PL::MLBYTES > NB ? PL::BYTES + PL::MLBYTES : NB;
   static_assert(NB <= PL::RINGBYTES, "node LDS and the wait flag inside the ring (the Q fragments stay)");
   __shared__ __attribute__((aligned(1024))) char lds[LB];
@@ -2649,8 +2668,8 @@ __global__ __launch_bounds__(512) void fused_kernel(TrieAttnArgs A) {
   // D = 128 the first chunk's K/V and the mask bytes are requested into
   // registers before the quarter combine (whose LDS traffic they then
   // overlap) and written into the ring after it.
-  const bool pf = A.NN > 0 && A.NN <= LY::RES * kChunk && r0 < rend;
-  constexpr bool kEarly = D <= 128;
+  const bool pf = !kStream && A.NN > 0 && A.NN <= LY::RES * kChunk && r0 < rend;
+  constexpr bool kEarly = D <= 128 && !kStream;
   NodePre<D> pre;
   u32x4 pc[node_pieces<D>()];
   const lds_char* qreg = (const lds_char*)lds + PL::RINGBYTES;
@@ -2678,7 +2697,7 @@ __global__ __launch_bounds__(512) void fused_kernel(TrieAttnArgs A) {
       },
       [] {});
   count_partial(A, g, rb, q);
-  block_tail<D, kRT>(A, lds, g, rb, q, r0, rend, pre, pf, old);
+  block_tail<D, kRT, kStream>(A, lds, g, rb, q, r0, rend, pre, pf, old);
 }
 
 // The same work as fused_kernel for grids twice as large as the device holds at
@@ -2692,7 +2711,7 @@ __global__ __launch_bounds__(512) void fused_kernel(TrieAttnArgs A) {
 template <int D, int kRT>
 __global__ __launch_bounds__(512) void fused2_kernel(TrieAttnArgs A) {
   using PL = PromptLds<D, kRT>;
-  constexpr int NB = node_area_bytes<D>() + 16;
+  constexpr int NB = node_area_bytes<D, false>() + 16;
   constexpr int LB = PL::BYTES + PL::MLBYTES > NB ? PL::BYTES + PL::MLBYTES : NB;
   static_assert(NB <= PL::RINGBYTES, "node LDS and the wait flag inside the ring (the Q fragments stay)");
   __shared__ __attribute__((aligned(1024))) char lds[LB];
@@ -2730,14 +2749,14 @@ __global__ __launch_bounds__(512) void fused2_kernel(TrieAttnArgs A) {
     count_partial(A, g, rb1, q);
   }
   if (pairs) {
-    block_tail<D, kRT>(A, lds, g, mrb, q, m0, mend, none, false, second ? old[1] : old[0]);
+    block_tail<D, kRT, false>(A, lds, g, mrb, q, m0, mend, none, false, second ? old[1] : old[0]);
   } else {
     int r0, rend;
     merge_share<kRT>(A, rbw, q, r0, rend);
-    block_tail<D, kRT>(A, lds, g, rbw, q, r0, rend, none, false, old[0]);
+    block_tail<D, kRT, false>(A, lds, g, rbw, q, r0, rend, none, false, old[0]);
     if (nb > 1) {
       merge_share<kRT>(A, rb1, q, r0, rend);
-      block_tail<D, kRT>(A, lds, g, rb1, q, r0, rend, none, false, old[1]);
+      block_tail<D, kRT, false>(A, lds, g, rb1, q, r0, rend, none, false, old[1]);
     }
   }
 }
@@ -2745,11 +2764,11 @@ __global__ __launch_bounds__(512) void fused2_kernel(TrieAttnArgs A) {
 // The same work as fused_kernel with 128-row blocks (pair_block), for grids up to
 // twice as large as the device holds at once in 64-row blocks (e.g. 128-node
 // tries at 8B heads: 512 rows per kv head): A.NRB counts 128-row blocks.
-template <int D>
+template <int D, bool kStream>
 __global__ __launch_bounds__(512) void fused_pair_kernel(TrieAttnArgs A) {
   using LY = NodeLds<D>;
   using PL = PairLds<D>;
-  constexpr int NB = node_area_bytes<D>() + 16;
+  constexpr int NB = node_area_bytes<D, kStream>() + 16;
   static_assert(NB <= PL::RINGBYTES, "node LDS and the wait flag inside the ring");
   __shared__ __attribute__((aligned(1024))) char lds[PL::BYTES];
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -2761,13 +2780,13 @@ __global__ __launch_bounds__(512) void fused_pair_kernel(TrieAttnArgs A) {
   merge_share<4>(A, rb, q, r0, rend);
   const int rend0 = min(rend, r0 + kNodeRows);               // the first batch of node rows
   const int old = counter_before(A, g, rb);
-  const bool pf = A.NN > 0 && A.NN <= LY::RES * kChunk && r0 < rend;
+  const bool pf = !kStream && A.NN > 0 && A.NN <= LY::RES * kChunk && r0 < rend;
   NodePre<D> pre;
   pair_block<D, true, false>(A, lds, g, rb, q, q + 1, [&] {
     if (pf) node_prefetch<D>(A, g, r0, rend0, (lds_char*)lds, w, pre);
   });
   count_partial(A, g, rb, q);
-  block_tail<D, 4>(A, lds, g, rb, q, r0, rend, pre, pf, old);
+  block_tail<D, 4, kStream>(A, lds, g, rb, q, r0, rend, pre, pf, old);
 }
 
 // ------------------------------------------------------------------ host side
@@ -2779,8 +2798,8 @@ struct Plan {
 
 static inline size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
 
-template <int D, int RT, bool TWO = false>
-static int fused_capacity();
+template <int D, int RT>
+static int fused_capacity(int NN);
 
 // Steps per group S = 4 NR and the group count NG <= 8 depend on P only.
 static int make_plan(int H, int HK, int M, int P, int NN, int D, int rows_per_wave, Plan* pl) {
@@ -2807,9 +2826,9 @@ static int make_plan(int H, int HK, int M, int P, int NN, int D, int rows_per_wa
     // D = 256 always takes one (two tiles of 256 columns exceed the registers).
     const int nrb1 = (pl->R + 31) / 32;
     const int cap1 = D == 256 ? 0
-                     : D == 128 ? fused_capacity<128, 1>()
-                     : D == 64  ? fused_capacity<64, 1>()
-                                : fused_capacity<32, 1>();
+                     : D == 128 ? fused_capacity<128, 1>(NN)
+                     : D == 64  ? fused_capacity<64, 1>(NN)
+                                : fused_capacity<32, 1>(NN);
     rt = (D == 256 || (pl->NG > 0 && HK * nrb1 * pl->NG <= cap1)) ? 1 : 2;
   }
   if (rt != 1 && rt != 2) return RSPX_EINVAL;
@@ -2831,10 +2850,10 @@ static int make_plan(int H, int HK, int M, int P, int NN, int D, int rows_per_wa
   return RSPX_OK;
 }
 
-// Workgroups of fused_kernel<D, RT> (TWO: fused_pair_kernel<D>, or at D = 256
-// fused2_kernel<D, RT>) the device holds at once (0 if unknown).
-template <int D, int RT, bool TWO>
-static int fused_capacity() {
+// Workgroups of fused_kernel<D, RT, kStream> (TWO: fused_pair_kernel<D, kStream>, or at
+// D = 256 fused2_kernel<D, RT>) the device holds at once (0 if unknown).
+template <int D, int RT, bool TWO, bool kStream>
+static int fused_capacity_of() {
   static int cap[64];
   static bool done[64];
   int dev = 0;
@@ -2842,18 +2861,29 @@ static int fused_capacity() {
   if (!done[dev]) {
     int a = 0, cus = 0;
     hipError_t e;
-    if constexpr (TWO && D <= 128) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&a, fused_pair_kernel<D>, 64 * kWavesA, 0);
+    if constexpr (TWO && D <= 128)
+      e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&a, fused_pair_kernel<D, kStream>, 64 * kWavesA, 0);
     else if constexpr (TWO) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&a, fused2_kernel<D, RT>, 64 * kWavesA, 0);
-    else e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&a, fused_kernel<D, RT>, 64 * kWavesA, 0);
+    else e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&a, fused_kernel<D, RT, kStream>, 64 * kWavesA, 0);
     if (e != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) {
       a = cus = 0;
     }
     cap[dev] = a * cus;
     done[dev] = true;
   }
+  // The streamed form needs fewer registers: at D = 32 two of its workgroups fit a CU, but
+  // calls of that size are faster in two launches (16 heads, 472 rows after 3163 keys: 42.4
+  // us, 67.8 in one), so the line is the plain form's.
+  if constexpr (kStream) return min(cap[dev], fused_capacity_of<D, RT, TWO, false>());
   return cap[dev];
 }
 
+// The same for fused_kernel in the node form of NN slots.
+template <int D, int RT>
+static int fused_capacity(int NN) {
+  if (streams<D>(NN)) return fused_capacity_of<D, RT, false, true>();
+  return fused_capacity_of<D, RT, false, false>();
+}
 
 // How many workgroups share the NG key groups of a 128-row block (S steps each),
 // blocks = kv heads x row blocks: the least time for the busiest CU, from what a
@@ -2869,13 +2899,13 @@ static int pair_splits(int blocks, int NG, int S) {
   return best;
 }
 
-template <int D, int RT>
+template <int D, int RT, bool kStream>
 static void launch_rt(const TrieAttnArgs& a, const Plan& pl, hipStream_t s, int mode) {
   const bool one = pl.NG > 0 && mode != 2 && 1 + 2 * pl.NRB * a.HK <= kSyncWords &&
                    (size_t)a.HK * pl.R * pl.NG * D * sizeof(float) < (size_t(1) << 31);
-  const int cap = one ? fused_capacity<D, RT>() : 0;
+  const int cap = one ? fused_capacity_of<D, RT, false, kStream>() : 0;
   if (one && pl.prompt_wgs <= cap) {
-    hipLaunchKernelGGL((fused_kernel<D, RT>), dim3(a.HK, pl.NRB, pl.NG), dim3(64 * kWavesA), 0, s, a);
+    hipLaunchKernelGGL((fused_kernel<D, RT, kStream>), dim3(a.HK, pl.NRB, pl.NG), dim3(64 * kWavesA), 0, s, a);
     return;
   }
   // Twice the rows per workgroup when that grid fits: 128-row blocks, or (D = 256)
@@ -2883,7 +2913,7 @@ static void launch_rt(const TrieAttnArgs& a, const Plan& pl, hipStream_t s, int 
   // nodes in a launch each.
   const int nrb2 = D == 256 ? (pl.NRB + 1) / 2 : (pl.R + 127) / 128;
   const dim3 g2(a.HK, nrb2, pl.NG), b8(64 * kWavesA);
-  const bool two = one && pl.NRB > 1 && a.HK * nrb2 * pl.NG <= fused_capacity<D, RT, true>();
+  const bool two = one && pl.NRB > 1 && a.HK * nrb2 * pl.NG <= fused_capacity_of<D, RT, true, kStream>();
   if constexpr (D == 256) {
     if (two) {
       hipLaunchKernelGGL((fused2_kernel<D, RT>), g2, b8, 0, s, a);
@@ -2894,7 +2924,7 @@ static void launch_rt(const TrieAttnArgs& a, const Plan& pl, hipStream_t s, int 
     if (two) {
       TrieAttnArgs b = a;
       b.NRB = nrb2;
-      hipLaunchKernelGGL((fused_pair_kernel<D>), g2, b8, 0, s, b);
+      hipLaunchKernelGGL((fused_pair_kernel<D, kStream>), g2, b8, 0, s, b);
       return;
     }
     if (pl.prompt_wgs > 0)
@@ -2912,14 +2942,19 @@ static void launch_rt(const TrieAttnArgs& a, const Plan& pl, hipStream_t s, int 
       return;
     }
   }
-  hipLaunchKernelGGL((node_merge_kernel<D>), dim3(pl.node_wgs), dim3(64 * kWavesA), 0, s, a);
+  hipLaunchKernelGGL((node_merge_kernel<D, kStream>), dim3(pl.node_wgs), dim3(64 * kWavesA), 0, s, a);
 }
 
 template <int D>
 static void launch_all(const TrieAttnArgs& a, const Plan& pl, hipStream_t s, int mode) {
-  if constexpr (D == 256) launch_rt<D, 1>(a, pl, s, mode);
-  else if (pl.RT == 1) launch_rt<D, 1>(a, pl, s, mode);
-  else launch_rt<D, 2>(a, pl, s, mode);
+  if constexpr (D == 256) launch_rt<D, 1, false>(a, pl, s, mode);
+  else if (streams<D>(a.NN)) {
+    if (pl.RT == 1) launch_rt<D, 1, true>(a, pl, s, mode);
+    else launch_rt<D, 2, true>(a, pl, s, mode);
+  } else {
+    if (pl.RT == 1) launch_rt<D, 1, false>(a, pl, s, mode);
+    else launch_rt<D, 2, false>(a, pl, s, mode);
+  }
 }
 
 static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }

@@ -534,6 +534,8 @@ def test_tiled_output_rejects_a_head_stride_other_than_d():
     (8, 2, 64, 1000, 100, "random"),       # 1024 slots: the longest segment node_stream takes
     (8, 2, 32, 500, 64, "open32k"),        # 512 slots: its longest at head_dim 32
     (8, 2, 32, 530, 33, "causal"),         # 544 slots: gathered
+    (8, 2, 64, 321, 64, "open32k"),        # 352 slots: the shortest segment node_stream takes
+    (16, 16, 32, 472, 3163, "causal"),     # head_dim 32 in 480 slots, a grid of two workgroups per CU
 ])
 def test_many_rows(H, HK, D, M, P, mask):
     """Calls whose grid never fits the device at once (prompt part and node part in a launch
