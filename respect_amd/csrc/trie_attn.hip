@@ -2888,8 +2888,15 @@ static int fused_capacity(int NN) {
 // How many workgroups share the NG key groups of a 128-row block (S steps each),
 // blocks = kv heads x row blocks: the least time for the busiest CU, from what a
 // workgroup spends (8B heads, in 0.1 us): 45 before its first round, 28 a round of
-// four steps, 15 a group's end.
+// four steps, 15 a group's end.  Workgroups of one group each run on as others end, so up
+// to an eighth more of them than CUs costs less than giving some two groups (36 blocks x 8
+// groups, head_dim 128, 5921 keys: 51.4 us with 8 splits, 55.3 with 7; head_dim 64, 5558 keys:
+// 36.1 / 41.5 with 4).  At head_dim 32 two workgroups fit a CU and a group's end is most of
+// the time: one group each is the fastest at 7 to 252 blocks (36 x 8: 23.5 us, 32.0 with 4;
+// 128 x 8, 6000 keys: 43.2, 51.4 with 2).
+template <int D>
 static int pair_splits(int blocks, int NG, int S) {
+  if (D == 32 || blocks * NG <= 288) return NG;
   int best = 1;
   int64_t t_best = 0;
   for (int z = 1; z <= NG; ++z) {
@@ -2928,7 +2935,7 @@ static void launch_rt(const TrieAttnArgs& a, const Plan& pl, hipStream_t s, int 
       return;
     }
     if (pl.prompt_wgs > 0)
-      hipLaunchKernelGGL((prompt_pair_kernel<D>), dim3(a.HK, nrb2, pair_splits(a.HK * nrb2, pl.NG, pl.S)), b8, 0, s, a);
+      hipLaunchKernelGGL((prompt_pair_kernel<D>), dim3(a.HK, nrb2, pair_splits<D>(a.HK * nrb2, pl.NG, pl.S)), b8, 0, s, a);
   }
   if constexpr (D <= 128) {
     // Nodes and merge: 64-row blocks once they give a quarter of the CUs a workgroup

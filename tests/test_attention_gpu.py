@@ -536,6 +536,8 @@ def test_tiled_output_rejects_a_head_stride_other_than_d():
     (8, 2, 32, 530, 33, "causal"),         # 544 slots: gathered
     (8, 2, 64, 321, 64, "open32k"),        # 352 slots: the shortest segment node_stream takes
     (16, 16, 32, 472, 3163, "causal"),     # head_dim 32 in 480 slots, a grid of two workgroups per CU
+    (16, 2, 32, 279, 5558, "causal"),      # 36 128-row blocks in 8 splits
+    (8, 2, 128, 570, 5921, "causal"),
 ])
 def test_many_rows(H, HK, D, M, P, mask):
     """Calls whose grid never fits the device at once (prompt part and node part in a launch
