@@ -2942,9 +2942,15 @@ static void launch_rt(const TrieAttnArgs& a, const Plan& pl, hipStream_t s, int 
     // (8B heads, causal rows after 2560 prompt keys: 130 rows 36.8 us for the call
     // instead of 44.4 with node_merge_kernel, 192 rows 46.9 / 56.7, 512 rows 89 / 241;
     // 8 q / 2 kv heads of 64, 320 rows, 40 blocks: 29.4 / 27.4, so below that
-    // node_merge_kernel's 8-row workgroups stay).
-    const int nrb64 = (pl.R + 63) / 64;
-    if (a.NN > 0 && nrb64 <= 65535 && a.HK * nrb64 >= 64) {
+    // node_merge_kernel's 8-row workgroups stay).  At head_dim 32 and 64, where two or more
+    // of those fit a CU, the line lies past 64 blocks (16 heads of 64, 234 rows, no prompt,
+    // 64 blocks: 16.7 / 15.2; 16 of 32, 221 rows: 15.2 / 13.0; 16 / 2 heads of 32, 266 rows,
+    // 68 blocks: 10.8 / 13.2; 32 / 4 heads of 64, 139 rows, 72 blocks: 9.45 / 13.2).
+    // Where node_merge_kernel would stream the segment and the rows are a prompt chunk's
+    // (more than 256), 40 blocks are enough (first chunks, 8 q / 2 kv heads: of 64, 385 rows
+    // 15.9 / 22.8; of 128, 489 rows 26.1 / 33.9; 4 heads of 128, 504 rows, 32 blocks: 33.9 / 25.7).
+    const int nrb64 = (pl.R + 63) / 64, line = kStream && D >= 64 && a.M > 256 ? 40 : D == 128 ? 64 : 65;
+    if (a.NN > 0 && nrb64 <= 65535 && a.HK * nrb64 >= line) {
       hipLaunchKernelGGL((node_block_kernel<D>), dim3(a.HK, nrb64), dim3(64 * kWavesA), 0, s, a);
       return;
     }

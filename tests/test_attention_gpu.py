@@ -536,6 +536,10 @@ def test_tiled_output_rejects_a_head_stride_other_than_d():
     (8, 2, 32, 530, 33, "causal"),         # 544 slots: gathered
     (8, 2, 64, 321, 64, "open32k"),        # 352 slots: the shortest segment node_stream takes
     (16, 16, 32, 472, 3163, "causal"),     # head_dim 32 in 480 slots, a grid of two workgroups per CU
+    (16, 16, 64, 234, 0, "causal"),        # 64 and 68 blocks of 64 rows, where head_dim 32 and 64 change kernels
+    (16, 2, 64, 266, 40, "causal"),
+    (8, 2, 64, 310, 0, "causal"),          # 40 blocks over a segment that would stream
+    (8, 2, 128, 300, 0, "causal"),         # 38
     (16, 2, 32, 279, 5558, "causal"),      # 36 128-row blocks in 8 splits
     (8, 2, 128, 570, 5921, "causal"),
 ])
