@@ -425,6 +425,7 @@ def test_linear_silu_tiled_w(M):
                                    (257, 8208, 256), (513, 4096, 512),
                                    (33, 16416, 512), (48, 4000, 2048), (49, 20512, 512), (64, 6128, 2048),
                                    (97, 24560, 256),    # 33 .. 64 rows: one column tile per wave; 6 waves
+                                   (200, 8192, 512), (300, 8192, 512),   # split one-round chunks, one and two per CU
                                    (130, 1040, 768), (100, 80, 1536),   # lower row tiles in a small grid
                                    (140, 12304, 1024), (400, 12304, 512), (129, 24592, 512)])   # three tiles, two
 def test_linear_many_rows(M, N, K):
