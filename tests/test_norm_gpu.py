@@ -347,10 +347,11 @@ def test_silu_mul_any_width(rows, F, off):
 
 
 @pytest.mark.parametrize("rows,F", [(1, 8), (3, 2056), (342, 12288), (1025, 4104), (383, 4104), (384, 4096),
-                                    (1537, 1028), (1537, 1030)])
+                                    (1537, 1028), (1537, 1030), (1366, 12288), (1365, 12288),
+                                    (6600, 2560), (8300, 2040)])
 def test_silu_mul_wide_forms(rows, F):
-    """Sizes on both sides of 1.5 M elements, from where a thread takes four of them, and widths
-    that are no multiple of four: the bits of the two- and one-element forms (the same values
+    """Sizes on both sides of 1.5 M and 16.8 M elements, from where a thread takes four and eight
+    of them, widths that fill the wider blocks badly or are no multiple of four: the bits of the two- and one-element forms (the same values
     at addresses only those take), and of contiguous halves as of a packed gate/up tensor;
     infinities and NaN among them."""
     from respect_amd import _lib
