@@ -1052,21 +1052,21 @@ static bool wide_fits(const gemm::Args& a) {
 // Whether gemm_wide_kernel runs the call.  Always above 64 rows, except that tiled
 // operands whose chunk is one round of gemm_kernel stay there while neither grid is
 // large ([4096, 1024]: 96 rows 5.3 us against 5.6, 128 rows 5.8 / 6.4; [576, 512],
-// 1024 rows 4.8 / 5.5; but [6144, 1024], 96 rows 8.7 / 7.5), or are split with at most one
-// of its workgroups per CU ([1024, 1024], 836 rows: 13.9 / 16.4; [6912, 512], 235 rows: 14.5 /
-// 15.9; with two [3840, 1024], 613 rows: 25.1 / 24.1).  For 33 .. 64 rows where waves of one column tile make one workgroup for most CUs and its chunk has
-// eight rounds or more: q/k/v [6144, 4096], o [4096, 4096], gate/up [24576, 4096] and
-// down [4096, 12288], tiled, at 64 rows 12.3 / 9.1 / 37.2 / 20.7 us instead of
-// 13.7 / 10.3 / 39.7 / 23.3 in gemm_kernel, at 48 rows 11.7 / 8.6 / 36.1 / 19.6
-// instead of 12.1 / 9.6 / 36.9 / 21.8, at 32 rows 11.4 / 8.3 / 35.7 / 19.0 and 11.2 /
-// 8.5 / 36.1 / 19.3; row-major at 64 rows 13.1 / 9.8 / 44.5 / 25.4 instead of 16.3 /
-// 11.7 / 47.6 / 28.1.  Tiled x with row-major w is the slower one there (gate/up, 48
-// rows: 43.6 / 40.6).  Below 208 workgroups tiled operands gain or lose up to a quarter with no rule in the
-// sizes ([9184, 8704], 35 rows 43.7 / 35.3; [12544, 2304], 55 rows 15.2 / 17.1), mostly gain.
-// gemm_kernel keeps more bytes of W in flight per wave, which
-// counts in short chunks and small grids ([4096, 1024], 64 rows: 5.1 against 5.3;
-// [1024, 3072], 64 workgroups, 48 rows: 5.9 / 6.1), and shares X between 128 columns
-// in large ones (vocabulary [151936, 4096]: 239 / 252).
+// 1024 rows 4.8 / 5.5; but [6144, 1024], 96 rows 8.7 / 7.5), or are split with at most
+// one workgroup per CU ([1024, 1024], 836 rows: 13.9 / 16.4; [6912, 512], 235 rows: 14.5 /
+// 15.9; with two [3840, 1024], 613 rows: 25.1 / 24.1).  For 33 .. 64 rows where waves of one
+// column tile make one workgroup for most CUs and its chunk has eight rounds or more:
+// q/k/v [6144, 4096], o [4096, 4096], gate/up [24576, 4096] and down [4096, 12288], tiled,
+// at 64 rows 12.3 / 9.1 / 37.2 / 20.7 us instead of 13.7 / 10.3 / 39.7 / 23.3 in
+// gemm_kernel, at 48 rows 11.7 / 8.6 / 36.1 / 19.6 instead of 12.1 / 9.6 / 36.9 / 21.8, at
+// 32 rows 11.4 / 8.3 / 35.7 / 19.0 and 11.2 / 8.5 / 36.1 / 19.3; row-major at 64 rows 13.1 /
+// 9.8 / 44.5 / 25.4 instead of 16.3 / 11.7 / 47.6 / 28.1.  Tiled x with row-major w is the
+// slower one there (gate/up, 48 rows: 43.6 / 40.6).  Below 208 workgroups tiled operands
+// gain or lose up to a quarter with no rule in the sizes ([9184, 8704], 35 rows 43.7 / 35.3;
+// [12544, 2304], 55 rows 15.2 / 17.1), mostly gain.  gemm_kernel keeps more bytes of W in
+// flight per wave, which counts in short chunks and small grids ([4096, 1024], 64 rows: 5.1
+// against 5.3; [1024, 3072], 64 workgroups, 48 rows: 5.9 / 6.1), and shares X between 128
+// columns in large ones (vocabulary [151936, 4096]: 239 / 252).
 static bool use_wide(const gemm::Args& a, WaveTile t) {
   if (!wide_fits(a) || a.M <= 32) return false;
   const bool w_tiled = a.sw == kTiled;
@@ -1220,7 +1220,10 @@ static int linear_any(const void* x, int64_t sx, const void* w, int64_t sw, void
   if (sx < K || sw < K || so < N) return RSPX_EINVAL;
   auto al = [](const void* p, unsigned a) { return (reinterpret_cast<uintptr_t>(p) & (a - 1)) == 0; };
   if (!al(x, 2) || !al(w, 2) || !al(out, out_fp32 ? 4 : 2)) return RSPX_EALIGN;
-  // 31-bit byte offsets inside one 64-row tile of x and one 16-row slice of w.
+  // Rows are addressed with 64-bit pointers.  What these limits bound is K (a row is at least
+  // K elements: K < 2^24), so that the kernels' int offsets inside a row, three rounds past K
+  // and beside the 0x40000000 that stands for no fragment, stay below 2^31; the M limit, that
+  // row numbers do.
   if (((int64_t)gemm::kRows * sx + K) * 2 >= (1ll << 31) - 64 || ((int64_t)16 * sw + K) * 2 >= (1ll << 31) - 64)
     return RSPX_EUNSUPPORTED;
   if ((M + gemm::kRows - 1) / gemm::kRows > 65535) return RSPX_EUNSUPPORTED;

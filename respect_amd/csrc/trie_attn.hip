@@ -1554,7 +1554,6 @@ __device__ __forceinline__ const lds_float* node_stream(const TrieAttnArgs& A, i
   const int lane = __lane_id();
   const int n16 = lane & 15, g4 = lane >> 4, e4 = n16 >> 2, c4 = n16 & 3;
   const int NN = A.NN, nch = (NN + kChunk - 1) / kChunk, nt = (NN + 15) / 16;
-  const float scale = score_scale(A);
   const int GQA = 1 << A.GQS, q0 = p0 >> A.GQS, ng = ((rend - 1) >> A.GQS) - q0 + 1;
   const int nrd = (rend - p0 - w + nw - 1) / nw;   // rows of this wave: p0 + w + 8 i
   lds_float* S = (lds_float*)(kv + LY::SOFF);
@@ -1614,7 +1613,7 @@ __device__ __forceinline__ const lds_float* node_stream(const TrieAttnArgs& A, i
 #pragma unroll
       for (int i = 0; i < DQ; ++i)
         sv = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, kf[u][i]), qf[i], sv, 0, 0, 0);
-      *(lds_f32x4*)(S + n16 * LY::SR + 16 * (tb + nw * u) + 4 * g4) = sv * scale;
+      *(lds_f32x4*)(S + n16 * LY::SR + 16 * (tb + nw * u) + 4 * g4) = sv * score_scale(A);
     }
   }
   lds_barrier();   // every score is in LDS
