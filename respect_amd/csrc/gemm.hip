@@ -1085,7 +1085,10 @@ static int wide_launch(const gemm::Args& a, WaveTile wt, int mtiles, hipStream_t
   const int64_t units = (int64_t)((a.N + cols - 1) / cols) * a.S;
   // Lower row tiles while the grid stays within one workgroup per CU ([1024, 3072],
   // tiled / row-major, 128 rows: 7.0 / 11.7 us in one tile, 4.7 / 6.1 in four).
-  if (wt.ct == 1 && units < 256) mtiles = max(mtiles, min((int)(256 / units), (a.M + 31) / 32));
+  // Units are dealt over the 8 XCDs of 32 CUs, so the XCD with the most of them counts
+  // (374 rows of [1280, 3840], row-major, 20 units: in 12 tiles, 36 workgroups on four XCDs,
+  // 33.1 us; in 10 20.1; 64-row tiles of gemm_kernel 29.5).
+  if (wt.ct == 1 && units < 256) mtiles = max(mtiles, min((int)(32 / ((units + 7) / 8)), (a.M + 31) / 32));
   const int mt = ((a.M + mtiles - 1) / mtiles + 15) / 16;
   mtiles = (a.M + 16 * mt - 1) / (16 * mt);
   const int64_t wgs = (units + 7) / 8 * 8 * mtiles;

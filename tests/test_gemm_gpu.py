@@ -426,6 +426,7 @@ def test_linear_silu_tiled_w(M):
                                    (33, 16416, 512), (48, 4000, 2048), (49, 20512, 512), (64, 6128, 2048),
                                    (97, 24560, 256),    # 33 .. 64 rows: one column tile per wave; 6 waves
                                    (200, 8192, 512), (300, 8192, 512),   # split one-round chunks, one and two per CU
+                                   (374, 1280, 768), (645, 704, 256),    # 20 and 11 units over 8 XCDs
                                    (130, 1040, 768), (100, 80, 1536),   # lower row tiles in a small grid
                                    (140, 12304, 1024), (400, 12304, 512), (129, 24592, 512)])   # three tiles, two
 def test_linear_many_rows(M, N, K):
