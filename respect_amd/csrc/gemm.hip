@@ -897,11 +897,13 @@ __global__ __launch_bounds__(256) void gemm_short_kernel(AnyArgs A) {
 }
 
 // K < 8: no row holds a 16-byte group.  One 16 x 16 tile per wave, its elements
-// loaded one by one into the single k-block of the chain.
-__global__ __launch_bounds__(64) void gemm_small_k_kernel(AnyArgs A, int ntiles) {
+// loaded one by one into the single k-block of the chain.  Grid: x = column tiles, y =
+// row tiles from row0 on (at most 65535 per launch): tiles counted along x alone would
+// reach the 2^32 threads that a grid dimension may have at 2^34 outputs.
+__global__ __launch_bounds__(64) void gemm_small_k_kernel(AnyArgs A, int row0) {
   const int lane = __lane_id(), n16 = lane & 15, g4 = lane >> 4;
-  const int n0 = 16 * (int)(blockIdx.x % ntiles);
-  const int64_t m0 = 16 * (int64_t)(blockIdx.x / ntiles);
+  const int n0 = 16 * (int)blockIdx.x;
+  const int64_t m0 = row0 + 16 * (int64_t)blockIdx.y;
   u32x4 wf = {0u, 0u, 0u, 0u}, xf = wf;
   if (g4 == 0) {
 #pragma unroll
@@ -1233,9 +1235,11 @@ static int linear_any(const void* x, int64_t sx, const void* w, int64_t sw, void
   gemm::AnyArgs a{static_cast<const uint16_t*>(x), sx, static_cast<const uint16_t*>(w), sw, out, so, M, N, K,
                   out_fp32 ? 1 : 0};
   if (K < 8) {
-    const int64_t tiles = (int64_t)((N + 15) / 16) * ((M + 15) / 16);
-    if (tiles > 0x7fffffff) return RSPX_EUNSUPPORTED;
-    hipLaunchKernelGGL(gemm::gemm_small_k_kernel, dim3((unsigned)tiles), dim3(64), 0, s, a, (N + 15) / 16);
+    constexpr int kRowsPerLaunch = 16 * 65535;
+    for (int row0 = 0; row0 < M; row0 += kRowsPerLaunch) {
+      const dim3 g((unsigned)((N + 15) / 16), (unsigned)((min(M - row0, kRowsPerLaunch) + 15) / 16));
+      hipLaunchKernelGGL(gemm::gemm_small_k_kernel, g, dim3(64), 0, s, a, row0);
+    }
     return hipGetLastError() == hipSuccess ? RSPX_OK : RSPX_ELAUNCH;
   }
   // Short K: gemm_short_kernel, in row tiles as high as leave a workgroup to every CU.

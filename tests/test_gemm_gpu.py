@@ -506,3 +506,22 @@ def test_linear_any_shape_edges(M, N, K):
                                             None, 0, s))
     torch.cuda.synchronize()
     assert torch.equal(ob, f32)
+
+
+# The last row tile of a launch, the first row of the next one, and 2^26 tiles (34 GB of output).
+@pytest.mark.parametrize("M,N,K", [(16 * 65535, 17, 3), (16 * 65535 + 1, 33, 7), (64 * 65535, 4112, 1)])
+def test_linear_small_k_many_tiles(M, N, K):
+    from respect_amd import _lib
+    print(f"[linear small K] M={M} N={N} K={K}", flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(N)
+    x = torch.randn(M, K, device="cuda", generator=gen).bfloat16()
+    w = torch.randn(N, K, device="cuda", generator=gen).bfloat16()
+    y = torch.empty(M, N, device="cuda", dtype=torch.bfloat16)
+    L, s = _lib.lib(), _lib.stream_ptr(x.device)
+    _lib.check("rspx_linear", L.rspx_linear(x.data_ptr(), K, w.data_ptr(), K, y.data_ptr(), N, M, N, K, 0, None, 0, s))
+    rows = [r for r in (0, 15, 16, M // 2, 16 * 65535 - 1, 16 * 65535, M - 17, M - 1) if r < M]
+    xr, wr = x[rows].double().cpu().numpy(), w.double().cpu().numpy()
+    ex = G.linear_exact(xr, wr)
+    bound = G.linear_error_bound(xr, wr)
+    out = y[rows].float().cpu().numpy()
+    assert np.all(np.abs(out - ex) <= bound + bf16.ulp(np.abs(ex) + bound))
